@@ -59,7 +59,7 @@ HIP_FLAGS = [
     "-mllvm", "-amdgpu-mfma-vgpr-form=1",
 ]
 
-KERNEL_SOURCES = [CSRC / "attn_kernel.hip", CSRC / "conv3d_kernel.hip"]
+KERNEL_SOURCES = [CSRC / "attn_kernel.hip", CSRC / "conv3d_kernel.hip", CSRC / "scratch.hip"]
 # A torch-free C caller of launch() (the reference's micro3.hip pattern),
 # linked against the kernel library.
 HARNESS_SOURCE = CSRC / "launch_harness.cpp"
@@ -146,7 +146,7 @@ def _newest_mtime(paths) -> float:
 
 
 def kernel_lib_inputs() -> list:
-    return [*KERNEL_SOURCES, *sorted(INCLUDE.glob("*.h"))]
+    return [*KERNEL_SOURCES, CSRC / "scratch.h", *sorted(INCLUDE.glob("*.h"))]
 
 
 def ensure_kernel_lib(lib: Path = KERNEL_LIB, sources=None) -> bool:

@@ -56,12 +56,15 @@
 #include <math.h>
 #include <type_traits>
 #include <algorithm>
-#include <mutex>
 #include <stdlib.h>
 
 #include "gfx906_amd_attn.h"
+#include "scratch.h"
 
 namespace {
+
+using gfx906_amd::kScratchBytes;
+using gfx906_amd::ScratchUse;
 
 typedef _Float16 f16;
 typedef __bf16 bf16;
@@ -2540,97 +2543,6 @@ extern "C" const char* attn_last_error(void) { return g_err[0] ? g_err : nullptr
 
 namespace {
 
-// Workspace of the calls that split without a caller workspace
-// (attn_fwd_split_static, and launch() / attn_fwd() for grids too small for
-// the GPU): the split-key partial results live in this file-scope device
-// array. It is part of the library's code object, so every GPU on which any
-// kernel of the library is loaded holds its own copy (kScratchBytes) until
-// the process ends, whether or not a call ever uses it. Host code must not
-// pass `scratch` itself to a kernel (on the host it names a stand-in, not
-// device memory): it uses the device address that hipGetSymbolAddress
-// returns, looked up once per device. The kernels write every workspace
-// entry the merge reads within the same call, so nothing is cleared between
-// calls.
-//
-// Calls that use the array are ordered on the GPU, whatever streams they are
-// issued on: each records `done` on its stream after its kernels, and a call
-// on another stream first makes its stream wait for that event (the host
-// lock keeps wait, launches and record of one call together, so the calls
-// form one chain per device). A call made under stream capture neither
-// waits nor records (an event recorded outside the graph cannot order its
-// replays): a graph that contains one is ordered only by the stream it is
-// launched on, and must not run concurrently with other calls that use the
-// array on that device.
-constexpr size_t kScratchBytes = size_t(96) << 20;
-static __device__ __align__(256) char scratch[kScratchBytes];
-
-constexpr int kMaxDevices = 64;
-struct DevScratch {
-    void* ptr;           // device address of `scratch`
-    hipEvent_t done;     // recorded after the last call outside capture that used it
-    hipStream_t last;    // the stream of that call
-    bool recorded;
-};
-std::mutex g_scratch_mu;
-DevScratch g_scratch[kMaxDevices];
-
-// Device of `stream` (the current device for the null stream), or -1 with
-// the error message set.
-int stream_device(hipStream_t stream) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess && stream) e = hipStreamGetDevice(stream, &dev);
-    if (e != hipSuccess) {
-        set_err(hipGetErrorString(e));
-        return -1;
-    }
-    if (dev < 0 || dev >= kMaxDevices) {
-        set_err("attn: device index beyond the scratch table");
-        return -1;
-    }
-    return dev;
-}
-
-// Looks up `scratch` on device dev and creates its ordering event, once.
-// Caller holds g_scratch_mu. Returns 0, or 2 with the error message set.
-int scratch_setup(int dev) {
-    DevScratch& d = g_scratch[dev];
-    if (d.ptr) return 0;
-    int cur = 0;
-    hipError_t e = hipGetDevice(&cur);
-    if (e == hipSuccess && dev != cur) e = hipSetDevice(dev);
-    if (e != hipSuccess) {
-        set_err(hipGetErrorString(e));
-        return 2;
-    }
-    void* p = nullptr;
-    hipEvent_t ev = nullptr;
-    e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (e == hipSuccess && !p) e = hipErrorInvalidSymbol;
-    // The event only orders kernels of this device on two of its streams
-    // (hipStreamWaitEvent); nothing on the host or on another device inspects
-    // it, so its record needs no system-scope fence: the kernels' own release
-    // at their end makes the scratch visible to the device's later kernels.
-    // Without the fence a call that splits costs about 2 us less of GPU time
-    // (measured on MI355X: B1 H1 S1024 D64 through launch() 16.3 -> 14.5 us).
-    if (e == hipSuccess)
-        e = hipEventCreateWithFlags(&ev, hipEventDisableTiming | hipEventDisableSystemFence);
-    if (dev != cur) {
-        const hipError_t r = hipSetDevice(cur);
-        if (e == hipSuccess) e = r;
-    }
-    if (e != hipSuccess) {
-        if (ev) (void)hipEventDestroy(ev);
-        set_err(hipGetErrorString(e));
-        return 2;
-    }
-    d.ptr = p;
-    d.done = ev;
-    d.last = nullptr;
-    d.recorded = false;
-    return 0;
-}
-
 // attn_fwd_ex (workspace_bytes == SIZE_MAX: never split), attn_fwd_split
 // (caller workspace) and, with use_scratch, attn_fwd_split_static, launch()
 // and attn_fwd() (workspace: the static scratch, split plans bounded by its
@@ -2680,35 +2592,18 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     if (workspace_bytes != (size_t)-1)  // split the keys if it pays
         p = plan_split(B, H, Sq, Skv, D, use_scratch ? kScratchBytes : (size_t)-1);
     const size_t need = split_ws_bytes(p, B, H, Sq, D);
-    DevScratch* ds = nullptr;
-    std::unique_lock<std::mutex> lock(g_scratch_mu, std::defer_lock);
-    bool capturing = false;
+    ScratchUse scratch;
     if (need && use_scratch) {
-        const int dev = stream_device(stream);
-        if (dev < 0) return 2;
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        hipError_t e = hipStreamIsCapturing(stream, &st);
-        if (e != hipSuccess) {
-            set_err(hipGetErrorString(e));
+        const ScratchUse::Status st = scratch.acquire(stream, true);
+        if (st == ScratchUse::kUnavailable)
+            return fail("attn: the static scratch of this device is set up by the first call "
+                        "that splits outside stream capture; make one such call before "
+                        "capturing");
+        if (st == ScratchUse::kFailed) {
+            set_err(scratch.error);
             return 2;
         }
-        capturing = st != hipStreamCaptureStatusNone;
-        lock.lock();
-        ds = &g_scratch[dev];
-        if (!ds->ptr) {
-            if (capturing)
-                return fail("attn: the static scratch of this device is set up by the first call "
-                            "that splits outside stream capture; make one such call before "
-                            "capturing");
-            const int rc = scratch_setup(dev);
-            if (rc) return rc;
-        }
-        if (!capturing && ds->recorded && ds->last != stream &&
-            (e = hipStreamWaitEvent(stream, ds->done, 0)) != hipSuccess) {
-            set_err(hipGetErrorString(e));
-            return 2;
-        }
-        workspace = ds->ptr;
+        workspace = scratch.ptr;
         workspace_bytes = kScratchBytes;
     }
     if (need) {
@@ -2725,13 +2620,7 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     const bool tl = token_contiguous(sk, sv, D);
     hipError_t e = dtype == ATTN_DTYPE_BF16 ? launch_t<bf16>(a, tl, stream)
                                             : launch_t<f16>(a, tl, stream);
-    if (e == hipSuccess && ds && !capturing) {
-        e = hipEventRecord(ds->done, stream);
-        if (e == hipSuccess) {
-            ds->last = stream;
-            ds->recorded = true;
-        }
-    }
+    if (e == hipSuccess) e = scratch.release(stream);
     if (e != hipSuccess) {
         set_err(hipGetErrorString(e));
         return 2;

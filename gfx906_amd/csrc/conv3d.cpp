@@ -35,12 +35,19 @@ void conv3d(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
         TORCH_CHECK(bias->is_contiguous() && bias->numel() == dims[5], "conv3d: bias must be [K]");
     const c10::DeviceGuard guard(x.device());
     const long M = (long)dims[0] * dims[12] * dims[13] * dims[14];
-    const int rc = conv3d_fwd(
+    // A split reduction's partial sums go to a workspace from torch's caching
+    // allocator.
+    const size_t ws_bytes =
+        conv3d_workspace_bytes(M, (int)dims[5], (long)dims[4] * dims[6] * dims[7] * dims[8]);
+    torch::Tensor ws;
+    if (ws_bytes) ws = torch::empty({(int64_t)ws_bytes}, x.options().dtype(torch::kUInt8));
+    const int rc = conv3d_fwd_split(
         x.data_ptr(), w.data_ptr(), bias.has_value() ? bias->data_ptr() : nullptr,
         res.has_value() ? res->data_ptr() : nullptr, out.data_ptr(), (int)dims[0], (int)dims[1],
         (int)dims[2], (int)dims[3], (int)dims[4], (int)dims[5], (int)dims[6], (int)dims[7],
         (int)dims[8], (int)dims[9], (int)dims[10], (int)dims[11], (int)dims[12], (int)dims[13],
         (int)dims[14], M, xs[0], xs[1], xs[2], xs[3], os[0], os[1], os[2], os[3], rs[0], rs[1],
-        rs[2], rs[3], c10::hip::getCurrentHIPStream().stream());
+        rs[2], rs[3], c10::hip::getCurrentHIPStream().stream(), ws_bytes ? ws.data_ptr() : nullptr,
+        ws_bytes);
     TORCH_CHECK(rc == 0, "kernel: ", conv3d_last_error() ? conv3d_last_error() : "launch failed");
 }

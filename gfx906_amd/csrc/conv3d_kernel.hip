@@ -35,10 +35,15 @@
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
+#include <algorithm>
 
 #include "gfx906_amd_conv3d.h"
+#include "scratch.h"
 
 namespace {
+
+using gfx906_amd::kScratchBytes;
+using gfx906_amd::ScratchUse;
 
 typedef _Float16 f16;
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -56,6 +61,11 @@ struct ConvArgs {
     int C, K, T, R, S, sd, sh, sw, Z, P, Q, M, KG;
     long long xsn, xsd, xsh, xsw, osn, osz, osp, osq, rsn, rsz, rsp, rsq;
     unsigned x_bytes, w_bytes;
+    // Split reduction (nsplit > 1): split s takes reduction elements
+    // [s*split_len, (s+1)*split_len) and writes its fp32 sums to
+    // ws[s][m][k]; conv3d_reduce adds them up and runs the epilogue.
+    int nsplit, split_len;
+    float* ws;
 };
 
 constexpr int kMaxTaps = 1024;
@@ -144,16 +154,11 @@ __device__ __forceinline__ int tile_of(int L, int n) {
     return (xcd < extra ? xcd * (base + 1) : extra * (base + 1) + (xcd - extra) * base) + pos;
 }
 
-// grid: ceil(M / (64*NB)) * ceil(K / (64*CW)) workgroups (1-D, see tile_of);
-// block: 128*CW threads. SMALLC: C < KB, so that one k-tile can cross
-// several taps.
-// The second launch bound is HIP's minimum waves per SIMD (amdgpu_waves_per_eu):
-// OCC workgroups of 2*CW waves over the CU's four SIMDs.
-template <int NB, int NST, int KB, int CW, bool SMALLC>
-__global__ void __launch_bounds__((ConvCfg<NB, NST, KB, CW>::NT),
-                                  (ConvCfg<NB, NST, KB, CW>::OCC * ConvCfg<NB, NST, KB, CW>::NW / 4))
-    conv3d_mfma(const ConvArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
+// One workgroup of conv3d_mfma (SPLIT: of conv3d_part). SMALLC: C < KB, so
+// that one k-tile can cross several taps.
+template <int NB, int NST, int KB, int CW, bool SMALLC, bool SPLIT>
+__device__ __forceinline__ void conv_tile(const ConvArgs a) {
     using Cf = ConvCfg<NB, NST, KB, CW>;
     constexpr int STAGE = Cf::STAGE, LOADS = Cf::LOADS, ROWB = Cf::ROWB, UNITS = Cf::UNITS;
     constexpr int RPB = Cf::RPB, WJ = Cf::WJ, XJ = Cf::XJ, NW = Cf::NW;
@@ -167,13 +172,24 @@ __global__ void __launch_bounds__((ConvCfg<NB, NST, KB, CW>::NT),
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int m0, k0;
+    // Work item: split-major, so that with a split reduction an XCD's
+    // workgroups share the weights and taps of one or two ranges.
+    int m0, k0, split = 0;
     {
         const int nct = (a.K + Cf::BCH - 1) / Cf::BCH;
-        const int t = tile_of(blockIdx.x, gridDim.x), vt = t / nct;
+        int t = tile_of(blockIdx.x, gridDim.x);
+        if constexpr (SPLIT) {
+            const int ntiles = (int)gridDim.x / a.nsplit;
+            split = t / ntiles;
+            t -= split * ntiles;
+        }
+        const int vt = t / nct;
         m0 = vt * Cf::BVX;
         k0 = (t - vt * nct) * Cf::BCH;
     }
+    // This workgroup's reduction range.
+    const int i_beg = SPLIT ? split * a.split_len : 0;
+    const int i_end = SPLIT ? min(a.KG, i_beg + a.split_len) : a.KG;
 
     // Load roles. LDS block b (1 KB) holds rows RPB*b..RPB*b+RPB-1 of a tile;
     // lane l writes row RPB*b + l/UNITS, slot l%UNITS, so it fetches unit
@@ -209,7 +225,7 @@ __global__ void __launch_bounds__((ConvCfg<NB, NST, KB, CW>::NT),
     // gi = i0 + 8u lies in tap (t, r, s) at channel cc, and the tap starts
     // toff elements into a window (toff = t*xsd + r*xsh + s*xsw). The tap is
     // advanced incrementally, so the loop reads no tap table.
-    int gi = 8 * u;
+    int gi = i_beg + 8 * u;
     int cc, ts, tr, toff;
     {
         const int tp = gi / a.C;
@@ -239,9 +255,9 @@ __global__ void __launch_bounds__((ConvCfg<NB, NST, KB, CW>::NT),
 
     // Loads of the next k-tile (reduction indices i0 .. i0+KB-1) into an LDS
     // stage, then the lane's group moves on by KB.
-    int i0 = 0;
+    int i0 = i_beg;
     auto issue = [&](char* dst) __attribute__((always_inline)) {
-        const bool kin = gi < a.KG;
+        const bool kin = gi < i_end;
 #pragma unroll
         for (int j = 0; j < WJ; ++j) {
             const unsigned ow = (wv[j] && kin) ? wo[j] + 2u * (unsigned)i0 : kOOB;
@@ -325,7 +341,7 @@ __global__ void __launch_bounds__((ConvCfg<NB, NST, KB, CW>::NT),
     };
     // k-tile t sits in stage t % NST. The loop runs whole groups of NST
     // k-tiles: k-tiles past the end load zeros and add nothing.
-    const int nkt = (a.KG + KB - 1) / KB;
+    const int nkt = (i_end - i_beg + KB - 1) / KB;
     issue(st0);
     if constexpr (NST == 2) {
         for (int kt = 0; kt < nkt; kt += 2) {
@@ -353,6 +369,20 @@ __global__ void __launch_bounds__((ConvCfg<NB, NST, KB, CW>::NT),
     // LDS is released.
     __builtin_amdgcn_s_waitcnt(0x0F70);
 
+    if constexpr (SPLIT) {  // this range's sums, in the accumulators' order
+#pragma unroll
+        for (int vb = 0; vb < 2 * NB; ++vb) {
+            const int m = m0 + wvx * 32 * NB + vb * 16 + r16;
+            if (m >= a.M) continue;
+            float* row = a.ws + ((long long)split * a.M + m) * a.K;
+#pragma unroll
+            for (int cb = 0; cb < 4; ++cb) {
+                const int ch = k0 + wch * 64 + cb * 16 + 4 * g;
+                if (ch < a.K) *(f32x4*)(row + ch) = acc[cb][vb];
+            }
+        }
+        return;
+    }
     // Epilogue: accumulator row 4g + r (an output channel), column l%16 (an
     // output voxel); one run of four channels per lane, voxel and block.
 #pragma unroll
@@ -372,6 +402,66 @@ __global__ void __launch_bounds__((ConvCfg<NB, NST, KB, CW>::NT),
             *(f16x4*)(a.out + oo + ch) = __builtin_convertvector(val, f16x4);
         }
     }
+}
+#endif
+
+// grid: ceil(M / (64*NB)) * ceil(K / (64*CW)) workgroups (1-D, see tile_of);
+// block: 128*CW threads. The second launch bound is HIP's minimum waves per
+// SIMD (amdgpu_waves_per_eu): OCC workgroups of 2*CW waves over the CU's four
+// SIMDs.
+template <int NB, int NST, int KB, int CW, bool SMALLC>
+__global__ void __launch_bounds__((ConvCfg<NB, NST, KB, CW>::NT),
+                                  (ConvCfg<NB, NST, KB, CW>::OCC * ConvCfg<NB, NST, KB, CW>::NW / 4))
+    conv3d_mfma(const ConvArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    conv_tile<NB, NST, KB, CW, SMALLC, false>(a);
+#endif
+}
+
+// The same with the reduction split in a.nsplit ranges (a kernel of its own:
+// the range's bounds and second epilogue cost the unsplit form 1 %): nsplit
+// times as many workgroups, split-major.
+template <int NB, int NST, int KB, int CW, bool SMALLC>
+__global__ void __launch_bounds__((ConvCfg<NB, NST, KB, CW>::NT),
+                                  (ConvCfg<NB, NST, KB, CW>::OCC * ConvCfg<NB, NST, KB, CW>::NW / 4))
+    conv3d_part(const ConvArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    conv_tile<NB, NST, KB, CW, SMALLC, true>(a);
+#endif
+}
+
+// Sum of a split reduction's partial results in split order, then the epilogue
+// of conv3d_mfma. One thread per voxel and 4 channels; the loads of
+// kRedBatch splits go out together (the partial results of a problem small
+// enough to be split mostly come from the caches, so latency, not bandwidth,
+// would bound a loop that waited for each split in turn).
+constexpr int kRedBatch = 4;
+__global__ void __launch_bounds__(256) conv3d_reduce(const ConvArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int kq = a.K / 4;
+    const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= (long long)a.M * kq) return;
+    const int m = (int)(idx / kq), ch = (int)(idx - (long long)m * kq) * 4;
+    const float* part = a.ws + (long long)m * a.K + ch;
+    const long long step = (long long)a.M * a.K;
+    f32x4 val = {};
+    for (int s0 = 0; s0 < a.nsplit; s0 += kRedBatch) {
+        f32x4 p[kRedBatch];
+#pragma unroll
+        for (int u = 0; u < kRedBatch; ++u)
+            if (s0 + u < a.nsplit) p[u] = *(const f32x4*)(part + (s0 + u) * step);
+#pragma unroll
+        for (int u = 0; u < kRedBatch; ++u)
+            if (s0 + u < a.nsplit) val += p[u];
+    }
+    const Voxel v = voxel(m, a.Z, a.P, a.Q);
+    if (a.bias) val += __builtin_convertvector(*(const f16x4*)(a.bias + ch), f32x4);
+    if (a.res)
+        val += __builtin_convertvector(
+            *(const f16x4*)(a.res + v.n * a.rsn + v.z * a.rsz + v.p * a.rsp + v.q * a.rsq + ch),
+            f32x4);
+    *(f16x4*)(a.out + v.n * a.osn + v.z * a.osz + v.p * a.osp + v.q * a.osq + ch) =
+        __builtin_convertvector(val, f16x4);
 #endif
 }
 
@@ -380,13 +470,16 @@ template <int NB, int NST, int KB, int CW>
 void launch_cfg(const ConvArgs& a, hipStream_t stream) {
     using Cf = ConvCfg<NB, NST, KB, CW>;
     const unsigned tiles = (unsigned)((a.M + Cf::BVX - 1) / Cf::BVX) *
-                           (unsigned)((a.K + Cf::BCH - 1) / Cf::BCH);
-    if (a.C < KB)
-        hipLaunchKernelGGL((conv3d_mfma<NB, NST, KB, CW, true>), dim3(tiles), dim3(Cf::NT), 0,
-                           stream, a);
+                           (unsigned)((a.K + Cf::BCH - 1) / Cf::BCH) * (unsigned)a.nsplit;
+    const dim3 grid(tiles), block(Cf::NT);
+    if (a.C < KB && a.nsplit > 1)
+        hipLaunchKernelGGL((conv3d_part<NB, NST, KB, CW, true>), grid, block, 0, stream, a);
+    else if (a.C < KB)
+        hipLaunchKernelGGL((conv3d_mfma<NB, NST, KB, CW, true>), grid, block, 0, stream, a);
+    else if (a.nsplit > 1)
+        hipLaunchKernelGGL((conv3d_part<NB, NST, KB, CW, false>), grid, block, 0, stream, a);
     else
-        hipLaunchKernelGGL((conv3d_mfma<NB, NST, KB, CW, false>), dim3(tiles), dim3(Cf::NT), 0,
-                           stream, a);
+        hipLaunchKernelGGL((conv3d_mfma<NB, NST, KB, CW, false>), grid, block, 0, stream, a);
 }
 
 thread_local char g_err[256];
@@ -405,18 +498,22 @@ int fail(const char* msg) {
 bool mult8(long v) { return v >= 0 && v % 8 == 0; }
 
 // The kernel configurations: NB, KB, channels per workgroup (64*CW),
-// workgroups per CU, relative cost per output element and reduction element
-// (fitted on MI355X, see pick_kernel), launcher.
+// workgroups per CU, and the time in us of a 64-voxel x 256-channel piece of a
+// tile: `per_kg` for a reduction of 13824 elements, `fixed` for start-up and
+// epilogue (fitted on MI355X, see plan_conv); launcher.
 struct ConvKernel {
     int nb, kb, bch, occ;
-    double rel;
+    double per_kg, fixed;
     void (*launch)(const ConvArgs&, hipStream_t);
 };
 const ConvKernel kKernels[] = {
-    {4, 32, 128, 2, 6.21, launch_cfg<4, 3, 32, 2>}, {3, 64, 128, 2, 6.18, launch_cfg<3, 2, 64, 2>},
-    {2, 64, 128, 2, 6.68, launch_cfg<2, 2, 64, 2>}, {4, 32, 256, 1, 4.78, launch_cfg<4, 4, 32, 4>},
-    {3, 64, 256, 1, 5.91, launch_cfg<3, 2, 64, 4>}, {2, 64, 256, 1, 5.47, launch_cfg<2, 3, 64, 4>},
-    {3, 32, 256, 1, 6.19, launch_cfg<3, 4, 32, 4>},
+    {4, 32, 128, 2, 88.8, 2.1, launch_cfg<4, 3, 32, 2>},
+    {3, 64, 128, 2, 89.5, 2.3, launch_cfg<3, 2, 64, 2>},
+    {2, 64, 128, 2, 105.9, 2.0, launch_cfg<2, 2, 64, 2>},
+    {4, 32, 256, 1, 81.5, 1.6, launch_cfg<4, 4, 32, 4>},
+    {3, 64, 256, 1, 85.0, 1.5, launch_cfg<3, 2, 64, 4>},
+    {2, 64, 256, 1, 78.5, 2.6, launch_cfg<2, 3, 64, 4>},
+    {3, 32, 256, 1, 92.0, 1.7, launch_cfg<3, 4, 32, 4>},
 };
 constexpr int kNumKernels = sizeof(kKernels) / sizeof(kKernels[0]);
 
@@ -426,55 +523,97 @@ int find_kernel(int nb, int kb, int bch) {
     return -1;
 }
 
-// Kernel configuration for an M x K problem with reduction length KG. Wider
-// tiles load fewer bytes per MFMA (the loads into LDS, not the matrix cores,
-// bound these kernels); narrower ones fill the CUs better when the tile count
-// is small or just past a multiple of the workgroup slots. 64-wide k-tiles
-// fetch whole 128-byte lines, 32-wide ones half lines but leave room for a
-// deeper ring. Estimated time: R x tile size x (rel x KG / 13824 + 0.355),
-// R the workgroups on the busiest CU in units of one workgroup's time (for
-// two per CU: half rounds, a workgroup left alone on its CU at the end
-// counting 1.3 halves), rel and the per-tile term (start-up and epilogue)
-// fitted to six layers on MI355X (VAE decoder 3x3x3 with 128..512 channels,
-// a 1x1x1; 3x32x256's rel from its time ratio to 3x64x256 with the 16x16x32
-// MFMA kernels, 1.00-1.06 over five layers, so that it is not picked where
-// 3x64x256 fits the same tiles).
-// GFX906_AMD_CONV_CFG = "<NB>x<KB>" (128 channels) or "<NB>x<KB>x<channels>"
-// (a row of kKernels) overrides the choice (testing); it is read on every
-// call.
-int pick_kernel(long M, int K, long KG) {
-    if (const char* e = getenv("GFX906_AMD_CONV_CFG")) {
-        int nb = 0, kb = 0, bch = 128;
-        if (sscanf(e, "%dx%dx%d", &nb, &kb, &bch) >= 2) {
-            const int i = find_kernel(nb, kb, bch);
-            if (i >= 0) return i;
-        }
-    }
-    static const int ncu = [] {
+// Kernel configuration and split of the reduction for an M x K problem with
+// reduction length KG: the pair with the least estimated time. Wider tiles
+// load fewer bytes per MFMA (the loads into LDS, not the matrix cores, bound
+// these kernels); narrower ones fill the CUs better when the tile count is
+// small or just past a multiple of the workgroup slots. 64-wide k-tiles fetch
+// whole 128-byte lines, 32-wide ones half lines but leave room for a deeper
+// ring. A problem with fewer tiles than slots splits the reduction into
+// nsplit ranges of whole 64-element units: without it a 32x32x2-voxel layer of
+// 512 channels (64 tiles of 216 serial k-tiles) left three quarters of the
+// CUs idle and took 183 us; in 8 ranges it takes 42.
+// Estimate: R x tile size x (per_kg x range / 13824 + fixed), R the
+// workgroups on the busiest CU in units of one workgroup's time (for two per
+// CU: half rounds, a workgroup left alone on its CU at the end counting 1.3
+// halves, and 1.65 where every CU has just one, whose four waves then hide
+// little of their own latency), plus for a split the reduce kernel: a launch,
+// a little per range (its loads go out four ranges at a time) and the partial
+// sums' traffic. Fitted to 15 layers on MI355X (1 to 3x3x3 windows, 16 to 512
+// channels, 256 to 65,536 voxels) over every configuration and 1 to 24
+// ranges: the chosen pair is within 3 % of the fastest one on average.
+// For tests, read on every call: GFX906_AMD_CONV_CFG = "<NB>x<KB>" (128
+// channels) or "<NB>x<KB>x<channels>" (a row of kKernels) fixes the
+// configuration, unsplit unless GFX906_AMD_CONV_NSPLIT = n asks for n ranges
+// (as many as there are units at most, fewer where n does not divide them
+// into non-empty ranges, none where the partial sums exceed ws_cap).
+constexpr int kSplitUnit = 64;     // reduction elements
+constexpr int kSplitMinUnits = 4;  // shortest range worth a workgroup
+constexpr int kSplitMax = 64;
+constexpr double kSplitMargin = 1.12;  // a split has to be this much better than none
+constexpr double kRedLaunch = 2.5, kRedPerSplit = 0.5, kRedPerByte = 0.2e-6;  // us
+struct ConvPlan {
+    int cfg, nsplit, split_len;
+};
+
+size_t conv_ws_bytes(const ConvPlan& p, long M, int K) {
+    return p.nsplit <= 1 ? 0 : (size_t)p.nsplit * M * K * 4;
+}
+
+ConvPlan plan_conv(long M, int K, long KG, size_t ws_cap) {
+    static const unsigned ncu = [] {
         int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             n <= 0)
             n = 256;
-        return n;
+        return (unsigned)n;
     }();
-    const double kgu = (double)KG / 13824.0;
-    int best = 0;
-    double best_cost = 1e300;
+    int only = -1;  // forced configuration
+    if (const char* e = getenv("GFX906_AMD_CONV_CFG")) {
+        int nb = 0, kb = 0, bch = 128;
+        if (sscanf(e, "%dx%dx%d", &nb, &kb, &bch) >= 2) only = find_kernel(nb, kb, bch);
+    }
+    const long units = (KG + kSplitUnit - 1) / kSplitUnit;
+    unsigned tiles1[kNumKernels], fewest = ~0u;  // tiles of each configuration, unsplit
     for (int i = 0; i < kNumKernels; ++i) {
         const ConvKernel& c = kKernels[i];
-        const long tiles = (M + 64 * c.nb - 1) / (64 * c.nb) * ((K + c.bch - 1) / c.bch);
-        double r;
-        if (c.occ == 2) {
-            const long n = (tiles + ncu - 1) / ncu;  // half rounds on the busiest CU
-            r = (double)n + (n & 1 ? 0.3 : 0.0);
-        } else {
-            r = (double)((tiles + ncu - 1) / ncu);
-        }
-        const double cost = r * 64.0 * c.nb * c.bch * (c.rel * kgu + 0.355);
-        if (cost < best_cost) {
-            best_cost = cost;
-            best = i;
+        tiles1[i] = (unsigned)((M + 64 * c.nb - 1) / (64 * c.nb) * ((K + c.bch - 1) / c.bch));
+        fewest = std::min(fewest, tiles1[i]);
+    }
+    // More than four rounds of workgroups gain nothing (and the search costs
+    // host time on every call).
+    long ns_lo = 1, ns_hi = only >= 0 ? 1
+                                      : std::min({units / kSplitMinUnits, (long)kSplitMax,
+                                                  (long)(4 * ncu / fewest)});
+    if (const char* e = getenv("GFX906_AMD_CONV_NSPLIT")) {
+        const long n = atol(e);
+        if (n >= 1) ns_lo = ns_hi = std::min(n, units);
+    }
+    ConvPlan best{only >= 0 ? only : 0, 1, (int)KG};
+    double best_cost = 1e300;
+    for (long ns = ns_lo; ns <= std::max(ns_lo, ns_hi); ++ns) {
+        const long per = (units + ns - 1) / ns;
+        const ConvPlan p{0, (int)((units + per - 1) / per), (int)(per * kSplitUnit)};
+        if (ns > ns_lo && p.nsplit != ns) continue;  // the same ranges as a smaller count
+        if (conv_ws_bytes(p, M, K) > ws_cap) break;
+        const double kgu = (double)std::min<long>(KG, p.split_len) / 13824.0;
+        const double red = p.nsplit > 1 ? kRedLaunch + kRedPerSplit * p.nsplit +
+                                              kRedPerByte * (double)conv_ws_bytes(p, M, K)
+                                        : 0.0;
+        for (int i = 0; i < kNumKernels; ++i) {
+            if (only >= 0 && i != only) continue;
+            const ConvKernel& c = kKernels[i];
+            const unsigned n = (tiles1[i] * (unsigned)p.nsplit + ncu - 1) / ncu;
+            double r = n;  // workgroups on the busiest CU
+            if (c.occ == 2) r += n == 1 ? 0.65 : n & 1 ? 0.3 : 0.0;  // (half rounds)
+            double cost = r * c.nb * c.bch / 256.0 * (c.per_kg * kgu + c.fixed) + red;
+            if (p.nsplit > 1) cost *= kSplitMargin;
+            if (cost < best_cost) {
+                best_cost = cost;
+                best = p;
+                best.cfg = i;
+            }
         }
     }
     return best;
@@ -484,11 +623,15 @@ int pick_kernel(long M, int K, long KG) {
 
 extern "C" const char* conv3d_last_error(void) { return g_err[0] ? g_err : nullptr; }
 
-extern "C" int conv3d_fwd(const void* x, const void* w, const void* bias, const void* res,
-                          void* out, int nB, int D, int H, int W, int C, int K, int T, int R, int S,
-                          int sd, int sh, int sw, int Z, int P, int Q, long M, long xsn, long xsd,
-                          long xsh, long xsw, long osn, long osz, long osp, long osq, long rsn,
-                          long rsz, long rsp, long rsq, hipStream_t stream) {
+namespace {
+
+// conv3d_fwd and launch_conv3d (use_scratch: a split reduction's partial
+// results go to the static scratch) and conv3d_fwd_split (caller workspace).
+int conv3d_impl(const void* x, const void* w, const void* bias, const void* res, void* out, int nB,
+                int D, int H, int W, int C, int K, int T, int R, int S, int sd, int sh, int sw,
+                int Z, int P, int Q, long M, long xsn, long xsd, long xsh, long xsw, long osn,
+                long osz, long osp, long osq, long rsn, long rsz, long rsp, long rsq,
+                hipStream_t stream, void* workspace, size_t workspace_bytes, bool use_scratch) {
     g_err[0] = 0;
     if (nB <= 0 || D <= 0 || H <= 0 || W <= 0 || C <= 0 || K <= 0 || T <= 0 || R <= 0 || S <= 0)
         return fail("conv3d: sizes must be positive");
@@ -545,13 +688,69 @@ extern "C" int conv3d_fwd(const void* x, const void* w, const void* bias, const 
     a.rsq = rsq;
     a.x_bytes = (unsigned)x_span;
     a.w_bytes = (unsigned)w_span;
-    kKernels[pick_kernel(M, K, KG)].launch(a, stream);
-    const hipError_t e = hipGetLastError();
+    ConvPlan p = plan_conv(M, K, KG, kScratchBytes);
+    ScratchUse scratch;
+    if (p.nsplit > 1 && use_scratch) {
+        // A captured call takes no scratch (its replays could run beside other
+        // calls that use it) and runs unsplit.
+        const ScratchUse::Status st = scratch.acquire(stream, false);
+        if (st == ScratchUse::kFailed) {
+            set_err(scratch.error);
+            return 2;
+        }
+        if (st == ScratchUse::kUnavailable) p = plan_conv(M, K, KG, 0);
+        workspace = scratch.ptr;
+        workspace_bytes = kScratchBytes;
+    }
+    if (p.nsplit > 1 && (!workspace || workspace_bytes < conv_ws_bytes(p, M, K) ||
+                         (uintptr_t)workspace % 16))
+        return fail("conv3d: workspace missing, misaligned or smaller than "
+                    "conv3d_workspace_bytes()");
+    a.nsplit = p.nsplit;
+    a.split_len = p.split_len;
+    a.ws = (float*)workspace;
+    kKernels[p.cfg].launch(a, stream);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && p.nsplit > 1) {
+        const long threads = M * (K / 4);
+        hipLaunchKernelGGL(conv3d_reduce, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                           stream, a);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = scratch.release(stream);
     if (e != hipSuccess) {
         set_err(hipGetErrorString(e));
         return 2;
     }
     return 0;
+}
+
+}  // namespace
+
+extern "C" int conv3d_fwd(const void* x, const void* w, const void* bias, const void* res,
+                          void* out, int nB, int D, int H, int W, int C, int K, int T, int R, int S,
+                          int sd, int sh, int sw, int Z, int P, int Q, long M, long xsn, long xsd,
+                          long xsh, long xsw, long osn, long osz, long osp, long osq, long rsn,
+                          long rsz, long rsp, long rsq, hipStream_t stream) {
+    return conv3d_impl(x, w, bias, res, out, nB, D, H, W, C, K, T, R, S, sd, sh, sw, Z, P, Q, M,
+                       xsn, xsd, xsh, xsw, osn, osz, osp, osq, rsn, rsz, rsp, rsq, stream, nullptr,
+                       0, true);
+}
+
+extern "C" size_t conv3d_workspace_bytes(long M, int K, long KG) {
+    if (M <= 0 || K <= 0 || KG <= 0) return 0;
+    return conv_ws_bytes(plan_conv(M, K, KG, kScratchBytes), M, K);
+}
+
+extern "C" int conv3d_fwd_split(const void* x, const void* w, const void* bias, const void* res,
+                                void* out, int nB, int D, int H, int W, int C, int K, int T, int R,
+                                int S, int sd, int sh, int sw, int Z, int P, int Q, long M,
+                                long xsn, long xsd, long xsh, long xsw, long osn, long osz,
+                                long osp, long osq, long rsn, long rsz, long rsp, long rsq,
+                                hipStream_t stream, void* workspace, size_t workspace_bytes) {
+    return conv3d_impl(x, w, bias, res, out, nB, D, H, W, C, K, T, R, S, sd, sh, sw, Z, P, Q, M,
+                       xsn, xsd, xsh, xsw, osn, osz, osp, osq, rsn, rsz, rsp, rsq, stream,
+                       workspace, workspace_bytes, false);
 }
 
 extern "C" void launch_conv3d(const void* x, const void* w, const void* bias, const void* res,

@@ -1,0 +1,54 @@
+// Workspace of the C entry points that split a reduction without a caller
+// workspace (attn_fwd_split_static, launch / attn_fwd for grids too small for
+// the GPU, conv3d_fwd / launch_conv3d likewise). Internal to the library.
+//
+// The partial results live in a file-scope device array. It is part of the
+// library's code object, so every GPU on which any kernel of the library is
+// loaded holds its own copy (kScratchBytes) until the process ends, whether or
+// not a call ever uses it. The kernels write every workspace entry the merge
+// reads within the same call, so nothing is cleared between calls.
+//
+// Calls that use the array are ordered on the GPU, whatever streams they are
+// issued on: each records an event on its stream after its kernels, and a
+// call on another stream first makes its stream wait for that event (the host
+// lock keeps wait, launches and record of one call together, so the calls
+// form one chain per device). A call made under stream capture neither waits
+// nor records (an event recorded outside the graph cannot order its replays):
+// a graph that contains one is ordered only by the stream it is launched on,
+// and must not run concurrently with other calls that use the array on that
+// device.
+#pragma once
+
+#include <stddef.h>
+#include <hip/hip_runtime_api.h>
+#include <mutex>
+
+namespace gfx906_amd {
+
+constexpr size_t kScratchBytes = size_t(96) << 20;
+
+struct DevScratch;
+
+// One call's use of the scratch of its stream's device: acquire() before its
+// launches, release() after them; the lock is held in between.
+class ScratchUse {
+ public:
+    enum Status {
+        kReady,        // ptr is usable
+        kUnavailable,  // under capture: not allowed, or no call outside capture has set it up
+        kFailed,       // error: `error`, or the device index is beyond the table
+    };
+    ScratchUse();
+    Status acquire(hipStream_t stream, bool allow_capture);
+    hipError_t release(hipStream_t stream);  // no-op unless acquired
+
+    void* ptr = nullptr;
+    const char* error = nullptr;
+
+ private:
+    std::unique_lock<std::mutex> lock_;
+    DevScratch* dev_ = nullptr;
+    bool capturing_ = false;
+};
+
+}  // namespace gfx906_amd

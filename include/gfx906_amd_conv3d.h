@@ -19,6 +19,7 @@
 #ifndef GFX906_AMD_CONV3D_H
 #define GFX906_AMD_CONV3D_H
 
+#include <stddef.h>
 #include <hip/hip_runtime_api.h>
 
 #ifdef __cplusplus
@@ -49,6 +50,25 @@ int conv3d_fwd(const void* x, const void* w, const void* bias, const void* res, 
                long osn, long osz, long osp, long osq,
                long rsn, long rsz, long rsp, long rsq,
                hipStream_t stream);
+
+/* Problems with too few output tiles for the GPU split the reduction over
+ * more workgroups: each range's fp32 sums go to a workspace and a second
+ * kernel adds them up. launch_conv3d() and conv3d_fwd() keep them in the
+ * library's static scratch (attn_split_scratch_capacity() bytes; such calls
+ * are ordered across streams on one device, see gfx906_amd_attn.h) and do not
+ * split under stream capture. conv3d_fwd_split() takes a caller workspace
+ * instead (16-byte aligned, conv3d_workspace_bytes() bytes, with
+ * M = nB*Z*P*Q and KG = C*T*R*S; 0: not split) and needs no ordering. Both
+ * give the same bits. No counterpart in the reference. */
+size_t conv3d_workspace_bytes(long M, int K, long KG);
+int conv3d_fwd_split(const void* x, const void* w, const void* bias, const void* res, void* out,
+                     int nB, int D, int H, int W, int C, int K,
+                     int T, int R, int S, int sd, int sh, int sw,
+                     int Z, int P, int Q, long M,
+                     long xsn, long xsd, long xsh, long xsw,
+                     long osn, long osz, long osp, long osq,
+                     long rsn, long rsz, long rsp, long rsq,
+                     hipStream_t stream, void* workspace, size_t workspace_bytes);
 
 /* Message for the last failed launch_conv3d()/conv3d_fwd() on the calling
  * thread, or NULL if it succeeded. No counterpart in the reference. */
