@@ -109,11 +109,16 @@ struct KArgs {
     Strides sq, sk, sv, so;
     int H, Sq, Skv, D;
     float c, qsign;
-    // Split key range (kernels instantiated with SPLIT): workgroup split s of
-    // nsplit takes keys [s*split_len, (s+1)*split_len) and writes its
-    // unnormalised O (fp32) to ws_o[s][bh][row][0..D) and its (m, l) to
-    // ws_ml[s][bh][row][0..1]; attn_combine merges them.
-    int BH, nsplit, split_len;
+    // Split key range (kernels instantiated with SPLIT). Work units are the
+    // query tiles of all heads, head-major. The first `whole` units run
+    // unsplit (the rounds of workgroups that fill the GPU; 0 when none does),
+    // the other `tail` units in nsplit workgroups each: split s takes keys
+    // [s*split_len, (s+1)*split_len) and writes its unnormalised O (fp32) to
+    // ws_o[s][r][0..D) and its (m, l) to ws_ml[s][r][0..1], r < tail_rows the
+    // row's place (head-major) among the tail's, which start at row0;
+    // attn_combine merges them.
+    int BH, nsplit, split_len, whole, tail;
+    long long row0, tail_rows;
     float* ws_o;
     float* ws_ml;
     // Every output row starts 16-byte aligned (o and its batch, head and
@@ -133,6 +138,44 @@ struct KArgs {
     // starts after them into L2).
     int ncu;
 };
+
+// What a workgroup works on: query tile qt of head bh; with SPLIT, key range
+// `split` of it when `part` is set, all its keys otherwise.
+struct WorkItem {
+    int qt, bh, split;
+    bool part;
+};
+// Work item of workgroup blk of a grid of n. The dispatcher deals workgroup w
+// to XCD w % 8; where the count divides by 8, consecutive items go to one XCD,
+// and items enumerate the query tiles of one key range consecutively, so that
+// an XCD's L2 streams the K/V of as few heads (or key ranges) as possible
+// (c2 +2 %).
+__device__ __forceinline__ int xcd_order(int w, int n) {
+    return (n & 7) == 0 ? (w & 7) * (n >> 3) + (w >> 3) : w;
+}
+template <bool SPLIT, bool TAIL>
+__device__ __forceinline__ WorkItem work_item(const KArgs& a, int blk, int n, int nqt) {
+    WorkItem it;
+    it.split = 0;
+    it.part = false;
+    int unit;
+    if constexpr (SPLIT) {
+        const int whole = TAIL ? a.whole : 0;
+        if (blk < whole) {
+            unit = xcd_order(blk, whole);
+        } else {
+            const int w = xcd_order(blk - whole, n - whole);
+            it.split = w / a.tail;
+            unit = whole + (w - it.split * a.tail);
+            it.part = true;
+        }
+    } else {
+        unit = xcd_order(blk, n);
+    }
+    it.bh = unit / nqt;
+    it.qt = unit - it.bh * nqt;
+    return it;
+}
 
 #if defined(__HIP_DEVICE_COMPILE__)
 // Per-element-type operations: vectors, MFMAs, packed RNE conversion from
@@ -279,6 +322,24 @@ __device__ __forceinline__ int lane_id_here() {
     return x;
 }
 
+// The kernel's arguments, read again where the epilogue uses them: behind an
+// asm the compiler cannot see through, so that it loads them there instead of
+// keeping them (or what it derives from them) in SGPRs across the main loop.
+// The TAIL kernels, whose two epilogues together need more than the other
+// kernels' one, spilled such values around the loop otherwise.
+__device__ __forceinline__ const KArgs& args_here() {
+    auto p = (const __attribute__((address_space(4))) KArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const KArgs*)p;
+}
+
+// The workgroup's index, likewise.
+__device__ __forceinline__ int block_here() {
+    int x = blockIdx.x;
+    asm volatile("" : "+s"(x));
+    return x;
+}
+
 // Sum / max over lanes i, i+16, i+32, i+48.
 __device__ __forceinline__ float quad_group_sum(float x) {
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
@@ -406,6 +467,14 @@ struct Cfg {
     static constexpr int BLKS = TILE / 1024;    // 1 KB direct-load blocks per tile
     static_assert(BLKS % NW == 0, "tile must split evenly over waves");
     static_assert(DP % 32 == 0 && DP <= 128, "head-dim class");
+    static constexpr bool TAIL = false;
+};
+// SPLIT kernels for a grid whose first units run unsplit (KArgs::whole > 0).
+// Instantiations of their own: the second epilogue and the arguments read
+// again for it cost a small split grid 3 % (B1 H1 S1024 D64 13.4 -> 13.8 us).
+template <int DP_, int NW_, int OCC_>
+struct CfgTail : Cfg<DP_, NW_, OCC_> {
+    static constexpr bool TAIL = true;
 };
 
 // Per-lane byte offsets of the direct HBM->LDS tile loads. Each wave fills
@@ -497,9 +566,8 @@ __device__ __forceinline__ void block_exp(const f32x4& S0, const f32x4& S1,
 }
 #endif
 
-// grid: ceil(Sq / BM) * B*H (* nsplit with SPLIT) workgroups, query tiles of
-// one head adjacent (the splits of one query tile adjacent); block: NW*64
-// threads. The second launch bound is HIP's minimum waves per SIMD
+// grid: ceil(Sq / BM) * B*H workgroups (SPLIT: whole + tail * nsplit), query
+// tiles of one head adjacent, see work_item; block: NW*64 threads. The second launch bound is HIP's minimum waves per SIMD
 // (amdgpu_waves_per_eu): OCC workgroups of NW waves over the CU's four SIMDs.
 template <class C, bool PAD, class T, bool SPLIT, bool TILEMAX>
 __global__ void __launch_bounds__(C::NT, C::OCC * C::NW / 4)
@@ -532,22 +600,12 @@ attn_fwd_pipe(const KArgs a) {
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i = lane & 15, g = lane >> 4;
     const int nqt = (Sq + C::BM - 1) / C::BM;
-    // Work item w = (head, key split, query tile), query tiles consecutive;
-    // consecutive items go to one XCD when the grid divides by 8 (the
-    // dispatcher deals workgroup w to XCD w % 8), so an XCD's L2 streams the
-    // K/V of as few heads as possible (c2 +2 %).
-    int w = blockIdx.x;
-    if ((gridDim.x & 7) == 0) w = (w & 7) * (int)(gridDim.x >> 3) + (w >> 3);
-    const int qt = w % nqt;
-    int bh = w / nqt, split = 0;
-    if constexpr (SPLIT) {
-        split = bh % a.nsplit;
-        bh /= a.nsplit;
-    }
+    const WorkItem it = work_item<SPLIT, C::TAIL>(a, blockIdx.x, gridDim.x, nqt);
+    const int qt = it.qt, bh = it.bh;
     const int b = bh / a.H, h = bh - b * a.H;
     // This workgroup's keys: [kv0, kv0 + Skv) of the head.
-    const int kv0 = SPLIT ? split * a.split_len : 0;
-    const int Skv = SPLIT ? max(0, min(a.Skv - kv0, a.split_len)) : a.Skv;
+    const int kv0 = SPLIT ? it.split * a.split_len : 0;
+    const int Skv = (SPLIT && !C::TAIL) || it.part ? max(0, min(a.Skv - kv0, a.split_len)) : a.Skv;
     const T* Qh = (const T*)a.q + b * a.sq.b + h * a.sq.h;
     const T* Kh = (const T*)a.k + b * a.sk.b + h * a.sk.h + kv0 * a.sk.s;
     const T* Vh = (const T*)a.v + b * a.sv.b + h * a.sv.h + kv0 * a.sv.s;
@@ -679,11 +737,8 @@ attn_fwd_pipe(const KArgs a) {
             int bytes = 0, off = 0;
             if (resident > 0 && (resident & 7) == 0 && nb < (long long)gridDim.x &&
                 span < (1LL << 31)) {  // (uniform)
-                int w2 = (int)nb;
-                if ((gridDim.x & 7) == 0) w2 = (w2 & 7) * (int)(gridDim.x >> 3) + (w2 >> 3);
-                const int qt2 = w2 % nqt;
-                int bh2 = w2 / nqt;
-                if constexpr (SPLIT) bh2 /= a.nsplit;
+                const WorkItem next = work_item<SPLIT, C::TAIL>(a, (int)nb, gridDim.x, nqt);
+                const int qt2 = next.qt, bh2 = next.bh;
                 const int b2 = bh2 / a.H, h2 = bh2 - b2 * a.H;
                 const int rows = min(Sq - qt2 * C::BM, C::BM);
                 bytes = (int)((rows - 1) * a.sq.s * 2 + D * 2);
@@ -1015,33 +1070,41 @@ attn_fwd_pipe(const KArgs a) {
     // Lane indices of the epilogue. D <= 64 runs at 128 VGPRs, and values
     // kept from the prologue would hold registers across the main loop (two
     // were spilled around it): they are recomputed from the lane id.
+    // TAIL kernels take everything else they use again from the arguments.
+    const KArgs& ea = C::TAIL ? args_here() : a;
+    const int Sqe = ea.Sq, De = ea.D;
+    const WorkItem ite =
+        C::TAIL ? work_item<SPLIT, C::TAIL>(ea, block_here(), gridDim.x, (Sqe + C::BM - 1) / C::BM) : it;
+    const int be = C::TAIL ? ite.bh / ea.H : b, he = C::TAIL ? ite.bh - be * ea.H : h;
+    T* const Oe = C::TAIL ? (T*)ea.o + be * ea.so.b + he * ea.so.h : Oh;
     int lane_e = lane, ie = i, ge = g, qrow0e = qrow0;
-    if constexpr (DP <= 64) {
+    if constexpr (DP <= 64 || C::TAIL) {
         lane_e = lane_id_here();
         ie = lane_e & 15;
         ge = lane_e >> 4;
-        qrow0e = qt * C::BM + wave * 32 + ie;
+        qrow0e = ite.qt * C::BM + wave * 32 + ie;
     }
-    if constexpr (SPLIT) {  // unnormalised O and (m, l) of this key range
+    if ((SPLIT && !C::TAIL) || ite.part) {  // unnormalised O and (m, l) of this key range
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
             const int row = qrow0e + 16 * nb;
             const float l = quad_group_sum(lacc[nb][0]);
-            if (row < Sq) {
-                const long long r = ((long long)split * a.BH + bh) * Sq + row;
-                float* wo = a.ws_o + r * D;
+            if (row < Sqe) {
+                const long long r = ite.split * ea.tail_rows +
+                                    ((long long)ite.bh * Sqe + row - (C::TAIL ? ea.row0 : 0));
+                float* wo = ea.ws_o + r * De;
 #pragma unroll
                 for (int ob = 0; ob < NOB; ++ob) {
                     const int d0 = 16 * ob + 4 * ge;
-                    if (!PAD || d0 < D) *reinterpret_cast<f32x4*>(wo + d0) = oacc[ob][nb];
+                    if (!PAD || d0 < De) *reinterpret_cast<f32x4*>(wo + d0) = oacc[ob][nb];
                 }
-                const float m = kLazy ? m_run[nb] : m_run[nb] * c;  // log2 units
-                if (ge == 0) *reinterpret_cast<f32x2*>(a.ws_ml + 2 * r) = f32x2{m, l};
+                const float m = kLazy ? m_run[nb] : m_run[nb] * ea.c;  // log2 units
+                if (ge == 0) *reinterpret_cast<f32x2*>(ea.ws_ml + 2 * r) = f32x2{m, l};
             }
         }
         return;
     }
-    if (!PAD && a.o16) {
+    if (!PAD && ea.o16) {
         // O through LDS: each wave writes its rows, in the element type, to a
         // row-major staging area (rows padded by 16 bytes) in the ring it no
         // longer reads, then stores them as 16-byte pieces of consecutive
@@ -1072,11 +1135,11 @@ attn_fwd_pipe(const KArgs a) {
             const int cidx = 64 * j + lane_e, r = cidx / CPR, col = cidx - r * CPR;
             const u32x4 val = *reinterpret_cast<const LDS_AS u32x4*>((const LDS_AS char*)stg +
                                                                      r * RS + col * 16);
-            if (row0 + r < Sq) {
+            if (row0 + r < Sqe) {
                 // D <= 64: non-temporal stores (O is not read again; c3, whose
                 // three rounds of short workgroups store 50 MB, +1.4 %; D = 128
                 // mixed, -0.6 % north star, +1 % c2: not used there).
-                u32x4* dst = reinterpret_cast<u32x4*>(Oh + (row0 + r) * a.so.s + col * 8);
+                u32x4* dst = reinterpret_cast<u32x4*>(Oe + (row0 + r) * ea.so.s + col * 8);
                 if constexpr (DP <= 64)
                     __builtin_nontemporal_store(val, dst);
                 else
@@ -1090,12 +1153,12 @@ attn_fwd_pipe(const KArgs a) {
         const int row = qrow0e + 16 * nb;
         const float l = quad_group_sum(lacc[nb][0]);
         const float inv = l > 0.f ? 1.f / l : 0.f;
-        if (row < Sq) {
-            T* op = Oh + row * a.so.s;
+        if (row < Sqe) {
+            T* op = Oe + row * ea.so.s;
 #pragma unroll
             for (int ob = 0; ob < NOB; ++ob) {
                 const int d0 = 16 * ob + 4 * ge;
-                if (!PAD || d0 < D) {
+                if (!PAD || d0 < De) {
                     const auto h0 = E::cvt2(oacc[ob][nb][0] * inv, oacc[ob][nb][1] * inv);
                     const auto h1 = E::cvt2(oacc[ob][nb][2] * inv, oacc[ob][nb][3] * inv);
                     *reinterpret_cast<typename E::x4*>(op + d0) =
@@ -1698,7 +1761,7 @@ attn_fwd_d512(const KArgs a) {
     const float l = quad_group_sum(l_run);
     if constexpr (SPLIT) {  // unnormalised O and (m, l) of this key range
         if (live) {
-            const long long r = ((long long)split * a.BH + bh) * Sq + qrow;
+            const long long r = split * a.tail_rows + ((long long)bh * Sq + qrow);
             float* wo = a.ws_o + r * D;
 #pragma unroll
             for (int ob = 0; ob < NOB; ++ob) *reinterpret_cast<f32x4*>(wo + 16 * ob + 4 * g) = oacc[ob];
@@ -1783,22 +1846,11 @@ attn_fwd_d512w(const KArgs a) {
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i = lane & 15, g = lane >> 4;
     const int nqt = (Sq + C::BM - 1) / C::BM;
-    // Workgroup w runs on XCD w % 8 (the dispatcher deals workgroups to the
-    // eight XCDs in turn). When the grid divides by 8, consecutive work items
-    // go to one XCD, and work items enumerate the query tiles of one K/V range
-    // (head, split) consecutively: an XCD's L2 then streams the K/V of as few
-    // heads as possible, each tile once for all its workgroups.
-    int w = blockIdx.x;
-    if ((gridDim.x & 7) == 0) w = (w & 7) * (int)(gridDim.x >> 3) + (w >> 3);
-    const int qt = w % nqt;
-    int bh = w / nqt, split = 0;
-    if constexpr (SPLIT) {
-        split = bh % a.nsplit;
-        bh /= a.nsplit;
-    }
+    const WorkItem it = work_item<SPLIT, true>(a, blockIdx.x, gridDim.x, nqt);
+    const int qt = it.qt, bh = it.bh;
     const int b = bh / a.H, h = bh - b * a.H;
-    const int kv0 = SPLIT ? split * a.split_len : 0;
-    const int Skv = SPLIT ? max(0, min(a.Skv - kv0, a.split_len)) : a.Skv;
+    const int kv0 = SPLIT ? it.split * a.split_len : 0;
+    const int Skv = SPLIT && it.part ? max(0, min(a.Skv - kv0, a.split_len)) : a.Skv;
     const T* Qh = (const T*)a.q + b * a.sq.b + h * a.sq.h;
     const T* Kh = (const T*)a.k + b * a.sk.b + h * a.sk.h + kv0 * a.sk.s;
     const T* Vh = (const T*)a.v + b * a.sv.b + h * a.sv.h + kv0 * a.sv.s;
@@ -2079,22 +2131,28 @@ attn_fwd_d512w(const KArgs a) {
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
     const int ie = lane_e & 15, ge = lane_e >> 4;
-    const int row0 = qt * C::BM + wave * 32;  // this wave's first row
-    const bool staged = !SPLIT && a.o16;
+    const KArgs& ea = SPLIT ? args_here() : a;  // (see args_here)
+    const int Sqe = ea.Sq;
+    const WorkItem& ite = it;
+    T* const Oe = SPLIT ? (T*)ea.o + b * ea.so.b + h * ea.so.h : Oh;
+    const int row0 = ite.qt * C::BM + wave * 32;  // this wave's first row
+    const bool part = SPLIT && ite.part;
+    const bool staged = !part && ea.o16;
     if (staged) lds_barrier();  // every wave is done with the ring
     char* const stg = wave == 0 ? kb0 : wave == 1 ? kb1 : wave == 2 ? vb0 : vb1;
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
         const int qrow = row0 + 16 * rb + ie;
         const float l = quad_group_sum(l_run[rb]);
-        if constexpr (SPLIT) {  // unnormalised O and (m, l) of this key range
-            if (qrow < Sq) {
-                const long long r = ((long long)split * a.BH + bh) * Sq + qrow;
-                float* wo = a.ws_o + r * D;
+        if (part) {  // unnormalised O and (m, l) of this key range
+            if (qrow < Sqe) {
+                const long long r =
+                    ite.split * ea.tail_rows + ((long long)ite.bh * Sqe + qrow - ea.row0);
+                float* wo = ea.ws_o + r * D;
 #pragma unroll
                 for (int ob = 0; ob < NOB; ++ob)
                     *reinterpret_cast<f32x4*>(wo + 16 * ob + 4 * ge) = oacc[rb][ob];
-                if (ge == 0) *reinterpret_cast<f32x2*>(a.ws_ml + 2 * r) = f32x2{m_run[rb], l};
+                if (ge == 0) *reinterpret_cast<f32x2*>(ea.ws_ml + 2 * r) = f32x2{m_run[rb], l};
             }
         } else if (staged) {
             constexpr int RS = D * 2 + 16;
@@ -2110,8 +2168,8 @@ attn_fwd_d512w(const KArgs a) {
             }
         } else {
             const float inv = l > 0.f ? 1.f / l : 0.f;
-            if (qrow < Sq) {
-                T* op = Oh + qrow * a.so.s;
+            if (qrow < Sqe) {
+                T* op = Oe + qrow * ea.so.s;
 #pragma unroll
                 for (int ob = 0; ob < NOB; ++ob) {
                     const auto h0 = E::cvt2(oacc[rb][ob][0] * inv, oacc[rb][ob][1] * inv);
@@ -2122,18 +2180,16 @@ attn_fwd_d512w(const KArgs a) {
             }
         }
     }
-    if constexpr (!SPLIT) {
-        if (staged) {
-            constexpr int RS = D * 2 + 16;
-            constexpr int CPR = D * 2 / 16;  // 16-byte pieces per row (one per lane)
-            static_assert(CPR == 64, "one row per store instruction");
+    if (staged) {
+        constexpr int RS = D * 2 + 16;
+        constexpr int CPR = D * 2 / 16;  // 16-byte pieces per row (one per lane)
+        static_assert(CPR == 64, "one row per store instruction");
 #pragma unroll
-            for (int r = 0; r < 32; ++r) {
-                const u32x4 val = *reinterpret_cast<const LDS_AS u32x4*>(
-                    (const LDS_AS char*)stg + r * RS + lane_e * 16);
-                if (row0 + r < Sq)
-                    *reinterpret_cast<u32x4*>(Oh + (row0 + r) * a.so.s + lane_e * 8) = val;
-            }
+        for (int r = 0; r < 32; ++r) {
+            const u32x4 val = *reinterpret_cast<const LDS_AS u32x4*>(
+                (const LDS_AS char*)stg + r * RS + lane_e * 16);
+            if (row0 + r < Sqe)
+                *reinterpret_cast<u32x4*>(Oe + (row0 + r) * ea.so.s + lane_e * 8) = val;
         }
     }
 #endif
@@ -2153,7 +2209,8 @@ struct CombArgs {
     const float* ws_ml;
     void* o;
     Strides so;
-    int H, Sq, D, BH, nsplit;
+    int H, Sq, D, nsplit;
+    long long row0, rows;  // the split rows: [row0, row0 + rows) of all heads' rows
 };
 
 template <class T>
@@ -2161,7 +2218,7 @@ __global__ void __launch_bounds__(256) attn_combine(const CombArgs c) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using E = Elem<T>;
     const int dq = c.D / 4;
-    const long long rows = (long long)c.BH * c.Sq;
+    const long long rows = c.rows;
     const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
     if (idx >= rows * dq) return;
     const long long row = idx / dq;
@@ -2201,7 +2258,8 @@ __global__ void __launch_bounds__(256) attn_combine(const CombArgs c) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
     const auto h0 = E::cvt2(acc[0] * inv, acc[1] * inv);
     const auto h1 = E::cvt2(acc[2] * inv, acc[3] * inv);
-    const int bh = (int)(row / c.Sq), srow = (int)(row - (long long)bh * c.Sq);
+    const long long grow = c.row0 + row;
+    const int bh = (int)(grow / c.Sq), srow = (int)(grow - (long long)bh * c.Sq);
     const int b = bh / c.H, h = bh - b * c.H;
     T* op = (T*)c.o + b * c.so.b + h * c.so.h + srow * c.so.s + d0 * c.so.d;
     if (c.so.d == 1 && (reinterpret_cast<uintptr_t>(op) & 7) == 0) {
@@ -2228,6 +2286,11 @@ using Cfg64 = Cfg<64, 8, 2>;    // 64 KB: two workgroups, four waves per SIMD
 
 int cu_count();
 
+// Query rows per workgroup (a work unit) of the ring and D = 512 kernels.
+int query_tile(int D) { return D == 512 ? Cfg512::BM : D == 128 ? Cfg128::BM : Cfg64::BM; }
+
+constexpr int kKvresMaxKeys = CfgRes::MAX_TILES * CfgRes::BN;  // 640
+
 // Query tiles of the K/V-resident kernel.
 long long kvres_items(const KArgs& a) {
     return (long long)a.BH * ((a.Sq + CfgRes::BM - 1) / CfgRes::BM);
@@ -2242,7 +2305,7 @@ long long kvres_items(const KArgs& a) {
 // kernel, 1 = resident kernel whatever the tile count, n > 1 = resident
 // kernel on at most n workgroups (several tiles, and heads, per workgroup).
 long long kvres_grid(const KArgs& a) {
-    if (a.D > 64 || a.Skv < 1 || a.Skv > CfgRes::MAX_TILES * CfgRes::BN) return 0;
+    if (a.D > 64 || a.Skv < 1 || a.Skv > kKvresMaxKeys) return 0;
     const long long items = kvres_items(a), cus = cu_count();
     const char* env = getenv("GFX906_AMD_ATTN_KVRES");
     const long long force = env ? atoll(env) : -1;
@@ -2279,33 +2342,53 @@ bool tile_max(int keys) {
     return keys <= kTileMaxKeys;
 }
 
+// The ring kernels' whole units and split tail.
+template <class T>
+void launch_tail(const KArgs& a, dim3 grid, hipStream_t s) {
+    using C128 = CfgTail<128, 8, 1>;
+    using C64 = CfgTail<64, 8, 2>;
+    const bool tm = tile_max(a.Skv);
+    if (a.D == 128)
+        hipLaunchKernelGGL((attn_fwd_pipe<C128, false, T, true, false>), grid, dim3(C128::NT), 0, s,
+                           a);
+    else if (a.D == 64 && tm)
+        hipLaunchKernelGGL((attn_fwd_pipe<C64, false, T, true, true>), grid, dim3(C64::NT), 0, s, a);
+    else if (a.D == 64)
+        hipLaunchKernelGGL((attn_fwd_pipe<C64, false, T, true, false>), grid, dim3(C64::NT), 0, s, a);
+    else if (tm)
+        hipLaunchKernelGGL((attn_fwd_pipe<C64, true, T, true, true>), grid, dim3(C64::NT), 0, s, a);
+    else
+        hipLaunchKernelGGL((attn_fwd_pipe<C64, true, T, true, false>), grid, dim3(C64::NT), 0, s, a);
+}
+
 template <class T, bool SPLIT>
-void launch_kernel(const KArgs& a, unsigned nwg, bool tl, hipStream_t s) {
+void launch_kernel(const KArgs& a, bool tl, hipStream_t s) {
     const int D = a.D;
+    const unsigned units = (unsigned)((a.Sq + query_tile(D) - 1) / query_tile(D)) * (unsigned)a.BH;
+    const dim3 grid(SPLIT ? (unsigned)a.whole + (unsigned)a.tail * (unsigned)a.nsplit : units);
     if (D == 512) {
-        dim3 grid((unsigned)((a.Sq + Cfg512::BM - 1) / Cfg512::BM) * nwg);
         if (tl)
             hipLaunchKernelGGL((attn_fwd_d512<T, true, SPLIT>), grid, dim3(Cfg512::NT), 0, s, a);
         else if (d512_wide())
             hipLaunchKernelGGL((attn_fwd_d512w<T, SPLIT>), grid, dim3(Cfg512W::NT), 0, s, a);
         else
             hipLaunchKernelGGL((attn_fwd_d512<T, false, SPLIT>), grid, dim3(Cfg512::NT), 0, s, a);
+    } else if (SPLIT && a.whole > 0) {
+        launch_tail<T>(a, grid, s);
     } else if (D == 128) {
-        dim3 grid((unsigned)((a.Sq + Cfg128::BM - 1) / Cfg128::BM) * nwg);
         hipLaunchKernelGGL((attn_fwd_pipe<Cfg128, false, T, SPLIT, false>), grid, dim3(Cfg128::NT),
                            0, s, a);
     } else {
         if constexpr (!SPLIT) {
             if (const long long wgs = kvres_grid(a)) {
-                const dim3 grid((unsigned)wgs);
+                const dim3 res((unsigned)wgs);
                 if (D == 64)
-                    hipLaunchKernelGGL((attn_fwd_kvres<false, T>), grid, dim3(CfgRes::NT), 0, s, a);
+                    hipLaunchKernelGGL((attn_fwd_kvres<false, T>), res, dim3(CfgRes::NT), 0, s, a);
                 else
-                    hipLaunchKernelGGL((attn_fwd_kvres<true, T>), grid, dim3(CfgRes::NT), 0, s, a);
+                    hipLaunchKernelGGL((attn_fwd_kvres<true, T>), res, dim3(CfgRes::NT), 0, s, a);
                 return;
             }
         }
-        dim3 grid((unsigned)((a.Sq + Cfg64::BM - 1) / Cfg64::BM) * nwg);
         const bool tm = tile_max(SPLIT ? a.split_len : a.Skv);
         if (D == 64 && tm)
             hipLaunchKernelGGL((attn_fwd_pipe<Cfg64, false, T, SPLIT, true>), grid, dim3(Cfg64::NT),
@@ -2327,10 +2410,10 @@ void launch_kernel(const KArgs& a, unsigned nwg, bool tl, hipStream_t s) {
 template <class T>
 hipError_t launch_t(const KArgs& a, bool tl, hipStream_t s) {
     if (a.nsplit <= 1) {
-        launch_kernel<T, false>(a, (unsigned)a.BH, tl, s);
+        launch_kernel<T, false>(a, tl, s);
         return hipGetLastError();
     }
-    launch_kernel<T, true>(a, (unsigned)a.BH * (unsigned)a.nsplit, tl, s);
+    launch_kernel<T, true>(a, tl, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     CombArgs c;
@@ -2341,9 +2424,10 @@ hipError_t launch_t(const KArgs& a, bool tl, hipStream_t s) {
     c.H = a.H;
     c.Sq = a.Sq;
     c.D = a.D;
-    c.BH = a.BH;
     c.nsplit = a.nsplit;
-    const long long threads = (long long)a.BH * a.Sq * (a.D / 4);
+    c.row0 = a.row0;
+    c.rows = a.tail_rows;
+    const long long threads = a.tail_rows * (a.D / 4);
     hipLaunchKernelGGL((attn_combine<T>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s,
                        c);
     return hipGetLastError();
@@ -2375,10 +2459,33 @@ int cu_count() {
 constexpr double kSplitFixedTiles = 2.0;
 constexpr double kSplitAloneRate = 0.7;
 constexpr double kSplitTileBytes = 11.0e6;
+//
+// A grid that fills the slots a whole number of times and a little more runs
+// its last round nearly empty: those whole rounds then run unsplit and only
+// the units past them (the tail) are split, by the same estimate. 16 heads of
+// 4250 queries, D = 128, are 272 units on 256 slots: two rounds before (206
+// us), one and a third with the last 16 units in 9 ranges each (139 us). A
+// tail costs more fixed time than a grid that is split from the start (its
+// workgroups start cold behind the whole rounds and the merge waits for them
+// alone: 9 us of workgroup start and end, 6 us of merge and 2 of its launch
+// there). The partial results are the tail's only, so they stay small (held
+// under the static scratch, so that every entry point makes the same plan).
+// A split tail has to save kTailMargin of the whole run time.
+constexpr double kTailFixedTiles = 5.0;
+constexpr double kTailMergeTiles = 4.0;
+constexpr double kTailMargin = 0.03;
 struct SplitPlan {
     int nsplit, split_len;
+    int whole;  // leading units that run unsplit
 };
+constexpr SplitPlan kNoSplit{1, 0, 0};
 size_t split_ws_bytes(const SplitPlan& p, int B, int H, int Sq, int D);
+
+// First row (of all heads' rows, head-major) past `whole` units.
+long long first_split_row(int whole, int Sq, int D) {
+    const int bm = query_tile(D), nqt = (Sq + bm - 1) / bm;
+    return (long long)(whole / nqt) * Sq + (long long)(whole % nqt) * bm;
+}
 // ws_cap bounds the workspace of the chosen plan (the static scratch's size
 // for callers that pass none); counts whose partial results do not fit are
 // skipped, down to no split at all. GFX906_AMD_ATTN_NSPLIT=n (tests) asks
@@ -2386,49 +2493,63 @@ size_t split_ws_bytes(const SplitPlan& p, int B, int H, int Sq, int D);
 // as there are key tiles at most, fewer where n does not divide them into
 // non-empty ranges of whole tiles (the same rule as below), and no split
 // when n = 1 or when the partial results would not fit ws_cap.
-SplitPlan plan_split(int B, int H, int Sq, int Skv, int D, size_t ws_cap = (size_t)-1) {
-    const int bm = D == 512 ? Cfg512::BM : (D == 128 ? Cfg128::BM : Cfg64::BM);
+// tail: whether the call can run a split tail after whole rounds (the kernels
+// of the token-contiguous layout and of 16 rows per wave cannot, and the
+// K/V-resident kernel balances its items itself).
+SplitPlan plan_split(int B, int H, int Sq, int Skv, int D, bool tail,
+                     size_t ws_cap = (size_t)-1) {
+    const int bm = query_tile(D);
     const int bn = D == 512 ? Cfg512::BN : Cfg128::BN;
     const int per_cu = D == 512 || D == 128 ? 1 : 2;
     const long long units = (long long)B * H * ((Sq + bm - 1) / bm);
-    if (Skv == 0 || units == 0) return {1, 0};
+    if (Skv == 0 || units == 0) return kNoSplit;
     const int tiles = (Skv + bn - 1) / bn;
     if (const char* env = getenv("GFX906_AMD_ATTN_NSPLIT")) {
         const long long n = atoll(env);
         if (n >= 1) {
             const int per = (int)((tiles + std::min<long long>(n, tiles) - 1) /
                                   std::min<long long>(n, tiles));
-            const SplitPlan p{(tiles + per - 1) / per, per * bn};
-            return p.nsplit > 1 && split_ws_bytes(p, B, H, Sq, D) <= ws_cap ? p : SplitPlan{1, 0};
+            const SplitPlan p{(tiles + per - 1) / per, per * bn, 0};
+            return p.nsplit > 1 && split_ws_bytes(p, B, H, Sq, D) <= ws_cap ? p : kNoSplit;
         }
     }
-    const long long slots = (long long)cu_count() * per_cu;
-    if (units >= slots) return {1, 0};
-    const double partial_bytes = 2.0 * B * H * (double)Sq * D * 4;  // per split
-    const long long cus = cu_count();
+    const long long cus = cu_count(), slots = cus * per_cu;
+    const long long whole = units / slots * slots, split_units = units - whole;
+    if (split_units == 0 || (whole > 0 && (!tail || (D <= 64 && Skv <= kKvresMaxKeys))))
+        return kNoSplit;
+    if (whole > 0) ws_cap = std::min(ws_cap, kScratchBytes);
+    const double partial_bytes =
+        2.0 * ((double)B * H * Sq - first_split_row((int)whole, Sq, D)) * D * 4;  // per split
     const int step = D == 512 ? 2 : 4;
+    // The split units' part of the run time.
     auto estimate = [&](int ns, int per) {
-        const long long wgs = units * ns, rounds = (wgs + slots - 1) / slots;
+        const long long wgs = split_units * ns, rounds = (wgs + slots - 1) / slots;
         const double rate = per_cu == 2 && wgs <= cus ? kSplitAloneRate : 1.0;
         const int run = (per + step - 1) / step * step;
-        return rounds * (run + kSplitFixedTiles) * rate +
-               (ns > 1 ? ns * partial_bytes / kSplitTileBytes : 0.0);
+        const double fixed = whole && ns > 1 ? kTailFixedTiles : kSplitFixedTiles;
+        return rounds * (run + fixed) * rate +
+               (ns > 1 ? ns * partial_bytes / kSplitTileBytes + (whole ? kTailMergeTiles : 0.0)
+                       : 0.0);
     };
-    SplitPlan best{1, 0};
+    SplitPlan best = kNoSplit;
     double best_t = estimate(1, tiles);
+    if (whole > 0)  // the margin is on the whole run time
+        best_t -= kTailMargin *
+                  (best_t + whole / slots * ((tiles + step - 1) / step * step + kSplitFixedTiles));
     // The search stops at eight times the count that fills the slots once
     // (eight rounds of workgroups), and at 1024 splits (a few microseconds of
     // host time per call at most).
-    const long long fill = (slots + units - 1) / units;
+    const long long fill = (slots + split_units - 1) / split_units;
     const int max_ns = (int)std::min<long long>(std::min<long long>(tiles / 4, 8 * fill), 1024);
     for (int ns = 2; ns <= max_ns; ++ns) {
         const int per = (tiles + ns - 1) / ns;  // tiles per split
         if ((tiles + per - 1) / per != ns) continue;  // would leave a split empty
-        if (split_ws_bytes({ns, per * bn}, B, H, Sq, D) > ws_cap) break;  // grows with ns
+        const SplitPlan p{ns, per * bn, (int)whole};
+        if (split_ws_bytes(p, B, H, Sq, D) > ws_cap) break;  // grows with ns
         const double t = estimate(ns, per);
         if (t < best_t) {
             best_t = t;
-            best = {ns, per * bn};
+            best = p;
         }
     }
     return best;
@@ -2436,7 +2557,8 @@ SplitPlan plan_split(int B, int H, int Sq, int Skv, int D, size_t ws_cap = (size
 
 size_t split_ws_bytes(const SplitPlan& p, int B, int H, int Sq, int D) {
     if (p.nsplit <= 1) return 0;
-    const size_t rows = (size_t)p.nsplit * B * H * Sq;
+    const size_t rows =
+        (size_t)p.nsplit * ((long long)B * H * Sq - first_split_row(p.whole, Sq, D));
     return rows * D * 4 + rows * 2 * 4 + 16;
 }
 
@@ -2588,14 +2710,30 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     a.o16 = (uintptr_t)o % 16 == 0 && so.b % 8 == 0 && so.h % 8 == 0 && so.s % 8 == 0 && so.d == 1;
     a.q_lds = sq.s <= (1LL << 24) && Skv > (D == 128 ? 256 : 1024);
     a.ncu = cu_count();
-    SplitPlan p{1, 0};
+    a.whole = 0;
+    a.tail = 0;
+    a.row0 = 0;
+    a.tail_rows = (long long)B * H * Sq;
+    const bool tl = token_contiguous(sk, sv, D);
+    SplitPlan p = kNoSplit;
     if (workspace_bytes != (size_t)-1)  // split the keys if it pays
-        p = plan_split(B, H, Sq, Skv, D, use_scratch ? kScratchBytes : (size_t)-1);
-    const size_t need = split_ws_bytes(p, B, H, Sq, D);
+        p = plan_split(B, H, Sq, Skv, D, !tl && (D != 512 || d512_wide()),
+                       use_scratch ? kScratchBytes : (size_t)-1);
+    size_t need = split_ws_bytes(p, B, H, Sq, D);
+    // A grid that fills the GPU needs no workspace: without one (under
+    // capture, where the static scratch would tie the graph's replays to
+    // other calls, or from the caller) its tail runs unsplit.
+    if (p.whole > 0 && !use_scratch && (!workspace || workspace_bytes < need)) {
+        p = kNoSplit;
+        need = 0;
+    }
     ScratchUse scratch;
     if (need && use_scratch) {
-        const ScratchUse::Status st = scratch.acquire(stream, true);
-        if (st == ScratchUse::kUnavailable)
+        const ScratchUse::Status st = scratch.acquire(stream, p.whole == 0);
+        if (st == ScratchUse::kUnavailable && p.whole > 0) {
+            p = kNoSplit;
+            need = 0;
+        } else if (st == ScratchUse::kUnavailable)
             return fail("attn: the static scratch of this device is set up by the first call "
                         "that splits outside stream capture; make one such call before "
                         "capturing");
@@ -2614,10 +2752,13 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
         }
         a.nsplit = p.nsplit;
         a.split_len = p.split_len;
+        a.whole = p.whole;
+        a.tail = B * H * ((Sq + query_tile(D) - 1) / query_tile(D)) - p.whole;
+        a.row0 = first_split_row(p.whole, Sq, D);
+        a.tail_rows -= a.row0;
         a.ws_o = (float*)workspace;
-        a.ws_ml = a.ws_o + (size_t)p.nsplit * B * H * Sq * D;
+        a.ws_ml = a.ws_o + (size_t)p.nsplit * a.tail_rows * D;
     }
-    const bool tl = token_contiguous(sk, sv, D);
     hipError_t e = dtype == ATTN_DTYPE_BF16 ? launch_t<bf16>(a, tl, stream)
                                             : launch_t<f16>(a, tl, stream);
     if (e == hipSuccess) e = scratch.release(stream);
@@ -2642,7 +2783,8 @@ extern "C" size_t attn_split_workspace_bytes(int B, int H, int Sq, int Skv, int 
     if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 ||
         !((D <= 64 && D > 0 && D % 8 == 0) || D == 128 || D == 512))
         return 0;
-    return split_ws_bytes(plan_split(B, H, Sq, Skv, D), B, H, Sq, D);
+    const bool tail = D != 512 || d512_wide();
+    return split_ws_bytes(plan_split(B, H, Sq, Skv, D, tail), B, H, Sq, D);
 }
 
 extern "C" int attn_fwd_split(const void* q, const void* k, const void* v, void* o, int B, int H,

@@ -155,3 +155,15 @@ def test_conv3d_kernels_do_not_spill(conv_asm):
     assert len(found) == 14, len(found)  # seven configurations, each for small and large C
     for name, vgprs, scratch, occ in found:
         assert scratch == 0 and occ >= 2 and vgprs <= 256, (name, vgprs, scratch, occ)
+
+
+def test_tail_kernels_keep_occupancy_without_spills(kernel_asm):
+    """The instantiations for whole units and a split tail (two epilogues)."""
+    seen = []
+    for m in RESOURCES.finditer(kernel_asm):
+        name, vgprs, scratch, occ = m.group(1), int(m.group(2)), int(m.group(3)), int(m.group(4))
+        if "7CfgTail" in name:
+            want = 2 if "7CfgTailILi128" in name else 4
+            seen.append(name)
+            assert occ >= want and vgprs <= 512 // want and scratch == 0, (name, vgprs, scratch)
+    assert len(seen) == 10, seen  # D = 128, and 64 and padded with and without the tile max
