@@ -146,7 +146,8 @@ def _newest_mtime(paths) -> float:
 
 
 def kernel_lib_inputs() -> list:
-    return [*KERNEL_SOURCES, CSRC / "scratch.h", *sorted(INCLUDE.glob("*.h"))]
+    return [*KERNEL_SOURCES, CSRC / "scratch.h", *sorted(CSRC.glob("*.inc")),
+            *sorted(INCLUDE.glob("*.h"))]
 
 
 def ensure_kernel_lib(lib: Path = KERNEL_LIB, sources=None) -> bool:

@@ -21,12 +21,9 @@
 //    .contiguous() (attn.cpp:15). The VAE's token-contiguous views
 //    ([b, c, h*w] seen as [b, 1, h*w, c], deploy/gfx906_attention.py:102-104,
 //    D = 512) are read in place, q and out with them, up to Skv = 6400; past
-//    that they are copied, on purpose: the in-place kernel needs transposing
-//    LDS reads for K and runs 16 query rows per wave, a cost that grows with
-//    Skv^2 while the copies grow with Skv (measured on MI355X with split key
-//    ranges, in place against copy and the 32-row kernel: 0.115 against 0.127
-//    ms at h*w = 4608, 0.161 against 0.169 ms at 6400, 0.226 against 0.192 ms
-//    at 7056, 0.775 against 0.605 ms at 16384).
+//    that they are copied, on purpose: the in-place kernel reads K and V in
+//    64-byte runs of a dim's tokens (half a cache line), a cost that grows
+//    with Skv^2 while the copies grow with Skv.
 //  * `out`, if given, is written instead of allocating: any [B, H, Sq, D]
 //    view of q's dtype and device whose elements do not overlap, e.g. the
 //    transpose of a [B, Sq, H, D] buffer or the VAE's [b, 1, h*w, c] view of

@@ -94,7 +94,7 @@ constexpr int kSgMfma = 0x008, kSgDsRead = 0x100;
 
 // Strides of one tensor in elements: batch, head, sequence, head dim. The
 // head dim is contiguous (d == 1) except in the token-contiguous D = 512
-// layout (attn_fwd_d512<T, true>).
+// layout (attn_fwd_tok512).
 struct Strides {
     long long b, h, s, d;
 };
@@ -132,6 +132,10 @@ struct KArgs {
     // where before the prefetch the two extra barriers cost more than the
     // gathered global loads).
     int q_lds;
+    // Token-contiguous D = 512 layout: q (o) is token-contiguous as well, with
+    // 16-byte aligned rows and (q) whole 8-token chunks, like K's, and a
+    // per-head span below 2^31 bytes.
+    int q_tok, o_tok;
     // Compute units of the device: with the kernel's workgroups per CU, how
     // many workgroups are resident at once (the D = 128 ring kernel and the
     // D <= 64 one with the tile max prefetch the Q tile of the workgroup that
@@ -1452,9 +1456,6 @@ struct Cfg512 {
 struct Cfg512T {
     static constexpr int ROWB = Cfg512::BN * 2;    // 64 bytes: one dim row of a tile
     static constexpr int TILE = Cfg512::DP * ROWB;  // 32 KB: K^T or V^T of one tile
-    static constexpr int STAGE = 2 * TILE;
-    static constexpr int LDS = 2 * STAGE;
-    static constexpr int LPW = TILE / 1024 / Cfg512::NW;  // 1 KB loads per wave, tensor, tile
 };
 
 // Slot swizzle of the token-contiguous K^T tiles: bit 2 of the row to bit 1 of
@@ -1503,10 +1504,8 @@ __device__ __attribute__((noinline)) Rescale512<T> d512_rescale(f32x4 S0, f32x4 
 }
 #endif
 
-// grid: ceil(Sq / 128) * B*H workgroups; block: 512 threads. TL: k and v in
-// the token-contiguous layout (Cfg512T), q and o read and written element by
-// element with any strides.
-template <class T, bool TL, bool SPLIT>
+// grid: ceil(Sq / 128) * B*H workgroups (times nsplit); block: 512 threads.
+template <class T, bool SPLIT>
 __global__ void __launch_bounds__(Cfg512::NT, 1)
 attn_fwd_d512(const KArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1517,9 +1516,9 @@ attn_fwd_d512(const KArgs a) {
     static_assert(NLD * C::NW == BN && D * 2 == 64 * 16, "one row per load instruction");
     constexpr int NQF = D / 32;  // Q fragments (32 dims each)
     constexpr int NOB = D / 16;  // 16-dim output blocks
-    constexpr int STAGE = TL ? Cfg512T::STAGE : C::STAGE;
-    constexpr int VOFF = TL ? Cfg512T::TILE : C::KTILE;  // V (V^T) tile within a stage
-    __shared__ __attribute__((aligned(1024))) char lds[TL ? Cfg512T::LDS : C::LDS];  // 2 x (K, V)
+    constexpr int STAGE = C::STAGE;
+    constexpr int VOFF = C::KTILE;  // V tile within a stage
+    __shared__ __attribute__((aligned(1024))) char lds[C::LDS];  // 2 x (K, V)
 
     const int Sq = a.Sq;
     const float c = a.c;
@@ -1550,43 +1549,7 @@ attn_fwd_d512(const KArgs a) {
     // Direct loads: one instruction per K or V row; lane l fetches dims
     // 8l..8l+7. Rows past Skv read as zeros (the descriptor covers the valid
     // rows only).
-    // Token-contiguous layout: lane l of 1 KB block j writes dim row
-    // 16j + l/4, slot l%4, so it fetches key chunk tu = (l%4) ^ tswz(row) of
-    // K and tv = (l%4) ^ vswz512(row) of V, the same in every block; chunks
-    // at or past Skv load zeros. Byte offsets of the lane's rows at key 0
-    // (the host keeps them below 2^31).
-    const int tu = (lane & 3) ^ ((((lane >> 4) & 1) << 1) | ((lane >> 5) & 1));
-    const int tv = (lane & 3) ^ ((lane >> 3) & 3);
-    unsigned ktrow[TL ? Cfg512T::LPW : 1], vtrow[TL ? Cfg512T::LPW : 1];
-    __amdgpu_buffer_rsrc_t rkt, rvt;
-    if constexpr (TL) {
-#pragma unroll
-        for (int n = 0; n < Cfg512T::LPW; ++n) {
-            const long long row = 16 * (wave + n * C::NW) + (lane >> 2);
-            ktrow[n] = (unsigned)((row * a.sk.d + 8 * tu) * 2);
-            vtrow[n] = (unsigned)((row * a.sv.d + 8 * tv) * 2);
-        }
-        const int kb = __builtin_amdgcn_readfirstlane((int)(((D - 1) * a.sk.d + Skv) * 2));
-        const int vb = __builtin_amdgcn_readfirstlane((int)(((D - 1) * a.sv.d + Skv) * 2));
-        rkt = __builtin_amdgcn_make_buffer_rsrc((void*)Kh, 0, kb, 0x00020000);
-        rvt = __builtin_amdgcn_make_buffer_rsrc((void*)Vh, 0, vb, 0x00020000);
-    }
     auto issue = [&](int t, char* dst) __attribute__((always_inline)) {
-        if constexpr (TL) {
-            const int k0 = t * BN;
-            const bool kin = k0 + 8 * tu < Skv, vin = k0 + 8 * tv < Skv;
-#pragma unroll
-            for (int n = 0; n < Cfg512T::LPW; ++n) {
-                const int blk = wave + n * C::NW;
-                const unsigned ok = kin ? ktrow[n] + 2u * (unsigned)k0 : 0xFFFFFFF0u;
-                const unsigned ov = vin ? vtrow[n] + 2u * (unsigned)k0 : 0xFFFFFFF0u;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rkt, (LDS_AS void*)(dst + blk * 1024), 16,
-                                                         (int)ok, 0, 0, 0);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    rvt, (LDS_AS void*)(dst + Cfg512T::TILE + blk * 1024), 16, (int)ov, 0, 0, 0);
-            }
-            return;
-        }
         const int rows = min(Skv - t * BN, BN);
         const int kbytes = (int)(((rows - 1) * kss + D) * 2);
         const int vbytes = (int)(((rows - 1) * vss + D) * 2);
@@ -1611,15 +1574,7 @@ attn_fwd_d512(const KArgs a) {
     const unsigned qneg = a.qsign < 0.f ? 0x80008000u : 0u;
 #pragma unroll
     for (int s = 0; s < NQF; ++s) {
-        if constexpr (TL) {  // any strides: eight element loads
-            x8 val = {};
-            if (live)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) val[e] = Qh[qrow * a.sq.s + (32 * s + 8 * g + e) * a.sq.d];
-            qf[s] = __builtin_bit_cast(x8, __builtin_bit_cast(u32x4, val) ^ qneg);
-        } else {
-            qf[s] = q_fragment(Qh + qrow * a.sq.s + 32 * s + 8 * g, live, qneg);
-        }
+        qf[s] = q_fragment(Qh + qrow * a.sq.s + 32 * s + 8 * g, live, qneg);
     }
 
     // K read: row kb*16 + i, dims 32s + 8g.. ; V^T read (transposed, per
@@ -1627,21 +1582,6 @@ attn_fwd_d512(const KArgs a) {
     // 16*db + 4*(i%4)..
     const int kbase = i * C::KS + g * 16;
     const int vbase = (4 * g + (i >> 2)) * C::VS + 8 * (i & 3);
-    // Token-contiguous layout. K^T read (ds_read_b64_tr_b16, two per
-    // fragment, h = 0, 1): lane 4e + j of group g reads keys tkey(kb, j, 0..3)
-    // of dim row 32s + 8g + 4h + e (chunk j, half (j + kb) & 1; the row's
-    // swizzle is tswz = 2h + g%2), so lane i receives key tkey(kb, i/4, i%4),
-    // dims 32s + 8g + 4h + 0..3. V^T read: dim row 16ob + i, keys 8g..8g+7
-    // (chunk g), one 16-byte read from slot g ^ vswz512(i).
-    int ktb[2][2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-            ktb[h][kb] = (8 * g + 4 * h + (i >> 2)) * Cfg512T::ROWB +
-                         (((i & 3) ^ ((h << 1) | (g & 1))) * 16) + (((i & 3) + kb) & 1) * 8;
-    const int vtb = i * Cfg512T::ROWB + ((g ^ vswz512(i)) * 16);
-
     f32x4 oacc[NOB];
 #pragma unroll
     for (int ob = 0; ob < NOB; ++ob) oacc[ob] = f32x4{};
@@ -1676,12 +1616,7 @@ attn_fwd_d512(const KArgs a) {
             f32x4 Sp[2] = {f32x4{}, f32x4{}};
 #pragma unroll
             for (int s = 0; s < NQF; ++s) {
-                x8 kf;
-                if constexpr (TL)
-                    kf = lds_read_tr2<T>(sk, ktb[0][kb] + s * 32 * Cfg512T::ROWB,
-                                         ktb[1][kb] + s * 32 * Cfg512T::ROWB);
-                else
-                    kf = lds_read16<T>(sk, kbase + kb * 16 * C::KS + s * 64);
+                const x8 kf = lds_read16<T>(sk, kbase + kb * 16 * C::KS + s * 64);
                 Sp[s & 1] = E::mma16(kf, qf[s], Sp[s & 1]);
             }
             __builtin_amdgcn_sched_group_barrier(kSgDsRead, 4, 0);
@@ -1697,10 +1632,8 @@ attn_fwd_d512(const KArgs a) {
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int key = TL ? tkey(kb, g, r) : kb * 16 + 4 * g + r;
-                    if (t * BN + key >= Skv) S[kb][r] = -INFINITY;
-                }
+                for (int r = 0; r < 4; ++r)
+                    if (t * BN + kb * 16 + 4 * g + r >= Skv) S[kb][r] = -INFINITY;
         }
         if (t == 0) {  // first tile: start from its exact max (O is still zero)
             float mx = fmaxf(max3(S[0][0], S[0][1], S[0][2]), max3(S[0][3], S[1][0], S[1][1]));
@@ -1727,20 +1660,10 @@ attn_fwd_d512(const KArgs a) {
 #pragma unroll
         for (int ob = 0; ob < NOB; ++ob) oacc[ob] *= alpha;
         l_run += l_tile;
-        if constexpr (TL) {  // odd lane groups: block 1 holds keys 8g..8g+3
-            const u32x4 pw = __builtin_bit_cast(u32x4, P);
-            const bool sw = g & 1;
-            P = __builtin_bit_cast(x8, u32x4{sw ? pw[2] : pw[0], sw ? pw[3] : pw[1],
-                                             sw ? pw[0] : pw[2], sw ? pw[1] : pw[3]});
-        }
         // O^T += V^T P^T, one 16x16x32 MFMA per 16-dim block.
 #pragma unroll
         for (int ob = 0; ob < NOB; ++ob) {
-            x8 vf;
-            if constexpr (TL)
-                vf = lds_read16<T>(sv, vtb + ob * 16 * Cfg512T::ROWB);
-            else
-                vf = lds_read_tr2<T>(sv, vbase + 32 * ob, vbase + 32 * ob + 16 * C::VS);
+            const x8 vf = lds_read_tr2<T>(sv, vbase + 32 * ob, vbase + 32 * ob + 16 * C::VS);
             oacc[ob] = E::mma16(vf, P, oacc[ob]);
         }
         __builtin_amdgcn_sched_group_barrier(kSgDsRead, 4, 0);
@@ -1777,14 +1700,7 @@ attn_fwd_d512(const KArgs a) {
             const auto h0 = E::cvt2(oacc[ob][0] * inv, oacc[ob][1] * inv);
             const auto h1 = E::cvt2(oacc[ob][2] * inv, oacc[ob][3] * inv);
             const int d0 = 16 * ob + 4 * g;
-            if constexpr (TL) {  // any strides: four element stores
-                op[(d0 + 0) * a.so.d] = h0[0];
-                op[(d0 + 1) * a.so.d] = h0[1];
-                op[(d0 + 2) * a.so.d] = h1[0];
-                op[(d0 + 3) * a.so.d] = h1[1];
-            } else {
-                *reinterpret_cast<typename E::x4*>(op + d0) = typename E::x4{h0[0], h0[1], h1[0], h1[1]};
-            }
+            *reinterpret_cast<typename E::x4*>(op + d0) = typename E::x4{h0[0], h0[1], h1[0], h1[1]};
         }
     }
 #endif
@@ -1823,377 +1739,27 @@ struct Cfg512W {
 };
 static_assert(Cfg512W::BM == Cfg512::BM, "same query tiling as attn_fwd_d512 (grid, split plan)");
 
-// grid: ceil(Sq / 128) * B*H workgroups (times nsplit); block: 256 threads.
-template <class T, bool SPLIT>
-__global__ void __launch_bounds__(Cfg512W::NT, 1)
-attn_fwd_d512w(const KArgs a) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    using C = Cfg512W;
-    using E = Elem<T>;
-    using x8 = typename E::x8;
-    constexpr int D = C::DP, BN = C::BN, NLD = C::NLD;
-    constexpr int NQF = D / 32;  // Q fragments (32 dims each) per column block
-    constexpr int NOB = D / 16;  // 16-dim output blocks
-    static_assert(2 * NLD == 16, "prologue wait counts");
-    __shared__ __attribute__((aligned(1024))) char kb0[C::TILE];
-    __shared__ __attribute__((aligned(1024))) char kb1[C::TILE];
-    __shared__ __attribute__((aligned(1024))) char vb0[C::TILE];
-    __shared__ __attribute__((aligned(1024))) char vb1[C::TILE];
-
-    const int Sq = a.Sq;
-    const float c = a.c;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i = lane & 15, g = lane >> 4;
-    const int nqt = (Sq + C::BM - 1) / C::BM;
-    const WorkItem it = work_item<SPLIT, true>(a, blockIdx.x, gridDim.x, nqt);
-    const int qt = it.qt, bh = it.bh;
-    const int b = bh / a.H, h = bh - b * a.H;
-    const int kv0 = SPLIT ? it.split * a.split_len : 0;
-    const int Skv = SPLIT && it.part ? max(0, min(a.Skv - kv0, a.split_len)) : a.Skv;
-    const T* Qh = (const T*)a.q + b * a.sq.b + h * a.sq.h;
-    const T* Kh = (const T*)a.k + b * a.sk.b + h * a.sk.h + kv0 * a.sk.s;
-    const T* Vh = (const T*)a.v + b * a.sv.b + h * a.sv.h + kv0 * a.sv.s;
-    T* Oh = (T*)a.o + b * a.so.b + h * a.so.h;
-    const long long kss = a.sk.s, vss = a.sv.s;
-    const int qrow0 = qt * C::BM + wave * 32 + i;  // this lane's rows: qrow0 + 16 rb
-    const int ntiles = (Skv + BN - 1) / BN;
-    // Direct loads of tile t of X into dst: one instruction per 1 KB row,
-    // lane l fetching dims 8l..8l+7 of rows wave + 4n. The descriptor covers
-    // the tile's valid rows only (none past the last tile), so the rest read
-    // as zeros.
-    auto issue = [&](const T* X, long long ss, int t, char* dst) __attribute__((always_inline)) {
-        const int rows = min(Skv - t * BN, BN);
-        const int bytes = rows > 0 ? (int)(((rows - 1) * ss + D) * 2) : 0;
-        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)(X + (rows > 0 ? t * BN * ss : 0)), 0, bytes, 0x00020000);
-#pragma unroll
-        for (int n = 0; n < NLD; ++n) {
-            const int row = wave + n * C::NW;  // wave-uniform
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LDS_AS void*)(dst + row * C::KS), 16,
-                                                     lane * 16, (int)(row * ss * 2), 0, 0);
-        }
-    };
-
-    // Q^T fragments (B operands: column = query 16rb + l%16, k = dims
-    // 32s + 8(l/16)..+7).
-    // Issue order Q, K(0), V(0), K(1): the prologue waits for the first two.
-    // Q goes through a range-checked descriptor where the workgroup's rows
-    // span less than 2 GiB; the sign of a negative scale is applied after the
-    // prologue's barrier, so that no wait for Q comes before the tiles are
-    // issued. (With the predicated fallback for larger spans, the compiler
-    // waits for every load in flight before the descriptor loads, so nothing
-    // is issued before Q.)
-    x8 qf[2][NQF];
-    const unsigned qneg = a.qsign < 0.f ? 0x80008000u : 0u;
-    if ((long long)(C::BM - 1) * a.sq.s * 2 + D * 2 < (1LL << 31)) {  // (uniform)
-        const int qrows = ntiles > 0 ? min(Sq - qt * C::BM, C::BM) : 0;
-        const __amdgpu_buffer_rsrc_t qr =
-            q_rsrc(Qh + (long long)qt * C::BM * a.sq.s, qrows, a.sq.s, D);
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-            for (int s = 0; s < NQF; ++s) {
-                const int r = wave * 32 + 16 * rb + i;
-                const unsigned off =
-                    r < qrows ? (unsigned)((r * a.sq.s + 32 * s + 8 * g) * 2) : kQOutOfRange;
-                qf[rb][s] = q_load<T>(qr, off);
-            }
-    } else {
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-            for (int s = 0; s < NQF; ++s) {
-                const int row = qrow0 + 16 * rb;
-                qf[rb][s] = q_fragment(Qh + row * a.sq.s + 32 * s + 8 * g, row < Sq && ntiles > 0, 0u);
-            }
-    }
-    // Issued whatever the key count (with no keys the descriptors are empty
-    // and the wait after the loop covers them): loads under a condition here
-    // make the compiler assume, after the barrier, that the Q loads may be
-    // the last ones issued, and wait for V(0) and K(1) in the first QK^T.
-    issue(Kh, kss, 0, kb0);
-    issue(Vh, vss, 0, vb0);
-    issue(Kh, kss, 1, kb1);
-
-    // K read: row 16kb + i, dims 32s + 8g..; V^T read (transposed, per
-    // 16-lane group g): rows 4g + i/4 and 16 + 4g + i/4, dims 16ob + 4(i%4)..
-    const int kbase = i * C::KS + g * 16;
-    const int vbase = (4 * g + (i >> 2)) * C::VS + 8 * (i & 3);
-
-    // S^T = K Q^T of one tile, per column block rb and 16-key block kb, in
-    // two MFMA chains (even and odd Q fragments) added at the end.
-    // K fragments in flight in the QK^T step: each read is issued six
-    // fragments (12 MFMAs, about 190 cycles) ahead of its use, which covers
-    // the LDS latency a single wave per SIMD cannot hide otherwise
-    // (measured on MI355X against 2, 4, 8 and 10 in flight). The softmax
-    // VALU work of the same basic block is left to the scheduler: pinning it
-    // between the MFMAs or ahead of them was measured slower.
-    constexpr int NKQ = 6;
-    auto qk = [&](const char* __restrict__ kt, f32x4 (&S)[2][2]) __attribute__((always_inline)) {
-        constexpr int NF = 2 * NQF;  // fragments: 16 per 16-key block
-        auto kread = [&](int f) __attribute__((always_inline)) {
-            return lds_read16<T>(kt, kbase + (f / NQF) * 16 * C::KS + (f % NQF) * 64);
-        };
-        x8 kq[NKQ];
-#pragma unroll
-        for (int j = 0; j < NKQ; ++j) kq[j] = kread(j);
-        f32x4 Sp[2][2];
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            const int kb = f / NQF, s = f % NQF;
-            if (s == 0) Sp[0][0] = Sp[0][1] = Sp[1][0] = Sp[1][1] = f32x4{};
-            const x8 kf = kq[f % NKQ];
-            if (f + NKQ < NF) kq[f % NKQ] = kread(f + NKQ);
-            Sp[0][s & 1] = E::mma16(kf, qf[0][s], Sp[0][s & 1]);
-            Sp[1][s & 1] = E::mma16(kf, qf[1][s], Sp[1][s & 1]);
-            if (s == NQF - 1) {
-                S[0][kb] = Sp[0][0] + Sp[0][1];
-                S[1][kb] = Sp[1][0] + Sp[1][1];
-            }
-        }
-        __builtin_amdgcn_sched_group_barrier(kSgDsRead, NKQ, 0);
-#pragma unroll
-        for (int f = 0; f < NF - NKQ; ++f) {
-            __builtin_amdgcn_sched_group_barrier(kSgMfma, 2, 0);
-            __builtin_amdgcn_sched_group_barrier(kSgDsRead, 1, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(kSgMfma, 2 * NKQ, 0);
-    };
-
-    // V^T fragment of 16-dim block ob.
-    // V^T fragments in flight in the PV step (two transposed reads each; 8
-    // measured best against 4 and 6).
-    constexpr int NVQ = 8;
-    auto vread = [&](const char* vt, int ob) __attribute__((always_inline)) {
-        return lds_read_tr2<T>(vt, vbase + 32 * ob, vbase + 32 * ob + 16 * C::VS);
-    };
-
-    // P of one column block from its two score blocks, with running max
-    // -nm; pm tracks the largest p and lsum sums the rounded p.
-    auto make_p = [&](const f32x4 (&S)[2], x8& P, float nm, float& lsum, f32x2& pm)
-        __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const f32x4& Sb = S[u >> 1];
-            const float p0 = __builtin_amdgcn_exp2f(fmaf(Sb[2 * (u & 1)], c, nm));
-            const float p1 = __builtin_amdgcn_exp2f(fmaf(Sb[2 * (u & 1) + 1], c, nm));
-            const auto hp = E::cvt2(p0, p1);
-            P[2 * u] = hp[0];
-            P[2 * u + 1] = hp[1];
-            lsum = E::sum2(hp, lsum);
-            pm[u & 1] = max3(pm[u & 1], p0, p1);
-        }
-    };
-
-    f32x4 oacc[2][NOB];
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int ob = 0; ob < NOB; ++ob) {
-            oacc[rb][ob] = f32x4{};
-            agpr_fence2(oacc[rb][ob]);
-        }
-    // Running max (log2 units; finite, so masked keys give p = 0) and row sum.
-    float m_run[2] = {-1e30f, -1e30f}, l_run[2] = {0.f, 0.f};
-
-    // The last tile's keys past Skv score -inf.
-    auto mask_tail = [&](int t, f32x4 (&S)[2][2]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (t * BN + kb * 16 + 4 * g + r >= Skv) S[rb][kb][r] = -INFINITY;
-    };
-
-    f32x4 S[2][2];  // scores of the tile the next iteration turns into P
-    // Iteration t: scores S of tile t in registers; K(t+1) in kc, V(t) in vc;
-    // K(t+2) loads into kf and V(t+1) into vf. P of tile t and the QK^T
-    // MFMAs of tile t+1 share a basic block; the rescale test of tile t (a
-    // rare branch) follows, then the PV MFMAs of tile t. Interleaving the
-    // softmax VALU work with the PV MFMAs instead (a single wave per SIMD
-    // issues both) was measured 3 % slower.
-    auto iter = [&](int t, char* __restrict__ kf, const char* __restrict__ kc,
-                    const char* __restrict__ vc, char* __restrict__ vf) __attribute__((always_inline)) {
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's K(t+1) and V(t) rows
-        lds_barrier();                      // ... every wave's; K(t) and V(t-1) buffers free
-        issue(Kh, kss, t + 2, kf);
-        issue(Vh, vss, t + 1, vf);
-        x8 P[2];
-        float lt[2] = {0.f, 0.f};
-        f32x2 pm[2] = {{0.f, 0.f}, {0.f, 0.f}};
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb) make_p(S[rb], P[rb], -m_run[rb], lt[rb], pm[rb]);
-        const bool up0 = __any(!(fmaxf(pm[0][0], pm[0][1]) <= kPmaxLimit));
-        const bool up1 = __any(!(fmaxf(pm[1][0], pm[1][1]) <= kPmaxLimit));
-        f32x4 Sn[2][2];
-        qk(kc, Sn);
-        // The first V^T fragments, read before the rare-path branch so that
-        // their LDS latency overlaps it.
-        x8 vq[NVQ];
-#pragma unroll
-        for (int j = 0; j < NVQ; ++j) vq[j] = vread(vc, j);
-        if (__builtin_expect(up0 || up1, 0)) {
-#pragma unroll
-            for (int rb = 0; rb < 2; ++rb) {
-                if (rb == 0 ? !up0 : !up1) continue;
-                // The exact max of the tile's rows; O, l and P follow.
-                float mx = fmaxf(max3(S[rb][0][0], S[rb][0][1], S[rb][0][2]),
-                                 max3(S[rb][0][3], S[rb][1][0], S[rb][1][1]));
-                mx = quad_group_max(max3(mx, S[rb][1][2], S[rb][1][3])) * c;
-                const float m_new = fmaxf(m_run[rb], mx);
-                const float alpha = __builtin_amdgcn_exp2f(m_run[rb] - m_new);
-#pragma unroll
-                for (int ob = 0; ob < NOB; ob += 4)
-                    agpr_fence24(oacc[rb][ob], oacc[rb][ob + 1], oacc[rb][ob + 2], oacc[rb][ob + 3]);
-#pragma unroll
-                for (int ob = 0; ob < NOB; ++ob) {
-                    oacc[rb][ob] *= alpha;
-                    agpr_fence2(oacc[rb][ob]);
-                }
-                l_run[rb] *= alpha;
-                m_run[rb] = m_new;
-                lt[rb] = 0.f;
-                f32x2 pm2 = {0.f, 0.f};
-                make_p(S[rb], P[rb], -m_new, lt[rb], pm2);
-            }
-        }
-        l_run[0] += lt[0];
-        l_run[1] += lt[1];
-        // O^T += V^T P^T: one V^T fragment per 16-dim block, two MFMAs, with
-        // NVQ fragments in flight (the MFMAs are volatile asm, so the LDS
-        // reads keep their place in this order).
-        vgpr_fence2(P[0], P[1]);
-#pragma unroll
-        for (int ob = 0; ob < NOB; ++ob) {
-            const x8 vfr = vq[ob % NVQ];
-            if (ob + NVQ < NOB) vq[ob % NVQ] = vread(vc, ob + NVQ);
-            mma16_agpr<T>(oacc[0][ob], vfr, P[0]);
-            if (ob + 1 < NOB)
-                mma16_agpr<T>(oacc[1][ob], vfr, P[1]);
-            else
-                mma16_agpr<T, true>(oacc[1][ob], vfr, P[1]);
-        }
-        if ((t + 2) * BN > Skv) mask_tail(t + 1, Sn);
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb) S[rb][kb] = Sn[rb][kb];
-    };
-
-    if (ntiles > 0) {
-        // Prologue: this wave's K(0) rows and Q have landed once at most the
-        // 16 loads of V(0) and K(1) are in flight; then every wave's. Scores
-        // of tile 0 and their exact max.
-        __builtin_amdgcn_s_waitcnt(0x4F70);  // vmcnt(16)
-        lds_barrier();
-        if (qneg) {  // (uniform)
-#pragma unroll
-            for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-                for (int s = 0; s < NQF; ++s) q_negate(qf[rb][s], qneg);
-        }
-        qk(kb0, S);
-        if (BN > Skv) mask_tail(0, S);
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
-            const float mx = fmaxf(max3(S[rb][0][0], S[rb][0][1], S[rb][0][2]),
-                                   max3(S[rb][0][3], S[rb][1][0], S[rb][1][1]));
-            m_run[rb] = quad_group_max(max3(mx, S[rb][1][2], S[rb][1][3])) * c;
-        }
-        for (int t = 0; t < ntiles; t += 2) {
-            iter(t, kb0, kb1, vb0, vb1);
-            if (t + 1 < ntiles) iter(t + 1, kb1, kb0, vb1, vb0);
-        }
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the (empty) loads past the end
-
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int ob = 0; ob < NOB; ob += 4)
-            agpr_fence24(oacc[rb][ob], oacc[rb][ob + 1], oacc[rb][ob + 2], oacc[rb][ob + 3]);
-    // The output leaves through LDS: each wave writes its 32 rows, in the
-    // element type, to a row-major staging area in the ring array of its
-    // index (rows padded by 16 bytes), then stores them as whole rows, 1 KB
-    // per instruction. A lane's accumulators hold pieces of 16 rows, which
-    // stored directly reach memory as 8-byte pieces of 16 rows per
-    // instruction (measured on MI355X: 64 workgroups of 128 rows over 128
-    // keys 0.0222 -> 0.0182 ms, 8 rounds of them 0.234 -> 0.211 ms, c4
-    // +0.7 %). The split path's fp32 partial rows, 64-byte pieces, gained
-    // nothing from staging and are stored directly, as is an output whose
-    // rows are not 16-byte aligned.
-    // The epilogue's addresses derive from the lane index read here, so the
-    // compiler cannot compute them ahead of the main loop and keep them live
-    // across it (it spilled them otherwise).
-    int lane_e = lane;
-    asm volatile("" : "+v"(lane_e));
-    const int ie = lane_e & 15, ge = lane_e >> 4;
-    const KArgs& ea = SPLIT ? args_here() : a;  // (see args_here)
-    const int Sqe = ea.Sq;
-    const WorkItem& ite = it;
-    T* const Oe = SPLIT ? (T*)ea.o + b * ea.so.b + h * ea.so.h : Oh;
-    const int row0 = ite.qt * C::BM + wave * 32;  // this wave's first row
-    const bool part = SPLIT && ite.part;
-    const bool staged = !part && ea.o16;
-    if (staged) lds_barrier();  // every wave is done with the ring
-    char* const stg = wave == 0 ? kb0 : wave == 1 ? kb1 : wave == 2 ? vb0 : vb1;
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-        const int qrow = row0 + 16 * rb + ie;
-        const float l = quad_group_sum(l_run[rb]);
-        if (part) {  // unnormalised O and (m, l) of this key range
-            if (qrow < Sqe) {
-                const long long r =
-                    ite.split * ea.tail_rows + ((long long)ite.bh * Sqe + qrow - ea.row0);
-                float* wo = ea.ws_o + r * D;
-#pragma unroll
-                for (int ob = 0; ob < NOB; ++ob)
-                    *reinterpret_cast<f32x4*>(wo + 16 * ob + 4 * ge) = oacc[rb][ob];
-                if (ge == 0) *reinterpret_cast<f32x2*>(ea.ws_ml + 2 * r) = f32x2{m_run[rb], l};
-            }
-        } else if (staged) {
-            constexpr int RS = D * 2 + 16;
-            static_assert(32 * RS <= C::TILE, "a wave's 32 rows per ring array");
-            const float inv = l > 0.f ? 1.f / l : 0.f;
-#pragma unroll
-            for (int ob = 0; ob < NOB; ++ob) {
-                const auto h0 = E::cvt2(oacc[rb][ob][0] * inv, oacc[rb][ob][1] * inv);
-                const auto h1 = E::cvt2(oacc[rb][ob][2] * inv, oacc[rb][ob][3] * inv);
-                *reinterpret_cast<LDS_AS typename E::x4*>(
-                    (LDS_AS char*)stg + (16 * rb + ie) * RS + (16 * ob + 4 * ge) * 2) =
-                    typename E::x4{h0[0], h0[1], h1[0], h1[1]};
-            }
-        } else {
-            const float inv = l > 0.f ? 1.f / l : 0.f;
-            if (qrow < Sqe) {
-                T* op = Oe + qrow * ea.so.s;
-#pragma unroll
-                for (int ob = 0; ob < NOB; ++ob) {
-                    const auto h0 = E::cvt2(oacc[rb][ob][0] * inv, oacc[rb][ob][1] * inv);
-                    const auto h1 = E::cvt2(oacc[rb][ob][2] * inv, oacc[rb][ob][3] * inv);
-                    *reinterpret_cast<typename E::x4*>(op + 16 * ob + 4 * ge) =
-                        typename E::x4{h0[0], h0[1], h1[0], h1[1]};
-                }
-            }
-        }
-    }
-    if (staged) {
-        constexpr int RS = D * 2 + 16;
-        constexpr int CPR = D * 2 / 16;  // 16-byte pieces per row (one per lane)
-        static_assert(CPR == 64, "one row per store instruction");
-#pragma unroll
-        for (int r = 0; r < 32; ++r) {
-            const u32x4 val = *reinterpret_cast<const LDS_AS u32x4*>(
-                (const LDS_AS char*)stg + r * RS + lane_e * 16);
-            if (row0 + r < Sqe)
-                *reinterpret_cast<u32x4*>(Oe + (row0 + r) * ea.so.s + lane_e * 8) = val;
-        }
-    }
-#endif
-}
+// attn_fwd_tok512: the same kernel for k and v in the token-contiguous layout
+// (Cfg512T: K^T and V^T tiles, the two LDS read patterns swapped), q and o of
+// any strides, fast where they are token-contiguous too. The 32 rows of a wave
+// are then query tkey(rb, i/4, i%4) of the wave's 32 for column i of column
+// block rb: Q^T arrives as a K^T tile does and is read the same way, and O is
+// staged by rows and read back transposed. One 4096-token fp16 head in 8 key
+// ranges: 57 us, and 69 with the 16-row kernel that served this layout before
+// (every fragment read from LDS fed one MFMA there instead of two).
+//
+// grid: ceil(Sq / 128) * B*H workgroups (SPLIT: whole + tail * nsplit); block:
+// 256 threads.
+#define D512W_KERNEL attn_fwd_d512w
+#define D512W_TL false
+#include "attn_d512w.inc"
+#undef D512W_KERNEL
+#undef D512W_TL
+#define D512W_KERNEL attn_fwd_tok512
+#define D512W_TL true
+#include "attn_d512w.inc"
+#undef D512W_KERNEL
+#undef D512W_TL
 
 // Merge of the split key ranges: per output row, with m* the largest
 // running max of its splits and w_s = exp2(m_s - m*),
@@ -2209,20 +1775,14 @@ struct CombArgs {
     const float* ws_ml;
     void* o;
     Strides so;
-    int H, Sq, D, nsplit;
+    int H, Sq, D, nsplit, whole;
     long long row0, rows;  // the split rows: [row0, row0 + rows) of all heads' rows
 };
 
-template <class T>
-__global__ void __launch_bounds__(256) attn_combine(const CombArgs c) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    using E = Elem<T>;
-    const int dq = c.D / 4;
+// Dims d0..d0+3 of the merged output row `row` (of the split rows).
+__device__ __forceinline__ f32x4 merge_row(const CombArgs& c, long long row, int d0) {
     const long long rows = c.rows;
-    const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= rows * dq) return;
-    const long long row = idx / dq;
-    const int d0 = (int)(idx - row * dq) * 4;
     const int ns = c.nsplit;
     const f32x2* ml = reinterpret_cast<const f32x2*>(c.ws_ml);
     float mx = -3.0e38f;
@@ -2255,9 +1815,22 @@ __global__ void __launch_bounds__(256) attn_combine(const CombArgs c) {
                 l += w * mlv[u][1];
             }
     }
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    const auto h0 = E::cvt2(acc[0] * inv, acc[1] * inv);
-    const auto h1 = E::cvt2(acc[2] * inv, acc[3] * inv);
+    return acc * (l > 0.f ? 1.f / l : 0.f);
+}
+#endif
+
+template <class T>
+__global__ void __launch_bounds__(256) attn_combine(const CombArgs c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    using E = Elem<T>;
+    const int dq = c.D / 4;
+    const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= c.rows * dq) return;
+    const long long row = idx / dq;
+    const int d0 = (int)(idx - row * dq) * 4;
+    const f32x4 val = merge_row(c, row, d0);
+    const auto h0 = E::cvt2(val[0], val[1]);
+    const auto h1 = E::cvt2(val[2], val[3]);
     const long long grow = c.row0 + row;
     const int bh = (int)(grow / c.Sq), srow = (int)(grow - (long long)bh * c.Sq);
     const int b = bh / c.H, h = bh - b * c.H;
@@ -2270,6 +1843,50 @@ __global__ void __launch_bounds__(256) attn_combine(const CombArgs c) {
         op[2 * c.so.d] = h1[0];
         op[3 * c.so.d] = h1[1];
     }
+#endif
+}
+
+// The same for a token-contiguous D = 512 output (KArgs::o_tok): a workgroup
+// merges 64 tokens x 32 dims and turns them in LDS, so that each dim's 64
+// tokens leave as one 128-byte line. Written element by element as above, a
+// wave's stores touch a line per dim for 2 bytes each (one 4096-token head in
+// 8 ranges: 26 us; this one 13).
+// grid: 128-row units past `whole`, x 2 (64 tokens) x 16 (32 dims).
+template <class T>
+__global__ void __launch_bounds__(256) attn_combine_tok(const CombArgs c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    using E = Elem<T>;
+    constexpr int BM = 128, ST = 72;  // unit rows; LDS row stride (tokens) of a dim
+    __shared__ __attribute__((aligned(16))) T tile[32 * ST];
+    const int nqt = (c.Sq + BM - 1) / BM;
+    const int unit = c.whole + (int)(blockIdx.x >> 5), part = blockIdx.x & 31;
+    const int bh = unit / nqt, tok0 = (unit - bh * nqt) * BM + (part >> 4) * 64;
+    const int dim0 = (part & 15) * 32;
+    if (tok0 >= c.Sq) return;  // (uniform)
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const int r = (tid >> 3) + 32 * p, d = (tid & 7) * 4;
+        if (tok0 + r < c.Sq) {
+            const f32x4 val =
+                merge_row(c, (long long)bh * c.Sq + tok0 + r - c.row0, dim0 + d);
+            const auto h0 = E::cvt2(val[0], val[1]);
+            const auto h1 = E::cvt2(val[2], val[3]);
+            tile[(d + 0) * ST + r] = h0[0];
+            tile[(d + 1) * ST + r] = h0[1];
+            tile[(d + 2) * ST + r] = h1[0];
+            tile[(d + 3) * ST + r] = h1[1];
+        }
+    }
+    __syncthreads();
+    const int b = bh / c.H, h = bh - b * c.H;
+    const int d = tid >> 3, r = (tid & 7) * 8, tok = tok0 + r;
+    T* op = (T*)c.o + b * c.so.b + h * c.so.h + (dim0 + d) * c.so.d + tok;
+    const T* src = tile + d * ST + r;
+    if (tok + 8 <= c.Sq)
+        *reinterpret_cast<u32x4*>(op) = *reinterpret_cast<const u32x4*>(src);
+    else
+        for (int e = 0; e < 8 && tok + e < c.Sq; ++e) op[e] = src[e];
 #endif
 }
 
@@ -2368,11 +1985,11 @@ void launch_kernel(const KArgs& a, bool tl, hipStream_t s) {
     const dim3 grid(SPLIT ? (unsigned)a.whole + (unsigned)a.tail * (unsigned)a.nsplit : units);
     if (D == 512) {
         if (tl)
-            hipLaunchKernelGGL((attn_fwd_d512<T, true, SPLIT>), grid, dim3(Cfg512::NT), 0, s, a);
+            hipLaunchKernelGGL((attn_fwd_tok512<T, SPLIT>), grid, dim3(Cfg512W::NT), 0, s, a);
         else if (d512_wide())
             hipLaunchKernelGGL((attn_fwd_d512w<T, SPLIT>), grid, dim3(Cfg512W::NT), 0, s, a);
         else
-            hipLaunchKernelGGL((attn_fwd_d512<T, false, SPLIT>), grid, dim3(Cfg512::NT), 0, s, a);
+            hipLaunchKernelGGL((attn_fwd_d512<T, SPLIT>), grid, dim3(Cfg512::NT), 0, s, a);
     } else if (SPLIT && a.whole > 0) {
         launch_tail<T>(a, grid, s);
     } else if (D == 128) {
@@ -2425,8 +2042,13 @@ hipError_t launch_t(const KArgs& a, bool tl, hipStream_t s) {
     c.Sq = a.Sq;
     c.D = a.D;
     c.nsplit = a.nsplit;
+    c.whole = a.whole;
     c.row0 = a.row0;
     c.rows = a.tail_rows;
+    if (tl && a.o_tok) {
+        hipLaunchKernelGGL((attn_combine_tok<T>), dim3((unsigned)a.tail * 32u), dim3(256), 0, s, c);
+        return hipGetLastError();
+    }
     const long long threads = a.tail_rows * (a.D / 4);
     hipLaunchKernelGGL((attn_combine<T>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s,
                        c);
@@ -2709,6 +2331,10 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     a.ws_ml = nullptr;
     a.o16 = (uintptr_t)o % 16 == 0 && so.b % 8 == 0 && so.h % 8 == 0 && so.s % 8 == 0 && so.d == 1;
     a.q_lds = sq.s <= (1LL << 24) && Skv > (D == 128 ? 256 : 1024);
+    a.q_tok = sq.s == 1 && sq.d != 1 && sq.b % 8 == 0 && sq.h % 8 == 0 && sq.d % 8 == 0 &&
+              (uintptr_t)q % 16 == 0 && Sq % 8 == 0 && (long long)(D - 1) * sq.d + Sq < (1LL << 30);
+    a.o_tok = so.s == 1 && so.d != 1 && so.b % 8 == 0 && so.h % 8 == 0 && so.d % 8 == 0 &&
+              (uintptr_t)o % 16 == 0;
     a.ncu = cu_count();
     a.whole = 0;
     a.tail = 0;
@@ -2717,7 +2343,7 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     const bool tl = token_contiguous(sk, sv, D);
     SplitPlan p = kNoSplit;
     if (workspace_bytes != (size_t)-1)  // split the keys if it pays
-        p = plan_split(B, H, Sq, Skv, D, !tl && (D != 512 || d512_wide()),
+        p = plan_split(B, H, Sq, Skv, D, D != 512 || tl || d512_wide(),
                        use_scratch ? kScratchBytes : (size_t)-1);
     size_t need = split_ws_bytes(p, B, H, Sq, D);
     // A grid that fills the GPU needs no workspace: without one (under

@@ -193,3 +193,12 @@ def test_compiled_d512w_respects_mfma_hazards(kernel_asm):
         assert n >= 64, (name, n)  # the PV MFMAs of at least one tile
         bad = check_function(instrs, labels)
         assert not bad, f"{name}: " + "\n".join(bad[:10])
+
+
+def test_compiled_token_contiguous_kernels_respect_mfma_hazards(kernel_asm):
+    funcs = parse_functions(kernel_asm, "attn_fwd_tok512")
+    assert len(funcs) == 4  # fp16/bf16 x split/unsplit
+    for name, (instrs, labels) in funcs.items():
+        assert sum(i.is_asm_mfma for i in instrs) >= 64, name
+        bad = check_function(instrs, labels)
+        assert not bad, f"{name}: " + "\n".join(bad[:10])
