@@ -15,12 +15,12 @@
 //    (The card is power-limited under sustained matrix load; the 16x16x32
 //    form costs less energy per FLOP than 32x32x16 and holds a higher clock:
 //    +6 % on a VAE decoder layer.)
-//  * Tiles of 64*CW channels x 64*NB voxels x KB reduction elements (CW = 2
-//    or 4, NB = 2, 3 or 4, KB = 32 or 64; seven configurations, chosen per
-//    problem for how the tile count fills the CUs and how long the
-//    reduction is), 2*CW waves of 64 x 32*NB (4 x 2NB MFMA blocks): with
-//    CW = 2 two workgroups per CU whose barriers are independent, with
-//    CW = 4 one workgroup of 8 waves that loads fewer bytes per MFMA.
+//  * Tiles of 64*CW channels x 32*NB*VW voxels x KB reduction elements (CW =
+//    1, 2 or 4, VW = 2 or 4, NB = 1 to 4, KB = 32 or 64; nine configurations,
+//    chosen per problem for how the tile count fills the CUs and how long the
+//    reduction is), CW*VW waves of 64 x 32*NB (4 x 2NB MFMA blocks): with 4
+//    waves two workgroups per CU whose barriers are independent, with 8 one
+//    workgroup that loads fewer bytes per MFMA.
 //    Both operand tiles go from HBM into LDS with buffer loads to LDS (no
 //    VGPR staging); the input gather uses a per-lane offset (voxel base +
 //    the offset of the lane's tap, advanced incrementally from k-tile to
@@ -72,19 +72,19 @@ constexpr int kMaxTaps = 1024;
 constexpr unsigned kOOB = 0xFFFFFFF0u;  // buffer offset past any range: loads zeros
 
 // Per-configuration sizes: NB 32-voxel MFMA blocks per wave, CW waves along
-// output channels x 2 along voxels (64*CW channels x 64*NB voxels per
+// output channels x VW along voxels (64*CW channels x 32*NB*VW voxels per
 // workgroup), NST stages in the LDS ring, KB reduction elements per k-tile
 // (LDS rows of 2*KB bytes: 32 -> 64-byte rows, 64 -> 128-byte rows, so that
 // each row of a tile is one whole 128-byte line of the weights or of a voxel).
-template <int NB, int NST, int KB, int CW>
+template <int NB, int NST, int KB, int CW, int VW = 2>
 struct ConvCfg {
-    static constexpr int NW = 2 * CW;               // waves
+    static constexpr int NW = VW * CW;              // waves
     static constexpr int NT = 64 * NW;              // threads
     static constexpr int BCH = 64 * CW;             // output channels per workgroup
     static constexpr int ROWB = 2 * KB;             // bytes per LDS row
     static constexpr int UNITS = ROWB / 16;         // 16-byte units per row
     static constexpr int RPB = 1024 / ROWB;         // rows per 1 KB load block
-    static constexpr int BVX = 64 * NB;             // output voxels per workgroup
+    static constexpr int BVX = 32 * NB * VW;        // output voxels per workgroup
     static constexpr int WTILE = BCH * ROWB;        // bytes of one W tile
     static constexpr int XTILE = BVX * ROWB;        // bytes of one X tile
     static constexpr int WJ = WTILE / 1024 / NW;    // W load blocks per wave per k-tile
@@ -97,9 +97,9 @@ struct ConvCfg {
     static constexpr int PAD = XJ * NW > XBLK ? 1024 : 0;
     static constexpr int STAGE = WTILE + XTILE + PAD;  // W tile, X tile, pad
     static constexpr int LOADS = WJ + XJ;
-    static constexpr int OCC = CW == 2 ? 2 : 1;     // workgroups per CU
+    static constexpr int OCC = NW == 4 ? 2 : 1;     // workgroups per CU
     static_assert(KB == 32 || KB == 64, "k-tile");
-    static_assert(CW == 2 || CW == 4, "channel waves");
+    static_assert(NW == 4 || NW == 8, "waves");
     static_assert(WJ * NW * 1024 == WTILE && XBLK * 1024 == XTILE, "whole load blocks");
     static_assert(NST * STAGE * OCC <= 160 * 1024, "LDS");
     static_assert(NST >= 2 && NST <= 4, "ring depth");
@@ -157,9 +157,9 @@ __device__ __forceinline__ int tile_of(int L, int n) {
 #if defined(__HIP_DEVICE_COMPILE__)
 // One workgroup of conv3d_mfma (SPLIT: of conv3d_part). SMALLC: C < KB, so
 // that one k-tile can cross several taps.
-template <int NB, int NST, int KB, int CW, bool SMALLC, bool SPLIT>
+template <int NB, int NST, int KB, int CW, int VW, bool SMALLC, bool SPLIT>
 __device__ __forceinline__ void conv_tile(const ConvArgs a) {
-    using Cf = ConvCfg<NB, NST, KB, CW>;
+    using Cf = ConvCfg<NB, NST, KB, CW, VW>;
     constexpr int STAGE = Cf::STAGE, LOADS = Cf::LOADS, ROWB = Cf::ROWB, UNITS = Cf::UNITS;
     constexpr int RPB = Cf::RPB, WJ = Cf::WJ, XJ = Cf::XJ, NW = Cf::NW;
     // The ring's stages are separate arrays, so that the compiler can tell
@@ -414,19 +414,20 @@ __global__ void __launch_bounds__((ConvCfg<NB, NST, KB, CW>::NT),
                                   (ConvCfg<NB, NST, KB, CW>::OCC * ConvCfg<NB, NST, KB, CW>::NW / 4))
     conv3d_mfma(const ConvArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    conv_tile<NB, NST, KB, CW, SMALLC, false>(a);
+    conv_tile<NB, NST, KB, CW, 2, SMALLC, false>(a);
 #endif
 }
 
-// The same with the reduction split in a.nsplit ranges (a kernel of its own:
-// the range's bounds and second epilogue cost the unsplit form 1 %): nsplit
-// times as many workgroups, split-major.
-template <int NB, int NST, int KB, int CW, bool SMALLC>
-__global__ void __launch_bounds__((ConvCfg<NB, NST, KB, CW>::NT),
-                                  (ConvCfg<NB, NST, KB, CW>::OCC * ConvCfg<NB, NST, KB, CW>::NW / 4))
+// Any number of voxel waves and, with SPLIT, the reduction split in a.nsplit
+// ranges: nsplit times as many workgroups, split-major. (Kernels of their own:
+// a range's bounds and second epilogue cost the unsplit form 1 %.)
+template <int NB, int NST, int KB, int CW, int VW, bool SMALLC, bool SPLIT>
+__global__ void __launch_bounds__((ConvCfg<NB, NST, KB, CW, VW>::NT),
+                                  (ConvCfg<NB, NST, KB, CW, VW>::OCC *
+                                   ConvCfg<NB, NST, KB, CW, VW>::NW / 4))
     conv3d_part(const ConvArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    conv_tile<NB, NST, KB, CW, SMALLC, true>(a);
+    conv_tile<NB, NST, KB, CW, VW, SMALLC, SPLIT>(a);
 #endif
 }
 
@@ -465,21 +466,28 @@ __global__ void __launch_bounds__(256) conv3d_reduce(const ConvArgs a) {
 #endif
 }
 
-// Launches configuration (NB, NST, KB, CW) over the whole problem.
-template <int NB, int NST, int KB, int CW>
-void launch_cfg(const ConvArgs& a, hipStream_t stream) {
-    using Cf = ConvCfg<NB, NST, KB, CW>;
+// Launches configuration (NB, NST, KB, CW, VW) over the whole problem.
+template <int NB, int NST, int KB, int CW, int VW, bool SMALLC>
+void launch_c(const ConvArgs& a, hipStream_t stream) {
+    using Cf = ConvCfg<NB, NST, KB, CW, VW>;
     const unsigned tiles = (unsigned)((a.M + Cf::BVX - 1) / Cf::BVX) *
                            (unsigned)((a.K + Cf::BCH - 1) / Cf::BCH) * (unsigned)a.nsplit;
     const dim3 grid(tiles), block(Cf::NT);
-    if (a.C < KB && a.nsplit > 1)
-        hipLaunchKernelGGL((conv3d_part<NB, NST, KB, CW, true>), grid, block, 0, stream, a);
-    else if (a.C < KB)
-        hipLaunchKernelGGL((conv3d_mfma<NB, NST, KB, CW, true>), grid, block, 0, stream, a);
-    else if (a.nsplit > 1)
-        hipLaunchKernelGGL((conv3d_part<NB, NST, KB, CW, false>), grid, block, 0, stream, a);
+    if (a.nsplit > 1)
+        hipLaunchKernelGGL((conv3d_part<NB, NST, KB, CW, VW, SMALLC, true>), grid, block, 0, stream,
+                           a);
+    else if constexpr (VW == 2)
+        hipLaunchKernelGGL((conv3d_mfma<NB, NST, KB, CW, SMALLC>), grid, block, 0, stream, a);
     else
-        hipLaunchKernelGGL((conv3d_mfma<NB, NST, KB, CW, false>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((conv3d_part<NB, NST, KB, CW, VW, SMALLC, false>), grid, block, 0,
+                           stream, a);
+}
+template <int NB, int NST, int KB, int CW, int VW = 2>
+void launch_cfg(const ConvArgs& a, hipStream_t stream) {
+    if (a.C < KB)
+        launch_c<NB, NST, KB, CW, VW, true>(a, stream);
+    else
+        launch_c<NB, NST, KB, CW, VW, false>(a, stream);
 }
 
 thread_local char g_err[256];
@@ -497,23 +505,32 @@ int fail(const char* msg) {
 
 bool mult8(long v) { return v >= 0 && v % 8 == 0; }
 
-// The kernel configurations: NB, KB, channels per workgroup (64*CW),
-// workgroups per CU, and the time in us of a 64-voxel x 256-channel piece of a
-// tile: `per_kg` for a reduction of 13824 elements, `fixed` for start-up and
-// epilogue (fitted on MI355X, see plan_conv); launcher.
+// The kernel configurations: voxels / 64, KB, channels per workgroup (64*CW),
+// workgroups per CU, the time in us of a 64-voxel x 256-channel piece of a tile
+// (`per_kg` for a reduction of 13824 elements, `fixed` for start-up and
+// epilogue; fitted on MI355X, see plan_conv) and how much longer a workgroup
+// that shares its CU takes than one alone; launcher. The last two have four
+// waves along the voxels: 256 voxels x 128 channels in one workgroup of eight
+// waves load a quarter less per output than two workgroups of 128 x 128 (a
+// strided 128 -> 128 layer of 65,536 voxels 69 -> 64 us, stride 1 66 -> 58),
+// 128 x 64 wastes less on 64 and 192 channels (64 -> 64 of 98,304 voxels 49 ->
+// 35 us) and makes more, shorter workgroups of small problems (512 -> 512 of
+// 256 voxels 22 -> 16 us).
 struct ConvKernel {
     int nb, kb, bch, occ;
-    double per_kg, fixed;
+    double per_kg, fixed, shared;
     void (*launch)(const ConvArgs&, hipStream_t);
 };
 const ConvKernel kKernels[] = {
-    {4, 32, 128, 2, 88.8, 2.1, launch_cfg<4, 3, 32, 2>},
-    {3, 64, 128, 2, 89.5, 2.3, launch_cfg<3, 2, 64, 2>},
-    {2, 64, 128, 2, 105.9, 2.0, launch_cfg<2, 2, 64, 2>},
-    {4, 32, 256, 1, 81.5, 1.6, launch_cfg<4, 4, 32, 4>},
-    {3, 64, 256, 1, 85.0, 1.5, launch_cfg<3, 2, 64, 4>},
-    {2, 64, 256, 1, 78.5, 2.6, launch_cfg<2, 3, 64, 4>},
-    {3, 32, 256, 1, 92.0, 1.7, launch_cfg<3, 4, 32, 4>},
+    {4, 32, 128, 2, 91.2, 3.7, 0.82, launch_cfg<4, 3, 32, 2>},
+    {3, 64, 128, 2, 91.9, 3.4, 0.55, launch_cfg<3, 2, 64, 2>},
+    {2, 64, 128, 2, 103.7, 3.9, 0.55, launch_cfg<2, 2, 64, 2>},
+    {4, 32, 256, 1, 74.7, 3.7, 0.0, launch_cfg<4, 4, 32, 4>},
+    {3, 64, 256, 1, 87.4, 3.0, 0.0, launch_cfg<3, 2, 64, 4>},
+    {2, 64, 256, 1, 77.8, 4.6, 0.0, launch_cfg<2, 3, 64, 4>},
+    {3, 32, 256, 1, 91.0, 3.1, 0.0, launch_cfg<3, 4, 32, 4>},
+    {4, 64, 128, 1, 81.4, 4.7, 0.0, launch_cfg<2, 3, 64, 2, 4>},
+    {2, 64, 64, 2, 116.2, 5.6, 0.77, launch_cfg<1, 3, 64, 1, 4>},
 };
 constexpr int kNumKernels = sizeof(kKernels) / sizeof(kKernels[0]);
 
@@ -535,13 +552,13 @@ int find_kernel(int nb, int kb, int bch) {
 // CUs idle and took 183 us; in 8 ranges it takes 42.
 // Estimate: R x tile size x (per_kg x range / 13824 + fixed), R the
 // workgroups on the busiest CU in units of one workgroup's time (for two per
-// CU: half rounds, a workgroup left alone on its CU at the end counting 1.3
-// halves, and 1.65 where every CU has just one, whose four waves then hide
-// little of their own latency), plus for a split the reduce kernel: a launch,
-// a little per range (its loads go out four ranges at a time) and the partial
-// sums' traffic. Fitted to 15 layers on MI355X (1 to 3x3x3 windows, 16 to 512
-// channels, 256 to 65,536 voxels) over every configuration and 1 to 24
-// ranges: the chosen pair is within 3 % of the fastest one on average.
+// CU: halves of a pair's time, one workgroup alone taking 2 - `shared` halves
+// and an odd last one 1.25), plus for a split the reduce kernel: a launch, a
+// little per range (its loads go out four ranges at a time) and the partial
+// sums' traffic. Fitted to 24 layers on MI355X (1 to 3x3x3 windows, 16 to 512
+// channels, 256 to 150,000 voxels) over every configuration and 1 to 24
+// ranges: the chosen pair is within 1 % of the fastest one on average, 6 % at
+// worst.
 // For tests, read on every call: GFX906_AMD_CONV_CFG = "<NB>x<KB>" (128
 // channels) or "<NB>x<KB>x<channels>" (a row of kKernels) fixes the
 // configuration, unsplit unless GFX906_AMD_CONV_NSPLIT = n asks for n ranges
@@ -550,8 +567,11 @@ int find_kernel(int nb, int kb, int bch) {
 constexpr int kSplitUnit = 64;     // reduction elements
 constexpr int kSplitMinUnits = 4;  // shortest range worth a workgroup
 constexpr int kSplitMax = 64;
-constexpr double kSplitMargin = 1.12;  // a split has to be this much better than none
-constexpr double kRedLaunch = 2.5, kRedPerSplit = 0.5, kRedPerByte = 0.2e-6;  // us
+// A split has to be this much better than none: CUs left idle let the others
+// hold a higher clock (512 -> 512 of 17,812 voxels, 186 workgroups unsplit: 250
+// us, and 274 in two ranges that the estimate has 1.4 % ahead).
+constexpr double kSplitMargin = 1.12;
+constexpr double kRedLaunch = 1.2, kRedPerSplit = 0.15, kRedPerByte = 0.14e-6;  // us
 struct ConvPlan {
     int cfg, nsplit, split_len;
 };
@@ -606,7 +626,7 @@ ConvPlan plan_conv(long M, int K, long KG, size_t ws_cap) {
             const ConvKernel& c = kKernels[i];
             const unsigned n = (tiles1[i] * (unsigned)p.nsplit + ncu - 1) / ncu;
             double r = n;  // workgroups on the busiest CU
-            if (c.occ == 2) r += n == 1 ? 0.65 : n & 1 ? 0.3 : 0.0;  // (half rounds)
+            if (c.occ == 2) r += n == 1 ? 1.0 - c.shared : n & 1 ? 0.25 : 0.0;  // (halves)
             double cost = r * c.nb * c.bch / 256.0 * (c.per_kg * kgu + c.fixed) + red;
             if (p.nsplit > 1) cost *= kSplitMargin;
             if (cost < best_cost) {

@@ -70,10 +70,10 @@ CASES = [  # x, (k, window), stride, bias, residual; C = 8: a unit spans taps, 2
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("nsplit", [2, 3, 4, 5, 8, 64])
+@pytest.mark.parametrize("nsplit", [1, 2, 3, 4, 5, 8, 64])
 @pytest.mark.parametrize("i", range(len(CASES)))
 @pytest.mark.parametrize("cfg", ["4x32", "3x64", "2x64", "4x32x256", "3x64x256", "2x64x256",
-                                 "3x32x256"])
+                                 "3x32x256", "4x64x128", "2x64x64"])
 def test_forced_split_counts(monkeypatch, cfg, i, nsplit):
     xs, ws, stride, has_b, has_r = CASES[i]
     print(f"case conv split: {cfg} {xs} {ws} n{nsplit}", flush=True)

@@ -167,3 +167,11 @@ def test_tail_kernels_keep_occupancy_without_spills(kernel_asm):
             seen.append(name)
             assert occ >= want and vgprs <= 512 // want and scratch == 0, (name, vgprs, scratch)
     assert len(seen) == 10, seen  # D = 128, and 64 and padded with and without the tile max
+
+
+def test_conv3d_split_and_wide_kernels_do_not_spill(conv_asm):
+    found = [(m.group(1), int(m.group(2)), int(m.group(3)), int(m.group(4)))
+             for m in RESOURCES.finditer(conv_asm) if "conv3d_part" in m.group(1)]
+    assert len(found) == 22, len(found)  # nine split configurations and two unsplit, x small/large C
+    for name, vgprs, scratch, occ in found:
+        assert scratch == 0 and occ >= 2 and vgprs <= 256, (name, vgprs, scratch, occ)
