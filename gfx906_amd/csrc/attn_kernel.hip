@@ -56,6 +56,7 @@
 #include <math.h>
 #include <type_traits>
 #include <algorithm>
+#include <stdio.h>
 #include <stdlib.h>
 
 #include "gfx906_amd_attn.h"
@@ -1420,6 +1421,245 @@ __global__ void __launch_bounds__(CfgRes::NT, 1) attn_fwd_kvres(const KArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// D <= 128, few query rows: the key range shared out inside the workgroup.
+//
+// A problem whose 256-row workgroups leave most CUs idle (one short head, a
+// few query rows against a long context) is bound by latencies, not by the
+// matrix cores: with the keys split over workgroups it pays a cold start of
+// every workgroup, the partial results' way through memory and the merge's
+// launch. Here a workgroup takes 32 query rows and its eight waves each every
+// eighth step of the keys (64 keys for D <= 64, 32 for D = 128: 8 KB of K and
+// 8 KB of V in LDS of the wave's own, so no barrier in the loop). A wave's K
+// and V have one buffer each: K of the next step loads while this step's
+// softmax and PV run, V while the next QK^T does. At the end the eight (O, m,
+// l) are merged through LDS, as attn_combine merges key ranges, and stored;
+// with SPLIT (few rows against many keys) the keys are also split over
+// workgroups and the merged (O, m, l) go to the workspace.
+// The running max is exact (raised over a whole step before its P), for every
+// head dim, so a row's dominant weight is 1.0 in its wave's range.
+template <int DP_, int NBQ_>
+struct CfgRows {
+    static constexpr int DP = DP_, WAVES = 8, NT = WAVES * 64;
+    static constexpr int NBQ = NBQ_, BM = 16 * NBQ;  // 16-row column blocks, rows
+    // A wave's K or V step as tile_offsets and issue_tile see it.
+    static constexpr int NW = 1, BN = DP == 64 ? 64 : 32, NU = DP / 8, RB = DP * 2;
+    static constexpr int TILE = BN * RB, BLKS = TILE / 1024;
+    static_assert(TILE == 8192, "8 KB per wave and operand");
+};
+
+// grid: ceil(Sq / (16*NBQ)) * B*H workgroups (times nsplit); block: 512 threads.
+template <int DP, int NBQ, bool PAD, class T, bool SPLIT>
+__global__ void __launch_bounds__((CfgRows<DP, NBQ>::NT), 2) attn_fwd_rows(const KArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    using C = CfgRows<DP, NBQ>;
+    using E = Elem<T>;
+    using x8 = typename E::x8;
+    constexpr int NU = C::NU, RB = C::RB, BN = C::BN, TILE = C::TILE, BLKS = C::BLKS;
+    constexpr int NQF = DP / 32, NOB = DP / 16, NB32 = BN / 32, W = C::WAVES;
+    static_assert(BLKS == 8, "wait counts");
+    __shared__ __attribute__((aligned(1024))) char kbuf[W * TILE];
+    __shared__ __attribute__((aligned(1024))) char vbuf[W * TILE];
+    __shared__ f32x2 ml[W * C::BM];
+
+    const int Sq = a.Sq, D = a.D;
+    const float c = a.c;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 15, g = lane >> 4;
+    const int nqt = (Sq + C::BM - 1) / C::BM;
+    const WorkItem it = work_item<SPLIT, false>(a, blockIdx.x, gridDim.x, nqt);
+    const int b = it.bh / a.H, h = it.bh - b * a.H;
+    const int kv0 = SPLIT ? it.split * a.split_len : 0;
+    const int Skv = SPLIT ? max(0, min(a.Skv - kv0, a.split_len)) : a.Skv;
+    const T* Qh = (const T*)a.q + b * a.sq.b + h * a.sq.h + (long long)it.qt * C::BM * a.sq.s;
+    const T* Kh = (const T*)a.k + b * a.sk.b + h * a.sk.h + kv0 * a.sk.s;
+    const T* Vh = (const T*)a.v + b * a.sv.b + h * a.sv.h + kv0 * a.sv.s;
+    const int rows = min(Sq - it.qt * C::BM, C::BM);
+    char* const kt = kbuf + wave * TILE;
+    char* const vt = vbuf + wave * TILE;
+
+    int koff[BLKS], voff[BLKS];
+    tile_offsets<C, PAD>(koff, voff, D, (int)a.sk.s, (int)a.sv.s, 0, lane);
+    const int nsteps = (Skv + BN - 1) / BN;
+    // This wave's loads of step st (past the end: an empty range, zeros).
+    auto issue_k = [&](int st) __attribute__((always_inline)) {
+        issue_tile<C>(Kh, st * BN, Skv, D, a.sk.s, kt, 0, koff);
+    };
+    auto issue_v = [&](int st) __attribute__((always_inline)) {
+        issue_tile<C>(Vh, st * BN, Skv, D, a.sv.s, vt, 0, voff);
+    };
+    // Q^T fragments of the rows, the same in every wave.
+    x8 qf[NBQ][NQF];
+    const unsigned qneg = a.qsign < 0.f ? 0x80008000u : 0u;
+    if ((long long)(C::BM - 1) * a.sq.s * 2 + DP * 2 < (1LL << 31)) {  // (uniform)
+        const __amdgpu_buffer_rsrc_t qr = q_rsrc(Qh, rows, a.sq.s, D);
+#pragma unroll
+        for (int nb = 0; nb < NBQ; ++nb)
+#pragma unroll
+            for (int s = 0; s < NQF; ++s) {
+                const int d0 = 32 * s + 8 * g, r = 16 * nb + i;
+                qf[nb][s] = q_load<T>(qr, r < rows && (!PAD || d0 < D)
+                                              ? (unsigned)((r * a.sq.s + d0) * 2)
+                                              : kQOutOfRange);
+            }
+    } else {
+#pragma unroll
+        for (int nb = 0; nb < NBQ; ++nb)
+#pragma unroll
+            for (int s = 0; s < NQF; ++s) {
+                const int d0 = 32 * s + 8 * g, r = 16 * nb + i;
+                qf[nb][s] = q_fragment(Qh + r * a.sq.s + d0, r < rows && (!PAD || d0 < D), 0u);
+            }
+    }
+    issue_k(wave);
+    issue_v(wave);
+
+    // LDS reads as in attn_fwd_pipe.
+    int kaddr[NQF], vaddr[NOB];
+#pragma unroll
+    for (int s = 0; s < NQF; ++s) kaddr[s] = i * RB + ((4 * s + g) ^ kswz<NU>(i)) * 16;
+    {
+        const int vrow = 4 * g + (i >> 2), vx = vswz<NU>(vrow) >> 1;
+#pragma unroll
+        for (int ob = 0; ob < NOB; ++ob) vaddr[ob] = vrow * RB + (ob ^ vx) * 32 + (i & 3) * 8;
+    }
+    f32x4 oacc[NOB][NBQ];
+    float m_run[NBQ], l_run[NBQ];  // running max (score units), sum of this lane's keys
+#pragma unroll
+    for (int nb = 0; nb < NBQ; ++nb) {
+        m_run[nb] = -INFINITY;
+        l_run[nb] = 0.f;
+#pragma unroll
+        for (int ob = 0; ob < NOB; ++ob) oacc[ob][nb] = f32x4{};
+    }
+
+    for (int st = wave; st < nsteps; st += W) {
+        if (st == wave && qneg) {
+#pragma unroll
+            for (int nb = 0; nb < NBQ; ++nb)
+#pragma unroll
+                for (int s = 0; s < NQF; ++s) q_negate(qf[nb][s], qneg);
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70 | BLKS);  // K of this step landed; V may be in flight
+        asm volatile("" ::: "memory");
+        f32x4 S[2 * NB32][NBQ];  // 16-key blocks x column blocks
+#pragma unroll
+        for (int kb = 0; kb < 2 * NB32; ++kb)
+#pragma unroll
+            for (int nb = 0; nb < NBQ; ++nb) S[kb][nb] = f32x4{};
+#pragma unroll
+        for (int s = 0; s < NQF; ++s)
+#pragma unroll
+            for (int kb = 0; kb < 2 * NB32; ++kb) {
+                const x8 kf = lds_read16<T>(kt, kaddr[s] + 16 * kb * RB);
+#pragma unroll
+                for (int nb = 0; nb < NBQ; ++nb) S[kb][nb] = E::mma16(kf, qf[nb][s], S[kb][nb]);
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // K is read: its buffer is free
+        issue_k(st + W);
+        if (st * BN + BN > Skv) {  // the last, partial step
+#pragma unroll
+            for (int kb = 0; kb < 2 * NB32; ++kb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (st * BN + 16 * kb + 4 * g + r >= Skv)
+#pragma unroll
+                        for (int nb = 0; nb < NBQ; ++nb) S[kb][nb][r] = -INFINITY;
+        }
+        x8 P[NB32][NBQ];
+#pragma unroll
+        for (int nb = 0; nb < NBQ; ++nb) {
+            float mx = S[0][nb][0];
+#pragma unroll
+            for (int kb = 0; kb < 2 * NB32; ++kb) {
+                mx = max3(mx, S[kb][nb][0], S[kb][nb][1]);
+                mx = max3(mx, S[kb][nb][2], S[kb][nb][3]);
+            }
+            if (__any(mx > m_run[nb])) {
+                const float m_new = max2(m_run[nb], quad_group_max(mx));
+                const float alpha = __builtin_amdgcn_exp2f((m_run[nb] - m_new) * c);
+                if (st != wave) {  // (O and l are still zero on the wave's first step)
+#pragma unroll
+                    for (int ob = 0; ob < NOB; ++ob) oacc[ob][nb] *= alpha;
+                    l_run[nb] *= alpha;
+                }
+                m_run[nb] = m_new;
+            }
+#pragma unroll
+            for (int blk = 0; blk < NB32; ++blk)
+                block_exp<T, true>(S[2 * blk][nb], S[2 * blk + 1][nb], P[blk][nb], -m_run[nb] * c,
+                                   c, l_run[nb]);
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70 | BLKS);  // V of this step landed; the next K may be
+        asm volatile("" ::: "memory");              // in flight
+#pragma unroll
+        for (int blk = 0; blk < NB32; ++blk)
+#pragma unroll
+            for (int ob = 0; ob < NOB; ++ob) {
+                const int off = vaddr[ob] + 32 * blk * RB;
+                const x8 vf = lds_read_tr2<T>(vt, off, off + 16 * RB);
+#pragma unroll
+                for (int nb = 0; nb < NBQ; ++nb)
+                    oacc[ob][nb] = E::mma16(vf, P[blk][nb], oacc[ob][nb]);
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // V is read: its buffer is free
+        issue_v(st + W);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): loads past the end must land first
+    lds_barrier();                      // every wave is done with its buffers
+    // O of wave w, fp32 rows of DP dims in 16-byte units: four (D = 128) or
+    // eight waves per array. Unit u of row r sits at u ^ (r & 15).
+    constexpr int OROW = DP * 4, OWAVE = C::BM * OROW, PERBUF = W * TILE / OWAVE, OU = DP / 4;
+    char* const od = (wave < PERBUF ? kbuf : vbuf) + (wave % PERBUF) * OWAVE;
+#pragma unroll
+    for (int nb = 0; nb < NBQ; ++nb) {
+        const int r = 16 * nb + i;
+        const float l = quad_group_sum(l_run[nb]);
+#pragma unroll
+        for (int ob = 0; ob < NOB; ++ob)
+            *(LDS_AS f32x4*)((LDS_AS char*)od + r * OROW + ((4 * ob + g) ^ (r & 15)) * 16) =
+                oacc[ob][nb];
+        if (g == 0) ml[wave * C::BM + r] = f32x2{m_run[nb] * c, l};  // log2 units
+    }
+    lds_barrier();
+#pragma unroll
+    for (int n = 0; n < C::BM * OU / C::NT; ++n) {
+        const int idx = n * C::NT + tid, r = idx / OU, u = idx - r * OU;
+        float mx = -3.0e38f;
+        f32x2 mlw[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            mlw[w] = ml[w * C::BM + r];
+            mx = fmaxf(mx, mlw[w][0]);
+        }
+        f32x4 acc = {};
+        float l = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const float wt = __builtin_amdgcn_exp2f(mlw[w][0] - mx);
+            acc += wt * *(const LDS_AS f32x4*)((const LDS_AS char*)(w < PERBUF ? kbuf : vbuf) +
+                                               (w % PERBUF) * OWAVE + r * OROW +
+                                               (u ^ (r & 15)) * 16);
+            l += wt * mlw[w][1];
+        }
+        const int row = it.qt * C::BM + r;
+        if (r >= rows || (PAD && 4 * u >= D)) continue;
+        if constexpr (SPLIT) {
+            const long long o = it.split * a.tail_rows + ((long long)it.bh * Sq + row);
+            *reinterpret_cast<f32x4*>(a.ws_o + o * D + 4 * u) = acc;
+            if (u == 0) *reinterpret_cast<f32x2*>(a.ws_ml + 2 * o) = f32x2{mx, l};
+        } else {
+            const float inv = l > 0.f ? 1.f / l : 0.f;
+            const auto h0 = E::cvt2(acc[0] * inv, acc[1] * inv);
+            const auto h1 = E::cvt2(acc[2] * inv, acc[3] * inv);
+            T* op = (T*)a.o + b * a.so.b + h * a.so.h + row * a.so.s + 4 * u;
+            *reinterpret_cast<typename E::x4*>(op) = typename E::x4{h0[0], h0[1], h1[0], h1[1]};
+        }
+    }
+#endif
+}
+
+// ---------------------------------------------------------------------------
 // D = 512: 16x16x32 MFMA tiles, 16 query rows per wave.
 //
 // With 32 query rows a wave would need a 256-register O accumulator; with 16
@@ -2022,15 +2262,37 @@ void launch_kernel(const KArgs& a, bool tl, hipStream_t s) {
     }
 }
 
+// The few-rows kernel (units of `rows` rows in a.tail).
+template <class T, bool SPLIT>
+void launch_rows(const KArgs& a, int rows, hipStream_t s) {
+    const dim3 grid((unsigned)a.tail * (unsigned)a.nsplit), block(CfgRows<64, 2>::NT);
+    if (a.D == 128)
+        hipLaunchKernelGGL((attn_fwd_rows<128, 2, false, T, SPLIT>), grid, block, 0, s, a);
+    else if (a.D == 64 && rows == 32)
+        hipLaunchKernelGGL((attn_fwd_rows<64, 2, false, T, SPLIT>), grid, block, 0, s, a);
+    else if (a.D == 64)
+        hipLaunchKernelGGL((attn_fwd_rows<64, 4, false, T, SPLIT>), grid, block, 0, s, a);
+    else if (rows == 32)
+        hipLaunchKernelGGL((attn_fwd_rows<64, 2, true, T, SPLIT>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((attn_fwd_rows<64, 4, true, T, SPLIT>), grid, block, 0, s, a);
+}
+
 // Launches the kernel for the whole problem, or (a.nsplit > 1) its split
 // key ranges and the merge.
 template <class T>
-hipError_t launch_t(const KArgs& a, bool tl, hipStream_t s) {
+hipError_t launch_t(const KArgs& a, bool tl, int rows, hipStream_t s) {
     if (a.nsplit <= 1) {
-        launch_kernel<T, false>(a, tl, s);
+        if (rows)
+            launch_rows<T, false>(a, rows, s);
+        else
+            launch_kernel<T, false>(a, tl, s);
         return hipGetLastError();
     }
-    launch_kernel<T, true>(a, tl, s);
+    if (rows)
+        launch_rows<T, true>(a, rows, s);
+    else
+        launch_kernel<T, true>(a, tl, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     CombArgs c;
@@ -2182,6 +2444,94 @@ size_t split_ws_bytes(const SplitPlan& p, int B, int H, int Sq, int D) {
     const size_t rows =
         (size_t)p.nsplit * ((long long)B * H * Sq - first_split_row(p.whole, Sq, D));
     return rows * D * 4 + rows * 2 * 4 + 16;
+}
+
+// The few-rows kernel for a problem it serves: rows per workgroup (0: another
+// kernel serves it), key ranges and their length.
+//
+// Both kernels' times are estimated in us and the smaller wins (the few-rows
+// kernel has to be kRowsMargin better, kRowsMarginRounds over several rounds,
+// where the estimate is 10-15 % off at times: B2 H4 Sq2439 Skv387 D64, 312
+// workgroups, 15.7 against 14.9). Few-rows: start + rounds of workgroups
+// (one per CU) x (fixed + step x steps of the busiest wave), combined in
+// quadrature with K and V's way from HBM, plus a split's merge. Ring:
+// start + rounds x (fixed + tile x tiles, in fours) of `ring`'s plan, plus its
+// merge. Fitted to 42 shapes on MI355X at each of D = 40, 64 and 128 (1 to
+// 4096 queries, 64 to 100,000 keys, 1 to 48 heads) with 1 to 128 ranges: the
+// choice costs 1 % over the faster kernel's best count on average. Measured
+// (us, ring kernel -> here): B1 H1 S1024 D64 13.2 -> 7.1, B1 H16 S512 D64 14.9
+// -> 6.0, B1 H8 S1024 D128 26.5 -> 12.1, one query over 100,000 keys, D = 64,
+// 43.6 -> 17.3, B1 H16 S1024 D64 (64 rows) 23.2 -> 11.6; past about two rounds
+// of workgroups the ring kernel's 256 rows per K/V tile win (B2 H16 Sq1024
+// Skv77 D64: 10.1 against 13.9).
+// For tests: GFX906_AMD_ATTN_ROWS = 0 selects the ring kernel, "n" or "n x 64"
+// (no spaces) this one with n ranges and 32 or 64 rows; the variables that
+// choose among the ring kernel's forms select it too.
+struct RowsPlan {
+    int rows, nsplit, split_len;
+};
+constexpr RowsPlan kNoRows{0, 0, 0};
+struct RowsCost {
+    double fixed, step, start;
+};
+constexpr RowsCost kRowsCost[3] = {{4.18, 1.26, 1.6},   // D = 128
+                                   {2.64, 1.24, 1.9},   // D <= 64, 32 rows
+                                   {3.50, 2.05, 2.0}};  // D <= 64, 64 rows
+constexpr double kRowsMergeLaunch = 1.6, kRowsMergeSplit = 0.13, kRowsMergeByte = 0.39e-6;
+constexpr double kRingFixed[2] = {4.7, 2.0}, kRingTile[2] = {1.66, 2.2};  // D = 128, <= 64
+constexpr double kRingStart = 1.3, kRingAlone = 0.68;
+constexpr double kRingMergeLaunch = 2.4, kRingMergeSplit = 0.13, kRingMergeByte = 0.27e-6;
+constexpr double kRowsHbm = 6.9e6;  // bytes per us
+constexpr double kRowsMargin = 1.06, kRowsMarginRounds = 1.13;
+RowsPlan rows_plan(int B, int H, int Sq, int Skv, int D, const SplitPlan& ring, size_t ws_cap) {
+    if (D > 128 || Skv == 0 || ring.whole > 0) return kNoRows;
+    const int bn = D == 128 ? CfgRows<128, 2>::BN : CfgRows<64, 2>::BN;
+    const int steps = (Skv + bn - 1) / bn;
+    if (const char* env = getenv("GFX906_AMD_ATTN_ROWS")) {
+        int n = 0, rows = 32;
+        if (sscanf(env, "%dx%d", &n, &rows) < 1 || n <= 0) return kNoRows;
+        const int per = (steps + std::min(n, steps) - 1) / std::min(n, steps);
+        return {D == 128 || rows != 64 ? 32 : 64, (steps + per - 1) / per, per * bn};
+    }
+    if (getenv("GFX906_AMD_ATTN_NSPLIT") || getenv("GFX906_AMD_ATTN_KVRES") ||
+        getenv("GFX906_AMD_ATTN_TILEMAX"))
+        return kNoRows;
+    const long long bh = (long long)B * H;
+    const int cus = cu_count(), cls = D == 128 ? 0 : 1;
+    const double rows_bytes = (double)bh * Sq * D * 8, kv_us = (double)bh * Skv * D * 4 / kRowsHbm;
+    // The ring kernel on its own plan.
+    const int slots = D == 128 ? cus : 2 * cus, tiles = (Skv + 63) / 64;
+    const long long wgs = bh * ((Sq + query_tile(D) - 1) / query_tile(D)) * ring.nsplit;
+    const int per_ring = (tiles + ring.nsplit - 1) / ring.nsplit;
+    const double alone = D != 128 && wgs <= cus ? kRingAlone : 1.0;
+    double best_t = kRingStart + (double)((wgs + slots - 1) / slots) *
+                                     (kRingFixed[cls] + kRingTile[cls] * alone * ((per_ring + 3) / 4 * 4));
+    if (ring.nsplit > 1)
+        best_t += kRingMergeLaunch + kRingMergeSplit * ring.nsplit +
+                  kRingMergeByte * rows_bytes * ring.nsplit;
+    RowsPlan best = kNoRows;
+    for (int rows = 32; rows <= (D == 128 ? 32 : 64); rows *= 2) {
+        const RowsCost& rc = kRowsCost[D == 128 ? 0 : rows / 32];
+        const long long units = bh * ((Sq + rows - 1) / rows);
+        if (units > 4LL * cus) continue;
+        for (int n = 1; n <= 128 && n <= steps; n += n < 4 ? 1 : n / 3) {
+            const int per = (steps + n - 1) / n, ns = (steps + per - 1) / per;
+            if (ns > 1 && (units * ns > 4LL * cus ||
+                           split_ws_bytes({ns, per * bn, 0}, B, H, Sq, D) > ws_cap))
+                break;
+            const long long rounds = (units * ns + cus - 1) / cus;
+            const double comp = (double)rounds * (rc.fixed + rc.step * ((per + 7) / 8));
+            double t = rc.start + sqrt(comp * comp + kv_us * kv_us);
+            if (ns > 1)
+                t += kRowsMergeLaunch + kRowsMergeSplit * ns + kRowsMergeByte * rows_bytes * ns;
+            t *= rounds > 1 ? kRowsMarginRounds : kRowsMargin;
+            if (t < best_t) {
+                best_t = t;
+                best = {rows, ns, per * bn};
+            }
+        }
+    }
+    return best;
 }
 
 // Whether two elements of an output tensor can share an address: the
@@ -2341,10 +2691,10 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     a.row0 = 0;
     a.tail_rows = (long long)B * H * Sq;
     const bool tl = token_contiguous(sk, sv, D);
-    SplitPlan p = kNoSplit;
-    if (workspace_bytes != (size_t)-1)  // split the keys if it pays
-        p = plan_split(B, H, Sq, Skv, D, D != 512 || tl || d512_wide(),
-                       use_scratch ? kScratchBytes : (size_t)-1);
+    // Split the keys if it pays and the call may.
+    const SplitPlan ring = plan_split(B, H, Sq, Skv, D, D != 512 || tl || d512_wide(),
+                                      use_scratch ? kScratchBytes : (size_t)-1);
+    SplitPlan p = workspace_bytes != (size_t)-1 ? ring : kNoSplit;
     size_t need = split_ws_bytes(p, B, H, Sq, D);
     // A grid that fills the GPU needs no workspace: without one (under
     // capture, where the static scratch would tie the graph's replays to
@@ -2353,8 +2703,17 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
         p = kNoSplit;
         need = 0;
     }
+    // Few rows: another kernel, whose partial results (if any) fit the
+    // workspace of the plan above. A call that never splits takes it where the
+    // plan is not to split, so that every entry point gives the same bits
+    // there.
+    RowsPlan rp = kNoRows;
+    if (p.nsplit == ring.nsplit && !(p.nsplit <= 1 && kvres_grid(a)))
+        rp = rows_plan(B, H, Sq, Skv, D, p, need);
+    if (rp.nsplit > 1 && split_ws_bytes({rp.nsplit, rp.split_len, 0}, B, H, Sq, D) > need)
+        rp = kNoRows;  // (a forced count)
     ScratchUse scratch;
-    if (need && use_scratch) {
+    if (need && use_scratch && rp.nsplit != 1) {
         const ScratchUse::Status st = scratch.acquire(stream, p.whole == 0);
         if (st == ScratchUse::kUnavailable && p.whole > 0) {
             p = kNoSplit;
@@ -2370,7 +2729,7 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
         workspace = scratch.ptr;
         workspace_bytes = kScratchBytes;
     }
-    if (need) {
+    if (need && !(use_scratch && rp.nsplit == 1)) {
         if (!workspace || workspace_bytes < need || (uintptr_t)workspace % 16) {
             set_err("attn: workspace missing, misaligned or smaller than "
                     "attn_split_workspace_bytes()");
@@ -2385,8 +2744,14 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
         a.ws_o = (float*)workspace;
         a.ws_ml = a.ws_o + (size_t)p.nsplit * a.tail_rows * D;
     }
-    hipError_t e = dtype == ATTN_DTYPE_BF16 ? launch_t<bf16>(a, tl, stream)
-                                            : launch_t<f16>(a, tl, stream);
+    if (rp.rows) {
+        a.nsplit = rp.nsplit;
+        a.split_len = rp.split_len;
+        a.tail = B * H * ((Sq + rp.rows - 1) / rp.rows);
+        a.ws_ml = a.ws_o + (size_t)rp.nsplit * a.tail_rows * D;
+    }
+    hipError_t e = dtype == ATTN_DTYPE_BF16 ? launch_t<bf16>(a, tl, rp.rows, stream)
+                                            : launch_t<f16>(a, tl, rp.rows, stream);
     if (e == hipSuccess) e = scratch.release(stream);
     if (e != hipSuccess) {
         set_err(hipGetErrorString(e));

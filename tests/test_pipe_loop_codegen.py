@@ -175,3 +175,11 @@ def test_conv3d_split_and_wide_kernels_do_not_spill(conv_asm):
     assert len(found) == 22, len(found)  # nine split configurations and two unsplit, x small/large C
     for name, vgprs, scratch, occ in found:
         assert scratch == 0 and occ >= 2 and vgprs <= 256, (name, vgprs, scratch, occ)
+
+
+def test_few_rows_kernels_do_not_spill(kernel_asm):
+    found = [(m.group(1), int(m.group(2)), int(m.group(3)), int(m.group(4)))
+             for m in RESOURCES.finditer(kernel_asm) if "attn_fwd_rows" in m.group(1)]
+    assert len(found) == 20, len(found)  # D = 128; 64 and padded x 32 and 64 rows; split, dtype
+    for name, vgprs, scratch, occ in found:
+        assert scratch == 0 and occ >= 2 and vgprs <= 256, (name, vgprs, scratch, occ)
