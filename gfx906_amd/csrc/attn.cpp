@@ -77,6 +77,15 @@ bool token_contiguous_kv(const torch::Tensor& t) {
     return (D - 1) * s[3] + S < (int64_t(1) << 30);
 }
 
+// Whether t's tokens lie in 16-byte aligned runs: sequence stride 1, the
+// other strides multiples of 8 (the head dim's other than 1).
+bool token_runs(const torch::Tensor& t) {
+    const auto s = strides4(t);
+    return t.stride(2) == 1 && s[3] != 1 && s[3] % 8 == 0 && s[0] >= 0 && s[1] >= 0 &&
+           s[0] % 8 == 0 && s[1] % 8 == 0 && s[3] > 0 &&
+           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+
 // Largest Skv for which reading token-contiguous k/v in place beats copying
 // them (see the file comment).
 constexpr int64_t kInPlaceMaxSkv = 6400;
@@ -118,11 +127,15 @@ torch::Tensor attn(torch::Tensor q, torch::Tensor k, torch::Tensor v, double sca
         o = torch::empty({B, H, Sq, D}, q.options().memory_format(at::MemoryFormat::Contiguous));
     }
     if (o.numel() == 0) return o;
-    // Token-contiguous k and v (D = 512, Skv <= kInPlaceMaxSkv): read in
-    // place, q and out with any strides. Otherwise the head dim of every
+    // Token-contiguous k and v (D = 512): read in place up to kInPlaceMaxSkv,
+    // q and out with any strides; above, with q and out of the same kind, the
+    // library makes row copies. Otherwise the head dim of every
     // tensor the kernel touches is contiguous: inputs are copied and out
     // staged as needed.
-    const bool tl = Skv <= kInPlaceMaxSkv && token_contiguous_kv(k) && token_contiguous_kv(v);
+    const bool tokens = token_contiguous_kv(k) && token_contiguous_kv(v) && Skv > 0;
+    const bool copied = tokens && Skv > kInPlaceMaxSkv && token_runs(q) && Sq % 8 == 0 &&
+                        token_runs(o) && B * H * 3 <= 65535;  // (the copies' grid)
+    const bool tl = tokens && (Skv <= kInPlaceMaxSkv || copied);
     const auto qi = tl ? q : as_input(q, false);
     const auto ki = tl ? k : as_input(k, true), vi = tl ? v : as_input(v, true);
     const bool staged = !tl && o.stride(3) != 1;
@@ -136,6 +149,17 @@ torch::Tensor attn(torch::Tensor q, torch::Tensor k, torch::Tensor v, double sca
     const size_t ws_bytes = attn_split_workspace_bytes((int)B, (int)H, (int)Sq, (int)Skv, (int)D);
     torch::Tensor ws;
     if (ws_bytes) ws = torch::empty({(int64_t)ws_bytes}, q.options().dtype(torch::kUInt8));
+    if (copied) {  // row copies made by the library, in one launch
+        const size_t n = attn_row_copies_bytes((int)B, (int)H, (int)Sq, (int)Skv, (int)D);
+        const auto rows = torch::empty({(int64_t)n}, q.options().dtype(torch::kUInt8));
+        const int rc = attn_fwd_split_copied(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), (int)B, (int)H, (int)Sq,
+            (int)Skv, (int)D, (float)scale, c10::hip::getCurrentHIPStream().stream(), dtype,
+            sq.data(), sk.data(), sv.data(), so.data(), ws_bytes ? ws.data_ptr() : nullptr,
+            ws_bytes, rows.data_ptr(), n);
+        TORCH_CHECK(rc == 0, "kernel: ", attn_last_error() ? attn_last_error() : "launch failed");
+        return o;
+    }
     const int rc = attn_fwd_split(qi.data_ptr(), ki.data_ptr(), vi.data_ptr(), oo.data_ptr(), (int)B,
                                   (int)H, (int)Sq, (int)Skv, (int)D, (float)scale,
                                   c10::hip::getCurrentHIPStream().stream(), dtype, sq.data(),

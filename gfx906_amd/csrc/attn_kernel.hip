@@ -2001,6 +2001,49 @@ static_assert(Cfg512W::BM == Cfg512::BM, "same query tiling as attn_fwd_d512 (gr
 #undef D512W_KERNEL
 #undef D512W_TL
 
+// Row copies of token-contiguous tensors ([D][S] per head to [S][D], D = 512):
+// 64 tokens x 64 dims per workgroup through LDS, read back transposed (eight
+// dims of one token per lane) so that loads and stores both move 16 bytes per
+// lane in 64- and 128-byte runs. q, k and v in one launch; bound by memory
+// (14,400 bf16 tokens: 88 MB; torch's copies took 31 us a tensor).
+struct TokCopyArgs {
+    const void* src[3];
+    void* dst[3];
+    Strides st[3];
+    int S[3];
+    int H, BH;
+};
+// grid: (ceil(max S / 64), 8, 3 * B*H); block: 256 threads.
+template <class T>
+__global__ void __launch_bounds__(256) tok_to_rows(const TokCopyArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    using x8 = typename Elem<T>::x8;
+    constexpr int RB = 144;  // LDS bytes per dim row: 64 tokens and 16 bytes of padding
+    __shared__ __attribute__((aligned(16))) char tile[64 * RB];
+    const int n = (int)blockIdx.z / a.BH, bh = (int)blockIdx.z - n * a.BH;
+    const int S = a.S[n], tok0 = (int)blockIdx.x * 64, dim0 = (int)blockIdx.y * 64;
+    if (tok0 >= S) return;  // (uniform)
+    const int b = bh / a.H, h = bh - b * a.H, tid = threadIdx.x;
+    const Strides st = a.st[n];
+    const T* src = (const T*)a.src[n] + b * st.b + h * st.h + dim0 * st.d + tok0;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const int d = (tid >> 3) + 32 * p, t = (tid & 7) * 8;
+        if (tok0 + t < S)  // (S is a multiple of 8)
+            *reinterpret_cast<x8*>(tile + d * RB + t * 2) = ld_global16(src + d * st.d + t);
+    }
+    __syncthreads();
+    const int lane = tid & 63, i = lane & 15, g = lane >> 4, tw = (tid >> 6) * 16;
+    T* dst = (T*)a.dst[n] + ((long long)bh * S + tok0 + tw + i) * 512 + dim0;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const int d = 32 * p + 8 * g, off = (d + (i >> 2)) * RB + (tw + 4 * (i & 3)) * 2;
+        const x8 val = lds_read_tr2<T>(tile, off, off + 4 * RB);
+        if (tok0 + tw + i < S) *reinterpret_cast<x8*>(dst + d) = val;
+    }
+#endif
+}
+
 // Merge of the split key ranges: per output row, with m* the largest
 // running max of its splits and w_s = exp2(m_s - m*),
 //     o = sum_s w_s O_s / sum_s w_s l_s
@@ -2226,7 +2269,7 @@ void launch_kernel(const KArgs& a, bool tl, hipStream_t s) {
     if (D == 512) {
         if (tl)
             hipLaunchKernelGGL((attn_fwd_tok512<T, SPLIT>), grid, dim3(Cfg512W::NT), 0, s, a);
-        else if (d512_wide())
+        else if (d512_wide() || a.o_tok)  // (only the wide kernel stores tokens)
             hipLaunchKernelGGL((attn_fwd_d512w<T, SPLIT>), grid, dim3(Cfg512W::NT), 0, s, a);
         else
             hipLaunchKernelGGL((attn_fwd_d512<T, SPLIT>), grid, dim3(Cfg512::NT), 0, s, a);
@@ -2307,7 +2350,7 @@ hipError_t launch_t(const KArgs& a, bool tl, int rows, hipStream_t s) {
     c.whole = a.whole;
     c.row0 = a.row0;
     c.rows = a.tail_rows;
-    if (tl && a.o_tok) {
+    if (a.D == 512 && a.o_tok) {
         hipLaunchKernelGGL((attn_combine_tok<T>), dim3((unsigned)a.tail * 32u), dim3(256), 0, s, c);
         return hipGetLastError();
     }
@@ -2645,17 +2688,49 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
                   int Skv, int D, float scale, hipStream_t stream, int dtype,
                   const long long* q_strides, const long long* k_strides,
                   const long long* v_strides, const long long* o_strides, void* workspace,
-                  size_t workspace_bytes, bool use_scratch = false) {
+                  size_t workspace_bytes, bool use_scratch = false, void* copies = nullptr,
+                  size_t copies_bytes = 0) {
     g_err[0] = 0;
     auto pick = [](const long long* p, Strides dflt) {
         return p ? Strides{p[0], p[1], p[2], p[3]} : dflt;
     };
-    const Strides sq = pick(q_strides, contiguous(H, Sq, D));
-    const Strides sk = pick(k_strides, contiguous(H, Skv, D));
-    const Strides sv = pick(v_strides, contiguous(H, Skv, D));
+    Strides sq = pick(q_strides, contiguous(H, Sq, D));
+    Strides sk = pick(k_strides, contiguous(H, Skv, D));
+    Strides sv = pick(v_strides, contiguous(H, Skv, D));
     const Strides so = pick(o_strides, contiguous(H, Sq, D));
     if (check_args(q, k, v, o, B, H, Sq, Skv, D, dtype, sq, sk, sv, so)) return 1;
     if (B == 0 || H == 0 || Sq == 0) return 0;
+    const auto tokens16 = [&](const Strides& s, const void* p) {  // 16-byte runs of tokens
+        return s.s == 1 && s.d != 1 && s.b % 8 == 0 && s.h % 8 == 0 && s.d % 8 == 0 &&
+               (uintptr_t)p % 16 == 0;
+    };
+    const bool o_tok = tokens16(so, o);
+    TokCopyArgs tc;
+    if (copies) {  // (copies are made after every check, before the kernel's launch)
+        if (!token_contiguous(sk, sv, D) || !tokens16(sq, q) || Sq % 8 || !o_tok || Skv == 0)
+            return fail("attn: row copies need token-contiguous q, k, v and o, D = 512 and query "
+                        "and key counts that are multiples of 8");
+        if (copies_bytes < attn_row_copies_bytes(B, H, Sq, Skv, D) || (uintptr_t)copies % 16)
+            return fail("attn: row copies buffer misaligned or smaller than "
+                        "attn_row_copies_bytes()");
+        char* c = (char*)copies;
+        const void* in[3] = {q, k, v};
+        const Strides st[3] = {sq, sk, sv};
+        for (int n = 0; n < 3; ++n) {
+            tc.src[n] = in[n];
+            tc.dst[n] = c;
+            tc.st[n] = st[n];
+            tc.S[n] = n == 0 ? Sq : Skv;
+            c += (size_t)B * H * tc.S[n] * D * 2;
+        }
+        tc.H = H;
+        tc.BH = B * H;
+        q = tc.dst[0];
+        k = tc.dst[1];
+        v = tc.dst[2];
+        sq = contiguous(H, Sq, D);
+        sk = sv = contiguous(H, Skv, D);
+    }
     KArgs a;
     a.q = q;
     a.k = k;
@@ -2681,10 +2756,8 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     a.ws_ml = nullptr;
     a.o16 = (uintptr_t)o % 16 == 0 && so.b % 8 == 0 && so.h % 8 == 0 && so.s % 8 == 0 && so.d == 1;
     a.q_lds = sq.s <= (1LL << 24) && Skv > (D == 128 ? 256 : 1024);
-    a.q_tok = sq.s == 1 && sq.d != 1 && sq.b % 8 == 0 && sq.h % 8 == 0 && sq.d % 8 == 0 &&
-              (uintptr_t)q % 16 == 0 && Sq % 8 == 0 && (long long)(D - 1) * sq.d + Sq < (1LL << 30);
-    a.o_tok = so.s == 1 && so.d != 1 && so.b % 8 == 0 && so.h % 8 == 0 && so.d % 8 == 0 &&
-              (uintptr_t)o % 16 == 0;
+    a.q_tok = tokens16(sq, q) && Sq % 8 == 0 && (long long)(D - 1) * sq.d + Sq < (1LL << 30);
+    a.o_tok = o_tok;
     a.ncu = cu_count();
     a.whole = 0;
     a.tail = 0;
@@ -2692,7 +2765,7 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     a.tail_rows = (long long)B * H * Sq;
     const bool tl = token_contiguous(sk, sv, D);
     // Split the keys if it pays and the call may.
-    const SplitPlan ring = plan_split(B, H, Sq, Skv, D, D != 512 || tl || d512_wide(),
+    const SplitPlan ring = plan_split(B, H, Sq, Skv, D, D != 512 || tl || o_tok || d512_wide(),
                                       use_scratch ? kScratchBytes : (size_t)-1);
     SplitPlan p = workspace_bytes != (size_t)-1 ? ring : kNoSplit;
     size_t need = split_ws_bytes(p, B, H, Sq, D);
@@ -2750,6 +2823,13 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
         a.tail = B * H * ((Sq + rp.rows - 1) / rp.rows);
         a.ws_ml = a.ws_o + (size_t)rp.nsplit * a.tail_rows * D;
     }
+    if (copies) {
+        const dim3 grid((unsigned)((std::max(Sq, Skv) + 63) / 64), 8, 3u * (unsigned)a.BH);
+        if (dtype == ATTN_DTYPE_BF16)
+            hipLaunchKernelGGL((tok_to_rows<bf16>), grid, dim3(256), 0, stream, tc);
+        else
+            hipLaunchKernelGGL((tok_to_rows<f16>), grid, dim3(256), 0, stream, tc);
+    }
     hipError_t e = dtype == ATTN_DTYPE_BF16 ? launch_t<bf16>(a, tl, rp.rows, stream)
                                             : launch_t<f16>(a, tl, rp.rows, stream);
     if (e == hipSuccess) e = scratch.release(stream);
@@ -2786,6 +2866,27 @@ extern "C" int attn_fwd_split(const void* q, const void* k, const void* v, void*
     if (workspace_bytes == (size_t)-1) workspace_bytes -= 1;
     return attn_fwd_impl(q, k, v, o, B, H, Sq, Skv, D, scale, stream, dtype, q_strides, k_strides,
                          v_strides, o_strides, workspace, workspace_bytes);
+}
+
+extern "C" size_t attn_row_copies_bytes(int B, int H, int Sq, int Skv, int D) {
+    if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || D != 512) return 0;
+    return (size_t)B * H * ((size_t)Sq + 2 * (size_t)Skv) * D * 2;
+}
+
+extern "C" int attn_fwd_split_copied(const void* q, const void* k, const void* v, void* o, int B,
+                                     int H, int Sq, int Skv, int D, float scale,
+                                     hipStream_t stream, int dtype, const long long* q_strides,
+                                     const long long* k_strides, const long long* v_strides,
+                                     const long long* o_strides, void* workspace,
+                                     size_t workspace_bytes, void* copies, size_t copies_bytes) {
+    if (workspace_bytes == (size_t)-1) workspace_bytes -= 1;
+    if (!copies) {
+        set_err("attn: row copies buffer missing");
+        return 1;
+    }
+    return attn_fwd_impl(q, k, v, o, B, H, Sq, Skv, D, scale, stream, dtype, q_strides, k_strides,
+                         v_strides, o_strides, workspace, workspace_bytes, false, copies,
+                         copies_bytes);
 }
 
 extern "C" size_t attn_split_scratch_capacity(void) { return kScratchBytes; }

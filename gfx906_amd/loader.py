@@ -76,6 +76,11 @@ def capi() -> ctypes.CDLL:
     lib.attn_split_workspace_bytes.restype = ctypes.c_size_t
     lib.attn_fwd_split_static.argtypes = lib.attn_fwd_ex.argtypes
     lib.attn_fwd_split_static.restype = ctypes.c_int
+    lib.attn_row_copies_bytes.argtypes = [ctypes.c_int] * 5
+    lib.attn_row_copies_bytes.restype = ctypes.c_size_t
+    lib.attn_fwd_split_copied.argtypes = lib.attn_fwd_split.argtypes + [ctypes.c_void_p,
+                                                                        ctypes.c_size_t]
+    lib.attn_fwd_split_copied.restype = ctypes.c_int
     lib.attn_split_scratch_capacity.argtypes = []
     lib.attn_split_scratch_capacity.restype = ctypes.c_size_t
     lib.attn_last_error.argtypes = []
