@@ -473,6 +473,7 @@ struct Cfg {
     static_assert(BLKS % NW == 0, "tile must split evenly over waves");
     static_assert(DP % 32 == 0 && DP <= 128, "head-dim class");
     static constexpr bool TAIL = false;
+    static constexpr int DU = DP;  // dims computed with (a multiple of 16)
 };
 // SPLIT kernels for a grid whose first units run unsplit (KArgs::whole > 0).
 // Instantiations of their own: the second epilogue and the arguments read
@@ -480,6 +481,14 @@ struct Cfg {
 template <int DP_, int NW_, int OCC_>
 struct CfgTail : Cfg<DP_, NW_, OCC_> {
     static constexpr bool TAIL = true;
+};
+// Head dims up to 48 in the 64-dim tiles: QK^T over DU dims rounded up to 32
+// and PV over DU (32 or 48), instead of 64 of both (tiles and loads are the
+// padded 64-dim ones, which cost nothing beside them).
+template <int DU_, bool TAIL_>
+struct CfgDims : Cfg<64, 8, 2> {
+    static constexpr bool TAIL = TAIL_;
+    static constexpr int DU = DU_;
 };
 
 // Per-lane byte offsets of the direct HBM->LDS tile loads. Each wave fills
@@ -581,8 +590,8 @@ attn_fwd_pipe(const KArgs a) {
     using E = Elem<T>;
     using x8 = typename E::x8;
     constexpr int DP = C::DP, NU = C::NU, RB = C::RB, TILE = C::TILE;
-    constexpr int NQF = DP / 32;          // Q fragments (32 dims each) per column block
-    constexpr int NOB = DP / 16;          // 16-dim output blocks
+    constexpr int NQF = (C::DU + 31) / 32;  // Q fragments (32 dims each) per column block
+    constexpr int NOB = C::DU / 16;         // 16-dim output blocks
     constexpr int LPT = C::BLKS / C::NW;  // loads per wave per K (or V) tile
     static_assert(2 * LPT < 16, "vmcnt immediate");
     constexpr int kWaitNext = 0x0F70 | (2 * LPT);  // vmcnt(one tile of loads)
@@ -783,7 +792,7 @@ attn_fwd_pipe(const KArgs a) {
             // The first A reads go out while the last kPvTail MFMAs of the
             // PV step before are still to issue (see pv).
             {
-                constexpr int A = DP == 64 ? 3 : 2;
+                constexpr int A = DP != 64 ? 2 : NQF == 1 ? 2 : 3;
                 __builtin_amdgcn_sched_group_barrier(kSgDsRead, A, 0);
                 if constexpr (kPvTail > 0) __builtin_amdgcn_sched_group_barrier(kSgMfma, kPvTail, 0);
 #pragma unroll
@@ -811,7 +820,7 @@ attn_fwd_pipe(const KArgs a) {
             // by a QK^T step, whose first K reads are placed ahead of this
             // step's last kPvTail MFMAs (D = 128: +1.2 % north star and c2
             // with 4 or 6, -5 % with 8, which also holds back QK^T MFMAs).
-            constexpr int kVAhead = DP == 128 ? 4 : 3;  // V fragments, two reads each
+            constexpr int kVAhead = DP == 128 ? 4 : NOB < 3 ? NOB : 3;  // V fragments, two reads each
             __builtin_amdgcn_sched_group_barrier(kSgDsRead, 2 * kVAhead, 0);
 #pragma unroll
             for (int n = 0; n < NOB - kVAhead; ++n) {
@@ -2242,6 +2251,15 @@ bool tile_max(int keys) {
     return keys <= kTileMaxKeys;
 }
 
+// The ring kernel for D < 64.
+template <class C, class T, bool SPLIT>
+void launch_narrow(const KArgs& a, bool tm, dim3 grid, hipStream_t s) {
+    if (tm)
+        hipLaunchKernelGGL((attn_fwd_pipe<C, true, T, SPLIT, true>), grid, dim3(C::NT), 0, s, a);
+    else
+        hipLaunchKernelGGL((attn_fwd_pipe<C, true, T, SPLIT, false>), grid, dim3(C::NT), 0, s, a);
+}
+
 // The ring kernels' whole units and split tail.
 template <class T>
 void launch_tail(const KArgs& a, dim3 grid, hipStream_t s) {
@@ -2255,10 +2273,12 @@ void launch_tail(const KArgs& a, dim3 grid, hipStream_t s) {
         hipLaunchKernelGGL((attn_fwd_pipe<C64, false, T, true, true>), grid, dim3(C64::NT), 0, s, a);
     else if (a.D == 64)
         hipLaunchKernelGGL((attn_fwd_pipe<C64, false, T, true, false>), grid, dim3(C64::NT), 0, s, a);
-    else if (tm)
-        hipLaunchKernelGGL((attn_fwd_pipe<C64, true, T, true, true>), grid, dim3(C64::NT), 0, s, a);
+    else if (a.D <= 32)
+        launch_narrow<CfgDims<32, true>, T, true>(a, tm, grid, s);
+    else if (a.D <= 48)
+        launch_narrow<CfgDims<48, true>, T, true>(a, tm, grid, s);
     else
-        hipLaunchKernelGGL((attn_fwd_pipe<C64, true, T, true, false>), grid, dim3(C64::NT), 0, s, a);
+        launch_narrow<C64, T, true>(a, tm, grid, s);
 }
 
 template <class T, bool SPLIT>
@@ -2296,12 +2316,12 @@ void launch_kernel(const KArgs& a, bool tl, hipStream_t s) {
         else if (D == 64)
             hipLaunchKernelGGL((attn_fwd_pipe<Cfg64, false, T, SPLIT, false>), grid,
                                dim3(Cfg64::NT), 0, s, a);
-        else if (tm)
-            hipLaunchKernelGGL((attn_fwd_pipe<Cfg64, true, T, SPLIT, true>), grid, dim3(Cfg64::NT),
-                               0, s, a);
+        else if (D <= 32)
+            launch_narrow<CfgDims<32, false>, T, SPLIT>(a, tm, grid, s);
+        else if (D <= 48)
+            launch_narrow<CfgDims<48, false>, T, SPLIT>(a, tm, grid, s);
         else
-            hipLaunchKernelGGL((attn_fwd_pipe<Cfg64, true, T, SPLIT, false>), grid, dim3(Cfg64::NT),
-                               0, s, a);
+            launch_narrow<Cfg64, T, SPLIT>(a, tm, grid, s);
     }
 }
 

@@ -158,15 +158,18 @@ def test_conv3d_kernels_do_not_spill(conv_asm):
 
 
 def test_tail_kernels_keep_occupancy_without_spills(kernel_asm):
-    """The instantiations for whole units and a split tail (two epilogues)."""
+    """The instantiations for whole units and a split tail (two epilogues), and
+    for head dims up to 32 and 48."""
     seen = []
     for m in RESOURCES.finditer(kernel_asm):
         name, vgprs, scratch, occ = m.group(1), int(m.group(2)), int(m.group(3)), int(m.group(4))
-        if "7CfgTail" in name:
+        if "7CfgTail" in name or "7CfgDims" in name:
             want = 2 if "7CfgTailILi128" in name else 4
             seen.append(name)
             assert occ >= want and vgprs <= 512 // want and scratch == 0, (name, vgprs, scratch)
-    assert len(seen) == 10, seen  # D = 128, and 64 and padded with and without the tile max
+    # tail: D = 128, and 64 and padded with and without the tile max; narrow: two
+    # head-dim classes x (unsplit, split, tail) x tile max; fp16 and bf16
+    assert len(seen) == 10 + 24, seen
 
 
 def test_conv3d_split_and_wide_kernels_do_not_spill(conv_asm):
