@@ -77,13 +77,10 @@ bool token_contiguous_kv(const torch::Tensor& t) {
     return (D - 1) * s[3] + S < (int64_t(1) << 30);
 }
 
-// Whether t's tokens lie in 16-byte aligned runs: sequence stride 1, the
-// other strides multiples of 8 (the head dim's other than 1).
+// Whether t is token-contiguous, whatever its other strides and alignment.
 bool token_runs(const torch::Tensor& t) {
     const auto s = strides4(t);
-    return t.stride(2) == 1 && s[3] != 1 && s[3] % 8 == 0 && s[0] >= 0 && s[1] >= 0 &&
-           s[0] % 8 == 0 && s[1] % 8 == 0 && s[3] > 0 &&
-           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+    return t.stride(2) == 1 && s[3] > 1 && s[0] >= 0 && s[1] >= 0;
 }
 
 // Largest Skv for which reading token-contiguous k/v in place beats copying
@@ -127,15 +124,15 @@ torch::Tensor attn(torch::Tensor q, torch::Tensor k, torch::Tensor v, double sca
         o = torch::empty({B, H, Sq, D}, q.options().memory_format(at::MemoryFormat::Contiguous));
     }
     if (o.numel() == 0) return o;
-    // Token-contiguous k and v (D = 512): read in place up to kInPlaceMaxSkv,
-    // q and out with any strides; above, with q and out of the same kind, the
-    // library makes row copies. Otherwise the head dim of every
+    // Token-contiguous k and v (D = 512): read in place up to kInPlaceMaxSkv
+    // where aligned, q and out with any strides; otherwise, with q and out of
+    // the same kind, the library makes row copies. Otherwise the head dim of every
     // tensor the kernel touches is contiguous: inputs are copied and out
     // staged as needed.
-    const bool tokens = token_contiguous_kv(k) && token_contiguous_kv(v) && Skv > 0;
-    const bool copied = tokens && Skv > kInPlaceMaxSkv && token_runs(q) && Sq % 8 == 0 &&
-                        token_runs(o) && B * H * 3 <= 65535;  // (the copies' grid)
-    const bool tl = tokens && (Skv <= kInPlaceMaxSkv || copied);
+    const bool in_place = Skv <= kInPlaceMaxSkv && token_contiguous_kv(k) && token_contiguous_kv(v);
+    const bool copied = !in_place && D == 512 && Skv > 0 && token_runs(q) && token_runs(k) &&
+                        token_runs(v) && token_runs(o) && B * H * 3 <= 65535;
+    const bool tl = in_place || copied;
     const auto qi = tl ? q : as_input(q, false);
     const auto ki = tl ? k : as_input(k, true), vi = tl ? v : as_input(v, true);
     const bool staged = !tl && o.stride(3) != 1;

@@ -133,10 +133,11 @@ struct KArgs {
     // where before the prefetch the two extra barriers cost more than the
     // gathered global loads).
     int q_lds;
-    // Token-contiguous D = 512 layout: q (o) is token-contiguous as well, with
-    // 16-byte aligned rows and (q) whole 8-token chunks, like K's, and a
-    // per-head span below 2^31 bytes.
-    int q_tok, o_tok;
+    // Token-contiguous D = 512 layout: q is token-contiguous as well, with
+    // 16-byte aligned rows and whole 8-token chunks, like K's, and a per-head
+    // span below 2^31 bytes; o is token-contiguous (o_tok), with 16-byte
+    // aligned rows (o_vec).
+    int q_tok, o_tok, o_vec;
     // Compute units of the device: with the kernel's workgroups per CU, how
     // many workgroups are resident at once (the D = 128 ring kernel and the
     // D <= 64 one with the tile max prefetch the Q tile of the workgroup that
@@ -2015,6 +2016,8 @@ static_assert(Cfg512W::BM == Cfg512::BM, "same query tiling as attn_fwd_d512 (gr
 // dims of one token per lane) so that loads and stores both move 16 bytes per
 // lane in 64- and 128-byte runs. q, k and v in one launch; bound by memory
 // (14,400 bf16 tokens: 88 MB; torch's copies took 31 us a tensor).
+// VEC: rows of 16-byte aligned 8-token chunks; otherwise any alignment and
+// token count, loaded element by element along the tokens.
 struct TokCopyArgs {
     const void* src[3];
     void* dst[3];
@@ -2023,7 +2026,7 @@ struct TokCopyArgs {
     int H, BH;
 };
 // grid: (ceil(max S / 64), 8, 3 * B*H); block: 256 threads.
-template <class T>
+template <class T, bool VEC>
 __global__ void __launch_bounds__(256) tok_to_rows(const TokCopyArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using x8 = typename Elem<T>::x8;
@@ -2035,11 +2038,22 @@ __global__ void __launch_bounds__(256) tok_to_rows(const TokCopyArgs a) {
     const int b = bh / a.H, h = bh - b * a.H, tid = threadIdx.x;
     const Strides st = a.st[n];
     const T* src = (const T*)a.src[n] + b * st.b + h * st.h + dim0 * st.d + tok0;
+    if constexpr (VEC) {
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        const int d = (tid >> 3) + 32 * p, t = (tid & 7) * 8;
-        if (tok0 + t < S)  // (S is a multiple of 8)
-            *reinterpret_cast<x8*>(tile + d * RB + t * 2) = ld_global16(src + d * st.d + t);
+        for (int p = 0; p < 2; ++p) {
+            const int d = (tid >> 3) + 32 * p, t = (tid & 7) * 8;
+            if (tok0 + t < S)  // (S is a multiple of 8)
+                *reinterpret_cast<x8*>(tile + d * RB + t * 2) = ld_global16(src + d * st.d + t);
+        }
+    } else {
+        const int t = tid & 63;
+        T val[16];
+#pragma unroll
+        for (int p = 0; p < 16; ++p)
+            val[p] = tok0 + t < S ? src[((tid >> 6) + 4 * p) * st.d + t] : (T)0.0f;
+#pragma unroll
+        for (int p = 0; p < 16; ++p)
+            *reinterpret_cast<T*>(tile + ((tid >> 6) + 4 * p) * RB + t * 2) = val[p];
     }
     __syncthreads();
     const int lane = tid & 63, i = lane & 15, g = lane >> 4, tw = (tid >> 6) * 16;
@@ -2067,7 +2081,7 @@ struct CombArgs {
     const float* ws_ml;
     void* o;
     Strides so;
-    int H, Sq, D, nsplit, whole;
+    int H, Sq, D, nsplit, whole, o_vec;
     long long row0, rows;  // the split rows: [row0, row0 + rows) of all heads' rows
 };
 
@@ -2172,13 +2186,19 @@ __global__ void __launch_bounds__(256) attn_combine_tok(const CombArgs c) {
     }
     __syncthreads();
     const int b = bh / c.H, h = bh - b * c.H;
-    const int d = tid >> 3, r = (tid & 7) * 8, tok = tok0 + r;
-    T* op = (T*)c.o + b * c.so.b + h * c.so.h + (dim0 + d) * c.so.d + tok;
-    const T* src = tile + d * ST + r;
-    if (tok + 8 <= c.Sq)
-        *reinterpret_cast<u32x4*>(op) = *reinterpret_cast<const u32x4*>(src);
-    else
-        for (int e = 0; e < 8 && tok + e < c.Sq; ++e) op[e] = src[e];
+    T* const oh = (T*)c.o + b * c.so.b + h * c.so.h + dim0 * c.so.d + tok0;
+    if (c.o_vec && tok0 + 64 <= c.Sq) {
+        const int d = tid >> 3, r = (tid & 7) * 8;
+        *reinterpret_cast<u32x4*>(oh + d * c.so.d + r) =
+            *reinterpret_cast<const u32x4*>(tile + d * ST + r);
+    } else {  // a wave per dim, 64 tokens
+        const int r = tid & 63;
+#pragma unroll
+        for (int p = 0; p < 8; ++p) {
+            const int d = (tid >> 6) + 4 * p;
+            if (tok0 + r < c.Sq) oh[d * c.so.d + r] = tile[d * ST + r];
+        }
+    }
 #endif
 }
 
@@ -2289,7 +2309,7 @@ void launch_kernel(const KArgs& a, bool tl, hipStream_t s) {
     if (D == 512) {
         if (tl)
             hipLaunchKernelGGL((attn_fwd_tok512<T, SPLIT>), grid, dim3(Cfg512W::NT), 0, s, a);
-        else if (d512_wide() || a.o_tok)  // (only the wide kernel stores tokens)
+        else if (d512_wide() || a.o_tok)  // (only the wide kernel stores by tokens)
             hipLaunchKernelGGL((attn_fwd_d512w<T, SPLIT>), grid, dim3(Cfg512W::NT), 0, s, a);
         else
             hipLaunchKernelGGL((attn_fwd_d512<T, SPLIT>), grid, dim3(Cfg512::NT), 0, s, a);
@@ -2368,6 +2388,7 @@ hipError_t launch_t(const KArgs& a, bool tl, int rows, hipStream_t s) {
     c.D = a.D;
     c.nsplit = a.nsplit;
     c.whole = a.whole;
+    c.o_vec = a.o_vec;
     c.row0 = a.row0;
     c.rows = a.tail_rows;
     if (a.D == 512 && a.o_tok) {
@@ -2718,24 +2739,34 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     Strides sk = pick(k_strides, contiguous(H, Skv, D));
     Strides sv = pick(v_strides, contiguous(H, Skv, D));
     const Strides so = pick(o_strides, contiguous(H, Sq, D));
-    if (check_args(q, k, v, o, B, H, Sq, Skv, D, dtype, sq, sk, sv, so)) return 1;
-    if (B == 0 || H == 0 || Sq == 0) return 0;
-    const auto tokens16 = [&](const Strides& s, const void* p) {  // 16-byte runs of tokens
+    // Whether tokens lie in 16-byte aligned runs.
+    const auto tokens16 = [&](const Strides& s, const void* p) {
         return s.s == 1 && s.d != 1 && s.b % 8 == 0 && s.h % 8 == 0 && s.d % 8 == 0 &&
                (uintptr_t)p % 16 == 0;
     };
-    const bool o_tok = tokens16(so, o);
     TokCopyArgs tc;
-    if (copies) {  // (copies are made after every check, before the kernel's launch)
-        if (!token_contiguous(sk, sv, D) || !tokens16(sq, q) || Sq % 8 || !o_tok || Skv == 0)
-            return fail("attn: row copies need token-contiguous q, k, v and o, D = 512 and query "
-                        "and key counts that are multiples of 8");
+    bool copy_vec = false;
+    if (copies) {  // (made after every check, just before the kernel's launch)
+        const Strides st[3] = {sq, sk, sv};
+        const Strides* all[4] = {&sq, &sk, &sv, &so};
+        for (const Strides* s : all) {
+            if (s->b < 0 || s->h < 0 || s->s < 0 || s->d < 0)
+                return fail("attn: strides must be non-negative");
+            if (D != 512 || s->s != 1 || s->d == 1)
+                return fail("attn: row copies need token-contiguous q, k, v and o and D = 512");
+        }
+        if (Sq <= 0 || Skv <= 0 || !q || !k || !v || !o ||
+            ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o) % 2)
+            return fail("attn: row copies need queries, keys and element-aligned tensors");
         if (copies_bytes < attn_row_copies_bytes(B, H, Sq, Skv, D) || (uintptr_t)copies % 16)
             return fail("attn: row copies buffer misaligned or smaller than "
                         "attn_row_copies_bytes()");
+        if ((long long)B * H * 3 > 65535) return fail("attn: too many heads for row copies");
+        if (output_overlaps(so, B, H, Sq, D)) return fail("attn: o strides make output rows overlap");
+        copy_vec = tokens16(sq, q) && tokens16(sk, k) && tokens16(sv, v) && Sq % 8 == 0 &&
+                   Skv % 8 == 0;
         char* c = (char*)copies;
         const void* in[3] = {q, k, v};
-        const Strides st[3] = {sq, sk, sv};
         for (int n = 0; n < 3; ++n) {
             tc.src[n] = in[n];
             tc.dst[n] = c;
@@ -2750,7 +2781,13 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
         v = tc.dst[2];
         sq = contiguous(H, Sq, D);
         sk = sv = contiguous(H, Skv, D);
+        // (o's layout is checked above; the rest as for contiguous tensors)
+        if (check_args(q, k, v, copies, B, H, Sq, Skv, D, dtype, sq, sk, sv, sq)) return 1;
+    } else if (check_args(q, k, v, o, B, H, Sq, Skv, D, dtype, sq, sk, sv, so)) {
+        return 1;
     }
+    if (B == 0 || H == 0 || Sq == 0) return 0;
+    const bool o_tok = D == 512 && so.s == 1 && so.d != 1;
     KArgs a;
     a.q = q;
     a.k = k;
@@ -2778,6 +2815,7 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     a.q_lds = sq.s <= (1LL << 24) && Skv > (D == 128 ? 256 : 1024);
     a.q_tok = tokens16(sq, q) && Sq % 8 == 0 && (long long)(D - 1) * sq.d + Sq < (1LL << 30);
     a.o_tok = o_tok;
+    a.o_vec = tokens16(so, o);
     a.ncu = cu_count();
     a.whole = 0;
     a.tail = 0;
@@ -2785,7 +2823,7 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     a.tail_rows = (long long)B * H * Sq;
     const bool tl = token_contiguous(sk, sv, D);
     // Split the keys if it pays and the call may.
-    const SplitPlan ring = plan_split(B, H, Sq, Skv, D, D != 512 || tl || o_tok || d512_wide(),
+    const SplitPlan ring = plan_split(B, H, Sq, Skv, D, D != 512 || tl || copies || d512_wide(),
                                       use_scratch ? kScratchBytes : (size_t)-1);
     SplitPlan p = workspace_bytes != (size_t)-1 ? ring : kNoSplit;
     size_t need = split_ws_bytes(p, B, H, Sq, D);
@@ -2845,10 +2883,11 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     }
     if (copies) {
         const dim3 grid((unsigned)((std::max(Sq, Skv) + 63) / 64), 8, 3u * (unsigned)a.BH);
-        if (dtype == ATTN_DTYPE_BF16)
-            hipLaunchKernelGGL((tok_to_rows<bf16>), grid, dim3(256), 0, stream, tc);
+        // (16-bit elements move the same whatever their type)
+        if (copy_vec)
+            hipLaunchKernelGGL((tok_to_rows<f16, true>), grid, dim3(256), 0, stream, tc);
         else
-            hipLaunchKernelGGL((tok_to_rows<f16>), grid, dim3(256), 0, stream, tc);
+            hipLaunchKernelGGL((tok_to_rows<f16, false>), grid, dim3(256), 0, stream, tc);
     }
     hipError_t e = dtype == ATTN_DTYPE_BF16 ? launch_t<bf16>(a, tl, rp.rows, stream)
                                             : launch_t<f16>(a, tl, rp.rows, stream);

@@ -113,11 +113,12 @@ int attn_fwd_split_static(const void* q, const void* k, const void* v, void* o,
                           const long long* v_strides, const long long* o_strides);
 
 /* attn_fwd_split() on row copies of token-contiguous q, k and v (D = 512, o
- * token-contiguous too, 16-byte aligned with strides that are multiples of 8,
- * Sq % 8 == Skv % 8 == 0): the tensors are first transposed into `copies`
- * (16-byte aligned, attn_row_copies_bytes() bytes, one launch) and the
- * row-contiguous kernel runs on those, which is faster than reading them in
- * place from about 7000 tokens. No counterpart in the reference. */
+ * token-contiguous too; any other strides, alignment and counts): the tensors
+ * are first transposed into `copies` (16-byte aligned,
+ * attn_row_copies_bytes() bytes, one launch) and the row-contiguous kernel
+ * runs on those. For layouts that attn_fwd_split() does not read in place,
+ * and faster than reading in place from about 7000 tokens. No counterpart in
+ * the reference. */
 size_t attn_row_copies_bytes(int B, int H, int Sq, int Skv, int D);
 int attn_fwd_split_copied(const void* q, const void* k, const void* v, void* o, int B, int H,
                           int Sq, int Skv, int D, float scale, hipStream_t stream, int dtype,

@@ -87,7 +87,9 @@ def test_tok512_whole_units_and_a_split_tail(monkeypatch):
 @pytest.mark.parametrize("nsplit", [1, 3, None])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B,H,Sq,Skv", [(1, 1, 8, 8), (2, 1, 56, 72), (1, 2, 64, 128),
-                                        (1, 1, 136, 200), (2, 2, 264, 1032), (1, 65, 504, 1032)])
+                                        (1, 1, 136, 200), (2, 2, 264, 1032), (1, 65, 504, 1032),
+                                        (1, 1, 1, 1), (2, 1, 33, 65), (1, 2, 127, 300),
+                                        (2, 1, 250, 515), (1, 65, 500, 1035)])
 def test_row_copies(monkeypatch, B, H, Sq, Skv, dtype, nsplit, wide):
     """attn_fwd_split_copied: the row-contiguous kernel's bits, stored by tokens
     (also with GFX906_AMD_ATTN_D512W=0, whose kernel stores rows only)."""
@@ -99,8 +101,9 @@ def test_row_copies(monkeypatch, B, H, Sq, Skv, dtype, nsplit, wide):
     ref = gfx906_amd.attn(q, k, v, 0.04)
     if wide:
         monkeypatch.setenv("GFX906_AMD_ATTN_D512W", wide)
-    (_, qt), (_, kt), (_, vt) = tokens(q), tokens(k, 8), tokens(v)
-    obuf, o = tokens(torch.zeros_like(q), 16)
+    odd = 0 if Sq % 8 == 0 else 1  # odd counts: rows of any alignment
+    (_, qt), (_, kt), (_, vt) = tokens(q, odd), tokens(k, 8), tokens(v, 3 * odd)
+    obuf, o = tokens(torch.zeros_like(q), 16 - odd)
     lib = gfx906_amd.capi()
     # (the plan without the override, whose own kernel runs no split tail)
     need = max(lib.attn_split_workspace_bytes(B, H, Sq, Skv, 512), 64 << 20)
@@ -135,8 +138,9 @@ def test_row_copies_rejects():
     for kw, msg in ((dict(copies=None), b"missing"), (dict(nbytes=n - 1), b"smaller"),
                     (dict(copies=ctypes.c_void_p(0x10008)), b"misaligned"),
                     (dict(q=rows), b"token-contiguous"), (dict(o=rows), b"token-contiguous"),
-                    (dict(k=rows, v=rows), b"head dim"), (dict(sq=63), b"multiples of 8"),
-                    (dict(skv=0), b"token-contiguous"), (dict(d=64), b"head dim")):
+                    (dict(k=rows, v=rows), b"token-contiguous"), (dict(skv=0), b"need queries"),
+                    (dict(d=64), b"token-contiguous"),
+                    (dict(o=(ctypes.c_longlong * 4)(64, 64, 1, 2)), b"overlap")):
         rc, err = call(**kw)
         assert rc == 1 and msg in err, (kw, err)
     assert lib.attn_row_copies_bytes(1, 1, 64, 64, 128) == 0
