@@ -10,7 +10,8 @@
  * rounded to the element type; rows with Skv == 0 are written as zeros.
  * Calls are asynchronous on `stream`. The only state kept between calls is
  * the static scratch of the calls that split key ranges without a caller
- * workspace (launch(), attn_fwd(), attn_fwd_split_static()): a device array
+ * workspace (launch(), attn_fwd(), attn_fwd_split_static(), and conv3d_fwd()
+ * and launch_conv3d(), which split reductions in it): a device array
  * of attn_split_scratch_capacity() bytes that is part of the library's code
  * object, so it is held on every GPU where the library's kernels are loaded,
  * until the process ends. Those calls are ordered on the GPU across streams
@@ -36,8 +37,9 @@ extern "C" {
  * declared at attn.cpp:4-5, defined at attn_kernel.hip:710-742. Returns
  * nothing; on a rejected argument or launch failure no kernel runs and the
  * reason is available from attn_last_error(). When B*H*Sq is too small to
- * fill the GPU (a one-head VAE attention) it splits the key range as
- * attn_fwd_split_static() does, in the static scratch. */
+ * fill the GPU (a one-head VAE attention), or fills it a whole number of times
+ * and a little more, it splits key ranges as attn_fwd_split_static() does, in
+ * the static scratch. */
 void launch(const void* q, const void* k, const void* v, void* o,
             int B, int H, int Sq, int Skv, int D, float scale, hipStream_t stream);
 
@@ -50,7 +52,7 @@ int attn_fwd(const void* q, const void* k, const void* v, void* o,
 
 /* attn_fwd() for fp16 or bf16 (dtype = ATTN_DTYPE_F16 / ATTN_DTYPE_BF16,
  * the same type for q, k, v and o) and strided tensors, never splitting the
- * key range (one workgroup per batch, head and query tile). Each *_strides
+ * key range over workgroups. Each *_strides
  * points to four element strides {batch, head, sequence, head dim} of that
  * tensor, or is NULL for the contiguous layout. Strides are non-negative;
  * input strides may be 0 (a tensor broadcast over batch or heads) but no two
@@ -72,19 +74,22 @@ int attn_fwd_ex(const void* q, const void* k, const void* v, void* o,
                 int dtype, const long long* q_strides, const long long* k_strides,
                 const long long* v_strides, const long long* o_strides);
 
-/* Bytes of device workspace attn_fwd_split() needs for this problem on the
- * current device: 0 when the problem's workgroups already fill the GPU (the
- * call then runs as attn_fwd_ex()), else room for the partial results of the
- * split key ranges. No counterpart in the reference. */
+/* Bytes of device workspace attn_fwd_split() takes for this problem on the
+ * current device: 0 when no split pays (the call then runs as attn_fwd_ex()),
+ * else room for the partial results of the split key ranges: of every row
+ * when the problem's workgroups do not fill the GPU, of the last rows alone
+ * (at most 96 MiB) when they fill it a whole number of times and a little
+ * more. No counterpart in the reference. */
 size_t attn_split_workspace_bytes(int B, int H, int Sq, int Skv, int D);
 
 /* attn_fwd_ex() that, when B*H*Sq is too small to fill the GPU (a VAE
- * attention over one head, short problems), splits the key range over more
- * workgroups: each writes its unnormalised partial output and running
+ * attention over one head, short problems) or leaves its last round of
+ * workgroups nearly empty, splits key ranges over more workgroups: each writes its unnormalised partial output and running
  * max/sum to `workspace` (device memory, 16-byte aligned, at least
  * attn_split_workspace_bytes() bytes; may be NULL when that is 0) and a
  * second kernel merges them into o. Same arguments and return codes as
- * attn_fwd_ex(), plus 1 for a missing or short workspace. Results agree with
+ * attn_fwd_ex(), plus 1 for a missing or short workspace (problems that fill
+ * the GPU then run unsplit instead). Results agree with
  * attn_fwd_ex() to fp32 rounding of the merge (not bit for bit). Calls on one
  * workspace must not overlap. No counterpart in the reference. */
 int attn_fwd_split(const void* q, const void* k, const void* v, void* o,
@@ -104,7 +109,8 @@ int attn_fwd_split(const void* q, const void* k, const void* v, void* o,
  * otherwise. Problems that do not split use no scratch. Calls that use the
  * scratch are ordered across streams on one device (see the top of this
  * file); under stream capture the first such call on a device must have
- * been made outside capture (it sets the scratch up), else status 1. Same
+ * been made outside capture (it sets the scratch up), else status 1; problems
+ * that fill the GPU do not use the scratch under capture and run unsplit. Same
  * arguments and return codes as attn_fwd_split() otherwise. No counterpart
  * in the reference. */
 int attn_fwd_split_static(const void* q, const void* k, const void* v, void* o,
