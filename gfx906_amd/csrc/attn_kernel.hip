@@ -687,14 +687,19 @@ attn_fwd_pipe(const KArgs a) {
     // row is exactly 1.0 in fp16: with a stale max it carries a rounding
     // error of up to 2^-11 relative, which on sharp rows with |o| near 4 and
     // above (c3: q, k ~ 2 N(0,1), 512 keys) moves the output past the 2e-3
-    // bar.
+    // bar. Where key ranges are split it starts finite (its product with c
+    // must be), below every finite score that fp16 gives: a range may hold
+    // nothing but -inf scores (keys with infinite elements), which must give
+    // p = 0 and not exp2(-inf + inf).
     float m_run[2];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
 #pragma unroll
         for (int ob = 0; ob < NOB; ++ob) oacc[ob][nb] = f32x4{};
-        m_run[nb] = kLazy ? -1e30f : -INFINITY;
+        m_run[nb] = kLazy ? -1e30f : SPLIT ? -1e37f : -INFINITY;
     }
+    // 1 / l of a row whose scores are all -inf: NaN, as the -inf start gives.
+    constexpr float kNoKeyInv = SPLIT && !kLazy ? NAN : 0.f;
     f32x4 lacc[2] = {f32x4{}, f32x4{}};
     x8 aone;
 #pragma unroll
@@ -1133,7 +1138,7 @@ attn_fwd_pipe(const KArgs a) {
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
             const float l = quad_group_sum(lacc[nb][0]);
-            const float inv = l > 0.f ? 1.f / l : 0.f;
+            const float inv = l > 0.f ? 1.f / l : kNoKeyInv;
 #pragma unroll
             for (int ob = 0; ob < NOB; ++ob) {
                 const int d0 = 16 * ob + 4 * ge;
@@ -1167,7 +1172,7 @@ attn_fwd_pipe(const KArgs a) {
     for (int nb = 0; nb < 2; ++nb) {
         const int row = qrow0e + 16 * nb;
         const float l = quad_group_sum(lacc[nb][0]);
-        const float inv = l > 0.f ? 1.f / l : 0.f;
+        const float inv = l > 0.f ? 1.f / l : kNoKeyInv;
         if (row < Sqe) {
             T* op = Oe + row * ea.so.s;
 #pragma unroll
@@ -1534,10 +1539,14 @@ __global__ void __launch_bounds__((CfgRows<DP, NBQ>::NT), 2) attn_fwd_rows(const
         for (int ob = 0; ob < NOB; ++ob) vaddr[ob] = vrow * RB + (ob ^ vx) * 32 + (i & 3) * 8;
     }
     f32x4 oacc[NOB][NBQ];
-    float m_run[NBQ], l_run[NBQ];  // running max (score units), sum of this lane's keys
+    // Running max (score units) and -max * c, which stays 0 while every score
+    // of the row is -inf (keys with infinite elements), so that such keys give
+    // p = 0 also where they are all that a wave has seen; sum of this lane's keys.
+    float m_run[NBQ], nm[NBQ], l_run[NBQ];
 #pragma unroll
     for (int nb = 0; nb < NBQ; ++nb) {
         m_run[nb] = -INFINITY;
+        nm[nb] = 0.f;
         l_run[nb] = 0.f;
 #pragma unroll
         for (int ob = 0; ob < NOB; ++ob) oacc[ob][nb] = f32x4{};
@@ -1587,18 +1596,20 @@ __global__ void __launch_bounds__((CfgRows<DP, NBQ>::NT), 2) attn_fwd_rows(const
             }
             if (__any(mx > m_run[nb])) {
                 const float m_new = max2(m_run[nb], quad_group_max(mx));
-                const float alpha = __builtin_amdgcn_exp2f((m_run[nb] - m_new) * c);
+                const float ref = m_new == -INFINITY ? 0.f : m_new;
+                const float alpha = __builtin_amdgcn_exp2f((m_run[nb] - ref) * c);
                 if (st != wave) {  // (O and l are still zero on the wave's first step)
 #pragma unroll
                     for (int ob = 0; ob < NOB; ++ob) oacc[ob][nb] *= alpha;
                     l_run[nb] *= alpha;
                 }
                 m_run[nb] = m_new;
+                nm[nb] = -ref * c;
             }
 #pragma unroll
             for (int blk = 0; blk < NB32; ++blk)
-                block_exp<T, true>(S[2 * blk][nb], S[2 * blk + 1][nb], P[blk][nb], -m_run[nb] * c,
-                                   c, l_run[nb]);
+                block_exp<T, true>(S[2 * blk][nb], S[2 * blk + 1][nb], P[blk][nb], nm[nb], c,
+                                   l_run[nb]);
         }
         __builtin_amdgcn_s_waitcnt(0x0F70 | BLKS);  // V of this step landed; the next K may be
         asm volatile("" ::: "memory");              // in flight
@@ -1659,7 +1670,7 @@ __global__ void __launch_bounds__((CfgRows<DP, NBQ>::NT), 2) attn_fwd_rows(const
             *reinterpret_cast<f32x4*>(a.ws_o + o * D + 4 * u) = acc;
             if (u == 0) *reinterpret_cast<f32x2*>(a.ws_ml + 2 * o) = f32x2{mx, l};
         } else {
-            const float inv = l > 0.f ? 1.f / l : 0.f;
+            const float inv = l > 0.f ? 1.f / l : DP == 64 ? NAN : 0.f;
             const auto h0 = E::cvt2(acc[0] * inv, acc[1] * inv);
             const auto h1 = E::cvt2(acc[2] * inv, acc[3] * inv);
             T* op = (T*)a.o + b * a.so.b + h * a.so.h + row * a.so.s + 4 * u;
@@ -2121,7 +2132,8 @@ __device__ __forceinline__ f32x4 merge_row(const CombArgs& c, long long row, int
                 l += w * mlv[u][1];
             }
     }
-    return acc * (l > 0.f ? 1.f / l : 0.f);
+    // (l is 0 where every score is -inf; D <= 64 gives NaN there, split or not)
+    return acc * (l > 0.f ? 1.f / l : c.D <= 64 ? NAN : 0.f);
 }
 #endif
 

@@ -69,8 +69,8 @@ def test_layouts_give_the_same_bits(monkeypatch, D, rows):
 @pytest.mark.parametrize("rows", ["1", "1x64", "3"])
 @pytest.mark.parametrize("D", [40, 64, 128])
 def test_special_values(monkeypatch, D, rows):
-    """A NaN query reaches its own row, a NaN key or value every row; a key of
-    -inf scores (its rows' scores all -inf but one) keeps the others."""
+    """A NaN query reaches its own row, a NaN key or value every row; a step of
+    keys far below the others adds nothing."""
     monkeypatch.setenv("GFX906_AMD_ATTN_ROWS", rows)
     monkeypatch.setenv("GFX906_AMD_ATTN_NSPLIT", rows.split("x")[0])
     print(f"case rows {rows} special D{D}", flush=True)
@@ -89,6 +89,35 @@ def test_special_values(monkeypatch, D, rows):
     k[0, :, 64:128] = -60000.0  # a whole step of one wave far below the others
     got = gfx906_amd.attn(q.to(DEV), k.to(DEV), v.to(DEV), 0.1).float().cpu()
     assert (got - sdpa_math_fp32(q, k, v, 0.1)).abs().max() <= MAX_ABS_TOL
+
+
+@pytest.mark.parametrize("form", ["default", "rows1", "rows1x64", "rows3", "ring1", "ring4", "tail"])
+@pytest.mark.parametrize("D", [40, 64, 128])
+def test_infinite_keys(monkeypatch, D, form):
+    """Keys whose scores are all -inf weigh nothing, also where they are all
+    that a wave's first step, a whole key range or a split tail's range sees;
+    rows of nothing else are NaN (0 for D = 128)."""
+    if form.startswith("rows"):
+        monkeypatch.setenv("GFX906_AMD_ATTN_ROWS", form[4:])
+        monkeypatch.setenv("GFX906_AMD_ATTN_NSPLIT", form[4])
+    elif form.startswith("ring"):
+        monkeypatch.setenv("GFX906_AMD_ATTN_ROWS", "0")
+        monkeypatch.setenv("GFX906_AMD_ATTN_NSPLIT", form[4])
+    # (tail: 272 or 527 query tiles, a little past the workgroup slots)
+    H, Sq, Skv = (16, 4250, 1400) if D == 128 else (17, 7700, 1400)
+    if form != "tail":
+        H, Sq, Skv = 2, 70, 1100
+    print(f"case {form} infinite keys D{D}", flush=True)
+    q, k, v = make_inputs(1, H, Sq, Skv, D, 1.0, 1.0, 78)
+    q = q.abs() + 0.01  # a key of -inf then scores -inf in every row
+    keep = torch.zeros(Skv, dtype=torch.bool)
+    keep[:70] = keep[640:660] = True
+    k[:, :, ~keep] = float("-inf")
+    got = gfx906_amd.attn(q.to(DEV), k.to(DEV), v.to(DEV), 0.1)[:, -1:, -100:].cpu()
+    near(got, sdpa_math_fp32(q[:, -1:, -100:], k[:, -1:, keep], v[:, -1:, keep], 0.1), False, form)
+    k[...] = float("-inf")
+    got = gfx906_amd.attn(q.to(DEV), k.to(DEV), v.to(DEV), 0.1)
+    assert bool((got == 0).all() if D == 128 else got.isnan().all())
 
 
 def test_default_dispatch(monkeypatch):
