@@ -90,6 +90,9 @@ constexpr float kPLazyLimit = 32768.0f;
 // Lazy-rescale threshold of the D = 512 kernel: a tile whose largest p
 // exceeds 2^8 takes the exact max.
 constexpr float kPmaxLimit = 256.0f;
+// A buffer offset past every descriptor's range (each is below 2^31 bytes):
+// loads zeros.
+constexpr unsigned kOutOfRange = 0x80000000u;
 // sched_group_barrier instruction classes
 constexpr int kSgMfma = 0x008, kSgDsRead = 0x100;
 
@@ -376,11 +379,10 @@ __device__ __forceinline__ typename Elem<T>::x8 q_fragment(const T* p, bool load
 // Q rows of one workgroup through a range-checked buffer descriptor: the
 // loads are unconditional (no per-row branch, so the compiler does not merge
 // them with a zero value through copies that wait for the data), and rows
-// past `valid_rows` or offsets past the range (kQOutOfRange) read as zeros.
+// past `valid_rows` or offsets past the range (kOutOfRange) read as zeros.
 // The caller applies the sign of a negative scale later, once the prologue
 // waits for its loads anyway: an XOR right after the loads would hold back
 // every later load of the prologue behind them.
-constexpr unsigned kQOutOfRange = 0x80000000u;
 template <class T>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t q_rsrc(const T* row0, int valid_rows,
                                                         long long ss, int D) {
@@ -496,9 +498,10 @@ struct CfgDims : Cfg<64, 8, 2> {
 // whole 1 KB LDS blocks (lane i writes 16-byte unit i of its block) for
 // BLKS/NW blocks of each K tile and as many of each V tile. The offsets are
 // relative to the tile's first row (rows kss / vss elements apart in HBM)
-// and do not change from tile to tile. Units past D (padded head dims) are
-// pointed at unit 0 of the row: finite data that meets zero Q columns (K) or
-// feeds unused output columns (V).
+// and do not change from tile to tile. K units past D (padded head dims) are
+// pointed past the descriptor's range and load zeros: they meet zero Q columns,
+// and anything else could be infinite (inf * 0 is NaN). V units past D are
+// pointed at unit 0 of the row: they feed unused output columns only.
 template <class C, bool PAD>
 __device__ __forceinline__ void tile_offsets(int (&koff)[C::BLKS / C::NW],
                                              int (&voff)[C::BLKS / C::NW], int D, int kss,
@@ -507,9 +510,8 @@ __device__ __forceinline__ void tile_offsets(int (&koff)[C::BLKS / C::NW],
     for (int i = 0; i < C::BLKS / C::NW; ++i) {
         const int unit = (wave + i * C::NW) * 64 + lane;
         const int row = unit / C::NU, slot = unit % C::NU;
-        int ck = slot ^ kswz<C::NU>(row);
-        if (PAD && ck * 8 >= D) ck = 0;
-        koff[i] = (row * kss + ck * 8) * 2;
+        const int ck = slot ^ kswz<C::NU>(row);
+        koff[i] = PAD && ck * 8 >= D ? (int)kOutOfRange : (row * kss + ck * 8) * 2;
         int cv = slot ^ vswz<C::NU>(row);
         if (PAD && cv * 8 >= D) cv = 0;
         voff[i] = (row * vss + cv * 8) * 2;
@@ -648,7 +650,7 @@ attn_fwd_pipe(const KArgs a) {
                     const int d0 = 32 * s + 8 * g, r = wave * 32 + 16 * nb + i;
                     const unsigned off = r < qrows && (!PAD || d0 < D)
                                              ? (unsigned)((r * a.sq.s + d0) * 2)
-                                             : kQOutOfRange;
+                                             : kOutOfRange;
                     qf[nb][s] = q_load<T>(qr, off);
                 }
         } else {
@@ -1515,7 +1517,7 @@ __global__ void __launch_bounds__((CfgRows<DP, NBQ>::NT), 2) attn_fwd_rows(const
                 const int d0 = 32 * s + 8 * g, r = 16 * nb + i;
                 qf[nb][s] = q_load<T>(qr, r < rows && (!PAD || d0 < D)
                                               ? (unsigned)((r * a.sq.s + d0) * 2)
-                                              : kQOutOfRange);
+                                              : kOutOfRange);
             }
     } else {
 #pragma unroll
