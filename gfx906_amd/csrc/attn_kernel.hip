@@ -93,6 +93,10 @@ constexpr float kPmaxLimit = 256.0f;
 // A buffer offset past every descriptor's range (each is below 2^31 bytes):
 // loads zeros.
 constexpr unsigned kOutOfRange = 0x80000000u;
+// Running max (log2 units) of a row none of whose scores is above -inf: finite,
+// so that a score of -inf gives p = 0 and not exp2(-inf + inf), and below every
+// other score.
+constexpr float kNoMax = -3.0e38f;
 // sched_group_barrier instruction classes
 constexpr int kSgMfma = 0x008, kSgDsRead = 0x100;
 
@@ -1648,7 +1652,7 @@ __global__ void __launch_bounds__((CfgRows<DP, NBQ>::NT), 2) attn_fwd_rows(const
 #pragma unroll
     for (int n = 0; n < C::BM * OU / C::NT; ++n) {
         const int idx = n * C::NT + tid, r = idx / OU, u = idx - r * OU;
-        float mx = -3.0e38f;
+        float mx = kNoMax;
         f32x2 mlw[W];
 #pragma unroll
         for (int w = 0; w < W; ++w) {
@@ -1900,7 +1904,7 @@ attn_fwd_d512(const KArgs a) {
         }
         if (t == 0) {  // first tile: start from its exact max (O is still zero)
             float mx = fmaxf(max3(S[0][0], S[0][1], S[0][2]), max3(S[0][3], S[1][0], S[1][1]));
-            m_run = quad_group_max(max3(mx, S[1][2], S[1][3])) * c;
+            m_run = fmaxf(quad_group_max(max3(mx, S[1][2], S[1][3])) * c, kNoMax);
         }
         x8 P;
         float l_tile = 0.f;
@@ -1955,7 +1959,8 @@ attn_fwd_d512(const KArgs a) {
         }
         return;
     }
-    const float inv = l > 0.f ? 1.f / l : 0.f;
+    // (l is 0 where every score is -inf: NaN)
+    const float inv = l > 0.f ? 1.f / l : Skv > 0 ? NAN : 0.f;
     if (live) {
         T* op = Oh + qrow * a.so.s;
 #pragma unroll
@@ -2104,7 +2109,7 @@ __device__ __forceinline__ f32x4 merge_row(const CombArgs& c, long long row, int
     const long long rows = c.rows;
     const int ns = c.nsplit;
     const f32x2* ml = reinterpret_cast<const f32x2*>(c.ws_ml);
-    float mx = -3.0e38f;
+    float mx = kNoMax;
     for (int s0 = 0; s0 < ns; s0 += 2 * kCombBatch) {
         float m[2 * kCombBatch];
 #pragma unroll
@@ -2134,8 +2139,8 @@ __device__ __forceinline__ f32x4 merge_row(const CombArgs& c, long long row, int
                 l += w * mlv[u][1];
             }
     }
-    // (l is 0 where every score is -inf; D <= 64 gives NaN there, split or not)
-    return acc * (l > 0.f ? 1.f / l : c.D <= 64 ? NAN : 0.f);
+    // (l is 0 where every score is -inf: NaN, but 0 for D = 128, as unsplit)
+    return acc * (l > 0.f ? 1.f / l : c.D == 128 ? 0.f : NAN);
 }
 #endif
 
