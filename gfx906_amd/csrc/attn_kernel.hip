@@ -95,7 +95,7 @@ constexpr float kPmaxLimit = 256.0f;
 constexpr unsigned kOutOfRange = 0x80000000u;
 // Running max (log2 units) of a row none of whose scores is above -inf: finite,
 // so that a score of -inf gives p = 0 and not exp2(-inf + inf), and below every
-// other score.
+// other score (bf16 products reach -1e38).
 constexpr float kNoMax = -3.0e38f;
 // sched_group_barrier instruction classes
 constexpr int kSgMfma = 0x008, kSgDsRead = 0x100;
@@ -117,6 +117,7 @@ struct KArgs {
     Strides sq, sk, sv, so;
     int H, Sq, Skv, D;
     float c, qsign;
+    float m0;  // kNoMax as a score: m0 * c >= kNoMax, and no finite score below it counts
     // Split key range (kernels instantiated with SPLIT). Work units are the
     // query tiles of all heads, head-major. The first `whole` units run
     // unsplit (the rounds of workgroups that fill the GPU; 0 when none does),
@@ -406,7 +407,7 @@ __device__ __forceinline__ void q_negate(X8& f, unsigned qneg) {
 
 // Whether some element of a block's rounded P (two 8-element operands, all
 // non-negative) exceeds `lim` or is NaN, in any lane of the wave. The first
-// block (running max -1e30, p = inf) always does. A tree of
+// block (running max kNoMax, p = inf) always does. A tree of
 // v_pk_maximum3_f16 over the eight packed registers (4 instructions), then
 // one compare per half. bf16 has no packed maximum; its registers go
 // through the same tree read as fp16: non-negative values of either type
@@ -686,23 +687,20 @@ attn_fwd_pipe(const KArgs a) {
     constexpr bool kTileMax = !kLazy && TILEMAX;
     // Running max of each query column block. D = 128 keeps a lazy one, in
     // log2 units (s*c), raised only when some p exceeds 2^15 (rare after the
-    // first blocks: every p stays finite in fp16); it starts at -1e30
-    // (finite, so that a masked key, score -inf, gives p = 0). D <= 64 keeps
-    // the exact running max, in score units (s), starting at -inf (the first
+    // first blocks: every p stays finite in fp16); it starts at kNoMax. D <= 64
+    // keeps the exact running max, in score units (s), starting at -inf (the first
     // block's scores always exceed it), so that the dominant weight of a
     // row is exactly 1.0 in fp16: with a stale max it carries a rounding
     // error of up to 2^-11 relative, which on sharp rows with |o| near 4 and
     // above (c3: q, k ~ 2 N(0,1), 512 keys) moves the output past the 2e-3
-    // bar. Where key ranges are split it starts finite (its product with c
-    // must be), below every finite score that fp16 gives: a range may hold
-    // nothing but -inf scores (keys with infinite elements), which must give
-    // p = 0 and not exp2(-inf + inf).
+    // bar. Where key ranges are split it starts at m0: a range may hold
+    // nothing but -inf scores (keys with infinite elements).
     float m_run[2];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
 #pragma unroll
         for (int ob = 0; ob < NOB; ++ob) oacc[ob][nb] = f32x4{};
-        m_run[nb] = kLazy ? -1e30f : SPLIT ? -1e37f : -INFINITY;
+        m_run[nb] = kLazy ? kNoMax : SPLIT ? a.m0 : -INFINITY;
     }
     // 1 / l of a row whose scores are all -inf: NaN, as the -inf start gives.
     constexpr float kNoKeyInv = SPLIT && !kLazy ? NAN : 0.f;
@@ -1852,7 +1850,7 @@ attn_fwd_d512(const KArgs a) {
     f32x4 oacc[NOB];
 #pragma unroll
     for (int ob = 0; ob < NOB; ++ob) oacc[ob] = f32x4{};
-    float m_run = -1e30f;  // running max (log2 units); finite so masked keys give p = 0
+    float m_run = kNoMax;  // running max (log2 units)
     float l_run = 0.f;
 
     // P (B operand of the PV step) from the two score blocks, with running
@@ -2824,6 +2822,7 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     // scale == 0, c = 1e-30 gives exp2(s*c - m) == 1.0f exactly for every
     // finite score, i.e. the same uniform weights as c == 0.
     a.c = fmaxf(fabsf(scale) * kLog2e, 1e-30f);
+    a.m0 = kNoMax / fmaxf(a.c, 1.f);
     a.qsign = scale < 0.f ? -1.f : 1.f;
     a.BH = B * H;
     a.nsplit = 1;

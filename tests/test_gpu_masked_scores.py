@@ -73,6 +73,26 @@ def test_padded_head_dims(monkeypatch, D, form):
 SPANS = [((300, 310),), ((590, 600),), ((70, 90), (599, 600))]
 
 
+@pytest.mark.parametrize("form", ["ring x 3", "ring x 3, block max", "rows x 3", "default"])
+@pytest.mark.parametrize("D", [40, 64, 128])
+def test_large_scales(monkeypatch, D, form):
+    force(monkeypatch, form)
+    print(f"case masked: scale 60 D{D} {form}", flush=True)
+    q, k, v, keep = masked_inputs(2, 70, 600, D, ((0, 70), (300, 310)), D, amp=0.05)
+    check(q, k, v, keep, 60.0, False, form)
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("D", [40, 64, 128])
+def test_scores_far_below_zero(monkeypatch, D, form):
+    """bf16 scores of -1.5e37 and less: the largest takes all the weight. (The
+    scale makes scores in log2 units exact, as any rounding of theirs is far
+    above 1.)"""
+    force(monkeypatch, form)
+    print(f"case masked: far scores D{D} {form}", flush=True)
+    far_scores(D, gfx906_amd.attn)
+
+
 def far_scores(D, run):
     q = torch.zeros(1, 2, 70, D, dtype=torch.bfloat16)
     k = torch.zeros(1, 2, 600, D, dtype=torch.bfloat16)
