@@ -688,22 +688,18 @@ attn_fwd_pipe(const KArgs a) {
     // Running max of each query column block. D = 128 keeps a lazy one, in
     // log2 units (s*c), raised only when some p exceeds 2^15 (rare after the
     // first blocks: every p stays finite in fp16); it starts at kNoMax. D <= 64
-    // keeps the exact running max, in score units (s), starting at -inf (the first
-    // block's scores always exceed it), so that the dominant weight of a
-    // row is exactly 1.0 in fp16: with a stale max it carries a rounding
-    // error of up to 2^-11 relative, which on sharp rows with |o| near 4 and
-    // above (c3: q, k ~ 2 N(0,1), 512 keys) moves the output past the 2e-3
-    // bar. Where key ranges are split it starts at m0: a range may hold
-    // nothing but -inf scores (keys with infinite elements).
+    // keeps the exact running max, in score units (s), starting at m0, so that
+    // the dominant weight of a row is exactly 1.0 in fp16: with a stale max it
+    // carries a rounding error of up to 2^-11 relative, which on sharp rows
+    // with |o| near 4 and above (c3: q, k ~ 2 N(0,1), 512 keys) moves the
+    // output past the 2e-3 bar.
     float m_run[2];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
 #pragma unroll
         for (int ob = 0; ob < NOB; ++ob) oacc[ob][nb] = f32x4{};
-        m_run[nb] = kLazy ? kNoMax : SPLIT ? a.m0 : -INFINITY;
+        m_run[nb] = kLazy ? kNoMax : a.m0;
     }
-    // 1 / l of a row whose scores are all -inf: NaN, as the -inf start gives.
-    constexpr float kNoKeyInv = SPLIT && !kLazy ? NAN : 0.f;
     f32x4 lacc[2] = {f32x4{}, f32x4{}};
     x8 aone;
 #pragma unroll
@@ -945,8 +941,8 @@ attn_fwd_pipe(const KArgs a) {
         // max over both blocks, then computes S's P; the second (S2 null)
         // computes the second block's P with no test. On the workgroup's first
         // tile (`first`, wave-uniform) O and l are still exactly zero and the
-        // running max is -inf: the max is raised with no rescale (the rescale
-        // would multiply zeros by exp2(-inf) = 0; c3 rescales on most of its
+        // running max is m0: the max is raised with no rescale (the rescale
+        // would multiply zeros by a factor of 0; c3 rescales on most of its
         // eight tiles, so this drops about one in seven).
         auto softmax_tile = [&](f32x4 (&S)[2][2], x8 (&P)[2], const f32x4 (*S2)[2][2],
                                 bool first) __attribute__((always_inline)) {
@@ -1101,6 +1097,8 @@ attn_fwd_pipe(const KArgs a) {
         C::TAIL ? work_item<SPLIT, C::TAIL>(ea, block_here(), gridDim.x, (Sqe + C::BM - 1) / C::BM) : it;
     const int be = C::TAIL ? ite.bh / ea.H : b, he = C::TAIL ? ite.bh - be * ea.H : h;
     T* const Oe = C::TAIL ? (T*)ea.o + be * ea.so.b + he * ea.so.h : Oh;
+    // 1 / l where l is 0: a row whose scores are all -inf (NaN, but 0 for D = 128), or no keys.
+    const float no_key_inv = !kLazy && ea.Skv > 0 ? NAN : 0.f;
     int lane_e = lane, ie = i, ge = g, qrow0e = qrow0;
     if constexpr (DP <= 64 || C::TAIL) {
         lane_e = lane_id_here();
@@ -1142,7 +1140,7 @@ attn_fwd_pipe(const KArgs a) {
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
             const float l = quad_group_sum(lacc[nb][0]);
-            const float inv = l > 0.f ? 1.f / l : kNoKeyInv;
+            const float inv = l > 0.f ? 1.f / l : no_key_inv;
 #pragma unroll
             for (int ob = 0; ob < NOB; ++ob) {
                 const int d0 = 16 * ob + 4 * ge;
@@ -1176,7 +1174,7 @@ attn_fwd_pipe(const KArgs a) {
     for (int nb = 0; nb < 2; ++nb) {
         const int row = qrow0e + 16 * nb;
         const float l = quad_group_sum(lacc[nb][0]);
-        const float inv = l > 0.f ? 1.f / l : kNoKeyInv;
+        const float inv = l > 0.f ? 1.f / l : no_key_inv;
         if (row < Sqe) {
             T* op = Oe + row * ea.so.s;
 #pragma unroll
@@ -1386,7 +1384,7 @@ __global__ void __launch_bounds__(CfgRes::NT, 1) attn_fwd_kvres(const KArgs a) {
 #pragma unroll
             for (int ob = 0; ob < NOB; ++ob) oacc[ob][nb] = f32x4{};
             lacc[nb] = f32x4{};
-            m_run[nb] = -INFINITY;
+            m_run[nb] = a.m0;
         }
 
         // Block pipeline over the resident tiles, as attn_fwd_pipe's tile():
@@ -1419,7 +1417,7 @@ __global__ void __launch_bounds__(CfgRes::NT, 1) attn_fwd_kvres(const KArgs a) {
         for (int nb = 0; nb < 2; ++nb) {
             const int row = qrow0e + 16 * nb;
             const float l = quad_group_sum(lacc[nb][0]);
-            const float inv = l > 0.f ? 1.f / l : 0.f;
+            const float inv = l > 0.f ? 1.f / l : Skv > 0 ? NAN : 0.f;  // (as attn_fwd_pipe)
             if (row < Sq) {
                 T* op = Oh + row * a.so.s;
 #pragma unroll

@@ -2,7 +2,8 @@
 
 A key whose score is -inf weighs nothing, whatever the head dim (padded ones
 among them), and wherever such keys lie: in the first tile, in a whole key
-range, between finite ones. A row of nothing else is NaN (D = 512). Finite scores of any size that fp32 holds count.
+range, between finite ones. A row of nothing else is NaN (0 for D = 128), in
+every kernel and split alike. Finite scores of any size that fp32 holds count.
 Outputs are held to the bars against SDPA MATH in fp32 over the keys that
 count. Each case prints its parameters first.
 """
@@ -71,6 +72,19 @@ def test_padded_head_dims(monkeypatch, D, form):
 
 # Finite keys past the first tiles only, in the middle range of three, in the last.
 SPANS = [((300, 310),), ((590, 600),), ((70, 90), (599, 600))]
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("D", [40, 64, 128])
+def test_first_tiles_and_whole_ranges(monkeypatch, D, form):
+    force(monkeypatch, form)
+    print(f"case masked: first tiles D{D} {form}", flush=True)
+    for n, spans in enumerate(SPANS):
+        for bf16 in (False, True):
+            q, k, v, keep = masked_inputs(2, 70, 600, D, spans, D + n, bf16)
+            check(q, k, v, keep, 0.1, bf16, (form, spans))
+    out = gfx906_amd.attn(q.to(DEV), torch.full_like(k, float("-inf")).to(DEV), v.to(DEV), 0.1)
+    assert bool((out == 0).all() if D == 128 else out.isnan().all())
 
 
 @pytest.mark.parametrize("form", ["ring x 3", "ring x 3, block max", "rows x 3", "default"])
@@ -155,7 +169,7 @@ def test_d512_split_tail(layout):
     near(got, ref, False, layout)
 
 
-@pytest.mark.parametrize("D", [512])
+@pytest.mark.parametrize("D", [40, 64, 128, 512])
 def test_no_keys_are_zeros(D):
     """Skv = 0 is not a row of -inf scores: zeros."""
     print(f"case masked: no keys D{D}", flush=True)
