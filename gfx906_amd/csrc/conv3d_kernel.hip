@@ -69,6 +69,8 @@ struct ConvArgs {
 };
 
 constexpr int kMaxTaps = 1024;
+constexpr long kMaxVoxels = (1L << 31) - 256;  // M
+constexpr long kMaxBytes = 1L << 31;           // span of x or w
 constexpr unsigned kOOB = 0xFFFFFFF0u;  // buffer offset past any range: loads zeros
 
 // Per-configuration sizes: NB 32-voxel MFMA blocks per wave, CW waves along
@@ -598,7 +600,10 @@ ConvPlan plan_conv(long M, int K, long KG, size_t ws_cap) {
     unsigned tiles1[kNumKernels], fewest = ~0u;  // tiles of each configuration, unsplit
     for (int i = 0; i < kNumKernels; ++i) {
         const ConvKernel& c = kKernels[i];
-        tiles1[i] = (unsigned)((M + 64 * c.nb - 1) / (64 * c.nb) * ((K + c.bch - 1) / c.bch));
+        // (held to 2^24, an output past the device's memory, so that 32 bits count the ranges too)
+        tiles1[i] = (unsigned)std::min((M + 64 * c.nb - 1) / (64 * c.nb) *
+                                           (((long)K + c.bch - 1) / c.bch),
+                                       1L << 24);
         fewest = std::min(fewest, tiles1[i]);
     }
     // More than four rounds of workgroups gain nothing (and the search costs
@@ -660,7 +665,7 @@ int conv3d_impl(const void* x, const void* w, const void* bias, const void* res,
     if (D < T || H < R || W < S || Z != (D - T) / sd + 1 || P != (H - R) / sh + 1 ||
         Q != (W - S) / sw + 1)
         return fail("conv3d: output size does not match a VALID convolution");
-    if (M != (long)nB * Z * P * Q || M >= (1L << 31) - 256)
+    if (M != (long)nB * Z * P * Q || M >= kMaxVoxels)
         return fail("conv3d: M must be nB*Z*P*Q < 2^31 - 256");
     if ((long)T * R * S > kMaxTaps) return fail("conv3d: more than 1024 taps");
     if (!x || !w || !out) return fail("conv3d: null pointer");
@@ -673,7 +678,7 @@ int conv3d_impl(const void* x, const void* w, const void* bias, const void* res,
     const long KG = (long)C * T * R * S;
     const long x_span = ((nB - 1) * xsn + (D - 1) * xsd + (H - 1) * xsh + (W - 1) * xsw + C) * 2;
     const long w_span = (long)K * KG * 2;
-    if (x_span >= (1L << 31) || w_span >= (1L << 31))
+    if (x_span >= kMaxBytes || w_span >= kMaxBytes)
         return fail("conv3d: x or w spans 2^31 bytes or more");
     ConvArgs a;
     a.x = (const f16*)x;
@@ -758,7 +763,10 @@ extern "C" int conv3d_fwd(const void* x, const void* w, const void* bias, const 
 }
 
 extern "C" size_t conv3d_workspace_bytes(long M, int K, long KG) {
-    if (M <= 0 || K <= 0 || KG <= 0) return 0;
+    // Sizes that conv3d_fwd_split() refuses need none.
+    if (M <= 0 || K <= 0 || KG <= 0 || M >= kMaxVoxels || KG >= kMaxBytes ||
+        (long)K * KG * 2 >= kMaxBytes)
+        return 0;
     return conv_ws_bytes(plan_conv(M, K, KG, kScratchBytes), M, K);
 }
 

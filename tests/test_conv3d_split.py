@@ -124,3 +124,24 @@ def test_plan_sizes(monkeypatch):
         assert ws(100, 64, 64 * 27) == -(-units // per) * 100 * 64 * 4
     monkeypatch.setenv("GFX906_AMD_CONV_NSPLIT", "8")
     assert ws(1 << 20, 512, 13824) == 0        # 17 GB of partial sums: not split
+
+
+@pytest.mark.parametrize("M,K,KG", [(1 << 40, 64, 1000), ((1 << 31) - 256, 64, 1728),
+                                    (1 << 32, 64, 1728), (256, 64, 1 << 40), (256, 64, 1 << 62),
+                                    (256, (1 << 31) - 8, 64), (256, 1 << 20, 1024),
+                                    ((1 << 31) - 512, 1 << 20, 8)])
+def test_sizes_past_the_limits_need_no_workspace(M, K, KG):
+    # (needs no GPU; such calls are refused by conv3d_fwd_split itself)
+    assert lib().conv3d_workspace_bytes(M, K, KG) == 0
+
+
+@pytest.mark.gpu
+def test_too_many_voxels_raise():
+    print("case conv split: M past 2^31", flush=True)
+    x, w, b, res = oc.make_case((1, 8, 1, 4, 4), (8, 1, 1, 1), (1, 1, 1), False, False, seed=1)
+    call = kitchen.plan(to_dev(x), to_dev(w), None, None, [1, 1, 1])
+    dims = list(call.dims)
+    dims[0] = 1 << 28  # M = 2^32: refused before any launch
+    with pytest.raises(RuntimeError, match="M must be"):
+        gfx906_amd.extension().conv3d(call.x, call.weight, None, None, call.out, dims, call.xs,
+                                      call.os, call.rs)
