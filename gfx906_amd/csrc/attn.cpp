@@ -77,10 +77,11 @@ bool token_contiguous_kv(const torch::Tensor& t) {
     return (D - 1) * s[3] + S < (int64_t(1) << 30);
 }
 
-// Whether t is token-contiguous, whatever its other strides and alignment.
+// Whether t is token-contiguous, whatever its other strides and alignment (by
+// the strides that the kernel gets: a single token is not).
 bool token_runs(const torch::Tensor& t) {
     const auto s = strides4(t);
-    return t.stride(2) == 1 && s[3] > 1 && s[0] >= 0 && s[1] >= 0;
+    return s[2] == 1 && s[3] > 1 && s[0] >= 0 && s[1] >= 0;
 }
 
 // Largest Skv for which reading token-contiguous k/v in place beats copying

@@ -144,3 +144,19 @@ def test_row_copies_rejects():
         rc, err = call(**kw)
         assert rc == 1 and msg in err, (kw, err)
     assert lib.attn_row_copies_bytes(1, 1, 64, 64, 128) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Sq,Skv", [(1, 6408), (1, 100), (1, 64), (40, 1), (1, 1)])
+def test_one_token(Sq, Skv):
+    """The op on token-strided tensors of one query or one key (whose token
+    stride says nothing), past the in-place limit, at a count that is no
+    multiple of 8, and in place."""
+    print(f"case tok512: one token, Sq{Sq} Skv{Skv}", flush=True)
+    g = torch.Generator().manual_seed(Sq + Skv)
+    q, k, v = (torch.randn(1, 2, s, 512, generator=g).half().to(DEV) for s in (Sq, Skv, Skv))
+    obuf, o = tokens(torch.zeros_like(q), 8)
+    got = gfx906_amd.attn(tokens(q)[1], tokens(k)[1], tokens(v)[1], 0.04, out=o)
+    mx, mn = error_stats(got.float().cpu(), sdpa_math_fp32(q.cpu(), k.cpu(), v.cpu(), 0.04))
+    assert mx <= MAX_ABS_TOL and mn <= MEAN_ABS_TOL, (mx, mn)
+    assert bool(obuf[..., Sq:].isnan().all())
