@@ -9,8 +9,8 @@
 // reads within the same call, so nothing is cleared between calls.
 //
 // Calls that use the array are ordered on the GPU, whatever streams they are
-// issued on: each records an event on its stream after its kernels, and a
-// call on another stream first makes its stream wait for that event (the host
+// issued on: each records an event on its stream after its kernels, and the
+// next call first makes its stream wait for that event (the host
 // lock keeps wait, launches and record of one call together, so the calls
 // form one chain per device). A call made under stream capture neither waits
 // nor records (an event recorded outside the graph cannot order its replays):

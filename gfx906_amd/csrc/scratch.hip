@@ -15,7 +15,6 @@ constexpr int kMaxDevices = 64;
 struct DevScratch {
     void* ptr;           // device address of `scratch`
     hipEvent_t done;     // recorded after the last call outside capture that used it
-    hipStream_t last;    // the stream of that call
     bool recorded;
 };
 
@@ -55,7 +54,6 @@ hipError_t scratch_setup(int dev) {
     }
     d.ptr = p;
     d.done = ev;
-    d.last = nullptr;
     d.recorded = false;
     return hipSuccess;
 }
@@ -88,8 +86,11 @@ ScratchUse::Status ScratchUse::acquire(hipStream_t stream, bool allow_capture) {
         if (capturing_) return kUnavailable;
         if ((e = scratch_setup(dev)) != hipSuccess) return failed(e);
     }
-    if (!capturing_ && d.recorded && d.last != stream &&
-        (e = hipStreamWaitEvent(stream, d.done, 0)) != hipSuccess)
+    // Also where the last call's stream has this one's handle: handles do not
+    // name streams (hipStreamPerThread is one value for every thread's own
+    // stream, and a new stream can get a destroyed one's). The runtime, which
+    // knows the stream, drops the wait where it really is the same.
+    if (!capturing_ && d.recorded && (e = hipStreamWaitEvent(stream, d.done, 0)) != hipSuccess)
         return failed(e);
     dev_ = &d;
     ptr = d.ptr;
@@ -99,10 +100,7 @@ ScratchUse::Status ScratchUse::acquire(hipStream_t stream, bool allow_capture) {
 hipError_t ScratchUse::release(hipStream_t stream) {
     if (!dev_ || capturing_) return hipSuccess;
     const hipError_t e = hipEventRecord(dev_->done, stream);
-    if (e == hipSuccess) {
-        dev_->last = stream;
-        dev_->recorded = true;
-    }
+    if (e == hipSuccess) dev_->recorded = true;
     return e;
 }
 

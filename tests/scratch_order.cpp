@@ -1,0 +1,77 @@
+// ScratchUse (gfx906_amd/csrc/scratch.hip) on a HIP runtime that only keeps
+// account: streams and events are numbers, and every wait and record is a line
+// of output. argv[1] names the sequence of calls. Built and run by
+// test_scratch_order.py with the host compiler; needs no GPU.
+#include <cstdio>
+#include <cstring>
+
+#include "scratch.h"
+
+using gfx906_amd::ScratchUse;
+
+static int n_events = 0, record_fails = 0;
+static bool capturing = false;
+
+extern "C" {
+hipError_t hipGetDevice(int* dev) { return *dev = 0, hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t* dev) { return *dev = 0, hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st) {
+    *st = capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void** p, const void*) {
+    return *p = reinterpret_cast<void*>(uintptr_t(1) << 40), hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    *e = reinterpret_cast<hipEvent_t>(uintptr_t(++n_events));
+    return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+    std::printf("wait s%d e%d\n", int((uintptr_t)s), int((uintptr_t)e));
+    return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+    if (record_fails > 0) return --record_fails, hipErrorUnknown;
+    std::printf("record s%d e%d\n", int((uintptr_t)s), int((uintptr_t)e));
+    return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t s) {
+    std::printf("synchronize s%d\n", int((uintptr_t)s));
+    return hipSuccess;
+}
+const char* hipGetErrorString(hipError_t) { return "error"; }
+}
+
+static hipStream_t stream(int n) { return reinterpret_cast<hipStream_t>(uintptr_t(n)); }
+
+// One call on stream n.
+static void call(int n) {
+    ScratchUse use;
+    if (use.acquire(stream(n), true) != ScratchUse::kReady) std::printf("not ready\n");
+    std::printf("call s%d\n", n);
+    if (use.release(stream(n)) != hipSuccess) std::printf("not released\n");
+}
+
+int main(int argc, char** argv) {
+    const char* what = argc > 1 ? argv[1] : "";
+    if (!std::strcmp(what, "same handle")) {
+        call(2);  // hipStreamPerThread's value: another stream in each thread
+        call(2);
+        call(2);
+    } else if (!std::strcmp(what, "two streams")) {
+        call(7);
+        call(8);
+        call(7);
+    } else if (!std::strcmp(what, "capture")) {
+        call(7);
+        capturing = true;
+        call(8);
+        capturing = false;
+        call(9);
+    } else {
+        return 1;
+    }
+    return 0;
+}
