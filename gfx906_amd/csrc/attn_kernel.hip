@@ -2907,7 +2907,7 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     }
     hipError_t e = dtype == ATTN_DTYPE_BF16 ? launch_t<bf16>(a, tl, rp.rows, stream)
                                             : launch_t<f16>(a, tl, rp.rows, stream);
-    if (e == hipSuccess) e = scratch.release(stream);
+    if (e == hipSuccess) e = scratch.release();
     if (e != hipSuccess) {
         set_err(hipGetErrorString(e));
         return 2;

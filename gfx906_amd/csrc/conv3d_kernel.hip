@@ -742,7 +742,7 @@ int conv3d_impl(const void* x, const void* w, const void* bias, const void* res,
                            stream, a);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = scratch.release(stream);
+    if (e == hipSuccess) e = scratch.release();
     if (e != hipSuccess) {
         set_err(hipGetErrorString(e));
         return 2;

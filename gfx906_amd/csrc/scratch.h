@@ -30,7 +30,9 @@ constexpr size_t kScratchBytes = size_t(96) << 20;
 struct DevScratch;
 
 // One call's use of the scratch of its stream's device: acquire() before its
-// launches, release() after them; the lock is held in between.
+// launches, release() after them; the lock is held in between. A call that ends
+// on an error releases it too (a launch before the failed one may be queued):
+// the destructor does.
 class ScratchUse {
  public:
     enum Status {
@@ -39,8 +41,11 @@ class ScratchUse {
         kFailed,       // error: `error`, or the device index is beyond the table
     };
     ScratchUse();
+    ~ScratchUse() { (void)release(); }
+    ScratchUse(const ScratchUse&) = delete;
+    ScratchUse& operator=(const ScratchUse&) = delete;
     Status acquire(hipStream_t stream, bool allow_capture);
-    hipError_t release(hipStream_t stream);  // no-op unless acquired
+    hipError_t release();  // no-op unless acquired
 
     void* ptr = nullptr;
     const char* error = nullptr;
@@ -48,6 +53,7 @@ class ScratchUse {
  private:
     std::unique_lock<std::mutex> lock_;
     DevScratch* dev_ = nullptr;
+    hipStream_t stream_ = nullptr;
     bool capturing_ = false;
 };
 

@@ -93,14 +93,20 @@ ScratchUse::Status ScratchUse::acquire(hipStream_t stream, bool allow_capture) {
     if (!capturing_ && d.recorded && (e = hipStreamWaitEvent(stream, d.done, 0)) != hipSuccess)
         return failed(e);
     dev_ = &d;
+    stream_ = stream;
     ptr = d.ptr;
     return kReady;
 }
 
-hipError_t ScratchUse::release(hipStream_t stream) {
-    if (!dev_ || capturing_) return hipSuccess;
-    const hipError_t e = hipEventRecord(dev_->done, stream);
-    if (e == hipSuccess) dev_->recorded = true;
+hipError_t ScratchUse::release() {
+    DevScratch* const d = dev_;
+    dev_ = nullptr;
+    if (!d || capturing_) return hipSuccess;
+    const hipError_t e = hipEventRecord(d->done, stream_);
+    if (e == hipSuccess)
+        d->recorded = true;
+    else  // (no event to order the next call by)
+        (void)hipStreamSynchronize(stream_);
     return e;
 }
 

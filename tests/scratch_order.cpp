@@ -51,7 +51,7 @@ static void call(int n) {
     ScratchUse use;
     if (use.acquire(stream(n), true) != ScratchUse::kReady) std::printf("not ready\n");
     std::printf("call s%d\n", n);
-    if (use.release(stream(n)) != hipSuccess) std::printf("not released\n");
+    if (use.release() != hipSuccess) std::printf("not released\n");
 }
 
 int main(int argc, char** argv) {
@@ -64,6 +64,17 @@ int main(int argc, char** argv) {
         call(7);
         call(8);
         call(7);
+    } else if (!std::strcmp(what, "failed call")) {
+        {
+            ScratchUse use;  // its second launch fails: no release()
+            use.acquire(stream(7), true);
+            std::printf("launch s7\n");
+        }
+        call(8);
+    } else if (!std::strcmp(what, "failed record")) {
+        record_fails = 1;
+        call(7);
+        call(8);
     } else if (!std::strcmp(what, "capture")) {
         call(7);
         capturing = true;

@@ -46,3 +46,14 @@ def test_two_streams_are_ordered(program):
 def test_captured_calls_neither_wait_nor_record(program):
     assert lines(program, "capture") == [
         "call s7", "record s7 e1", "call s8", "wait s9 e1", "call s9", "record s9 e1"]
+
+
+def test_a_failed_call_is_waited_for(program):
+    """A call whose merge cannot be launched leaves a kernel queued."""
+    assert lines(program, "failed call") == [
+        "launch s7", "record s7 e1", "wait s8 e1", "call s8", "record s8 e1"]
+
+
+def test_a_failed_record_waits_on_the_host(program):
+    assert lines(program, "failed record") == [
+        "call s7", "synchronize s7", "not released", "call s8", "record s8 e1"]
