@@ -2861,7 +2861,7 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
         rp = kNoRows;  // (a forced count)
     ScratchUse scratch;
     if (need && use_scratch && rp.nsplit != 1) {
-        const ScratchUse::Status st = scratch.acquire(stream, p.whole == 0);
+        const ScratchUse::Status st = scratch.acquire(stream, need, p.whole == 0);
         if (st == ScratchUse::kUnavailable && p.whole > 0) {
             p = kNoSplit;
             need = 0;
@@ -2874,7 +2874,7 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
             return 2;
         }
         workspace = scratch.ptr;
-        workspace_bytes = kScratchBytes;
+        workspace_bytes = need;
     }
     if (need && !(use_scratch && rp.nsplit == 1)) {
         if (!workspace || workspace_bytes < need || (uintptr_t)workspace % 16) {

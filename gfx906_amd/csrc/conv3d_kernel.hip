@@ -718,14 +718,15 @@ int conv3d_impl(const void* x, const void* w, const void* bias, const void* res,
     if (p.nsplit > 1 && use_scratch) {
         // A captured call takes no scratch (its replays could run beside other
         // calls that use it) and runs unsplit.
-        const ScratchUse::Status st = scratch.acquire(stream, false);
+        const size_t need = conv_ws_bytes(p, M, K);
+        const ScratchUse::Status st = scratch.acquire(stream, need, false);
         if (st == ScratchUse::kFailed) {
             set_err(scratch.error);
             return 2;
         }
         if (st == ScratchUse::kUnavailable) p = plan_conv(M, K, KG, 0);
         workspace = scratch.ptr;
-        workspace_bytes = kScratchBytes;
+        workspace_bytes = need;
     }
     if (p.nsplit > 1 && (!workspace || workspace_bytes < conv_ws_bytes(p, M, K) ||
                          (uintptr_t)workspace % 16))

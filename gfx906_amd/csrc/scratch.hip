@@ -12,10 +12,20 @@ namespace gfx906_amd {
 static __device__ __align__(256) char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
+constexpr int kPieces = kScratchBytes / kScratchPiece;
+static_assert(kPieces * kScratchPiece == kScratchBytes, "whole pieces");
+
+// A piece of a device's scratch as the last call outside capture left it.
+struct ScratchPiece {
+    hipEvent_t done;     // recorded by the last call whose first piece this was
+    int guard;           // the piece whose `done` covers the last call that used this one
+    const void* stream;  // that call's stream, a preference only
+    unsigned long long used;  // number of that call (0: none)
+};
 struct DevScratch {
-    void* ptr;           // device address of `scratch`
-    hipEvent_t done;     // recorded after the last call outside capture that used it
-    bool recorded;
+    void* ptr;  // device address of `scratch`
+    unsigned long long calls;
+    ScratchPiece piece[kPieces];
 };
 
 namespace {
@@ -23,7 +33,7 @@ namespace {
 std::mutex g_scratch_mu;
 DevScratch g_scratch[kMaxDevices];
 
-// Looks up `scratch` on device dev and creates its ordering event, once.
+// Looks up `scratch` on device dev and creates its ordering events, once.
 // Caller holds g_scratch_mu.
 hipError_t scratch_setup(int dev) {
     DevScratch& d = g_scratch[dev];
@@ -33,36 +43,59 @@ hipError_t scratch_setup(int dev) {
     if (e == hipSuccess && dev != cur) e = hipSetDevice(dev);
     if (e != hipSuccess) return e;
     void* p = nullptr;
-    hipEvent_t ev = nullptr;
     e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
     if (e == hipSuccess && !p) e = hipErrorInvalidSymbol;
-    // The event only orders kernels of this device on two of its streams
+    // The events only order kernels of this device on two of its streams
     // (hipStreamWaitEvent); nothing on the host or on another device inspects
-    // it, so its record needs no system-scope fence: the kernels' own release
+    // them, so their records need no system-scope fence: the kernels' own release
     // at their end makes the scratch visible to the device's later kernels.
     // Without the fence a call that splits costs about 2 us less of GPU time
     // (measured on MI355X: B1 H1 S1024 D64 through launch() 16.3 -> 14.5 us).
-    if (e == hipSuccess)
-        e = hipEventCreateWithFlags(&ev, hipEventDisableTiming | hipEventDisableSystemFence);
+    int made = 0;
+    while (e == hipSuccess && made < kPieces) {
+        e = hipEventCreateWithFlags(&d.piece[made].done,
+                                    hipEventDisableTiming | hipEventDisableSystemFence);
+        made += e == hipSuccess;
+    }
     if (dev != cur) {
         const hipError_t r = hipSetDevice(cur);
         if (e == hipSuccess) e = r;
     }
     if (e != hipSuccess) {
-        if (ev) (void)hipEventDestroy(ev);
+        while (made > 0) (void)hipEventDestroy(d.piece[--made].done);
         return e;
     }
     d.ptr = p;
-    d.done = ev;
-    d.recorded = false;
     return hipSuccess;
+}
+
+// First of the n pieces for a call on `stream`: pieces that the stream's last
+// calls used (no other call to wait for), else the ones unused for longest.
+int pick_pieces(const DevScratch& d, int n, const void* stream) {
+    int best = 0;
+    unsigned long long best_used = ~0ull;
+    for (int p = 0; p + n <= kPieces; ++p) {
+        bool own = true;
+        unsigned long long used = 0;
+        for (int k = p; k < p + n; ++k) {
+            own = own && d.piece[k].used && d.piece[k].stream == stream;
+            if (d.piece[k].used > used) used = d.piece[k].used;
+        }
+        if (own) return p;
+        if (used < best_used) {
+            best_used = used;
+            best = p;
+        }
+    }
+    return best;
 }
 
 }  // namespace
 
 ScratchUse::ScratchUse() : lock_(g_scratch_mu, std::defer_lock) {}
 
-ScratchUse::Status ScratchUse::acquire(hipStream_t stream, bool allow_capture) {
+ScratchUse::Status ScratchUse::acquire(hipStream_t stream, size_t bytes,
+                                       bool allow_capture) {
     auto failed = [&](hipError_t e) {
         error = hipGetErrorString(e);
         return kFailed;
@@ -86,15 +119,32 @@ ScratchUse::Status ScratchUse::acquire(hipStream_t stream, bool allow_capture) {
         if (capturing_) return kUnavailable;
         if ((e = scratch_setup(dev)) != hipSuccess) return failed(e);
     }
-    // Also where the last call's stream has this one's handle: handles do not
-    // name streams (hipStreamPerThread is one value for every thread's own
-    // stream, and a new stream can get a destroyed one's). The runtime, which
-    // knows the stream, drops the wait where it really is the same.
-    if (!capturing_ && d.recorded && (e = hipStreamWaitEvent(stream, d.done, 0)) != hipSuccess)
-        return failed(e);
+    if (bytes > kScratchBytes) {
+        error = "more than the scratch holds";
+        return kFailed;
+    }
     dev_ = &d;
     stream_ = stream;
+    count_ = (int)((bytes + kScratchPiece - 1) / kScratchPiece);
+    first_ = 0;
     ptr = d.ptr;
+    if (capturing_) return kReady;
+    static thread_local char this_thread;
+    key_ = stream == hipStreamPerThread ? (const void*)&this_thread : (const void*)stream;
+    first_ = pick_pieces(d, count_, key_);
+    ptr = (char*)d.ptr + first_ * kScratchPiece;
+    // Also where the last call's stream has this one's handle: handles do not
+    // name streams (a new stream can get a destroyed one's). The runtime, which
+    // knows the stream, drops the wait where it really is the same.
+    for (int k = first_; k < first_ + count_; ++k) {
+        const ScratchPiece& sp = d.piece[k];
+        if (!sp.used || (k > first_ && sp.guard == d.piece[k - 1].guard && d.piece[k - 1].used))
+            continue;
+        if ((e = hipStreamWaitEvent(stream, d.piece[sp.guard].done, 0)) != hipSuccess) {
+            dev_ = nullptr;
+            return failed(e);
+        }
+    }
     return kReady;
 }
 
@@ -102,12 +152,21 @@ hipError_t ScratchUse::release() {
     DevScratch* const d = dev_;
     dev_ = nullptr;
     if (!d || capturing_) return hipSuccess;
-    const hipError_t e = hipEventRecord(d->done, stream_);
-    if (e == hipSuccess)
-        d->recorded = true;
-    else  // (no event to order the next call by)
+    // One record covers all pieces. It may replace one that other pieces still
+    // name as their guard; this call waited for that one, so the new one covers
+    // it too.
+    const hipError_t e = hipEventRecord(d->piece[first_].done, stream_);
+    if (e != hipSuccess) {  // (no event to order the next call by)
         (void)hipStreamSynchronize(stream_);
-    return e;
+        return e;
+    }
+    ++d->calls;
+    for (int k = first_; k < first_ + count_; ++k) {
+        d->piece[k].guard = first_;
+        d->piece[k].stream = key_;
+        d->piece[k].used = d->calls;
+    }
+    return hipSuccess;
 }
 
 }  // namespace gfx906_amd

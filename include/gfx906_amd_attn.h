@@ -14,10 +14,13 @@
  * and launch_conv3d(), which split reductions in it): a device array
  * of attn_split_scratch_capacity() bytes that is part of the library's code
  * object, so it is held on every GPU where the library's kernels are loaded,
- * until the process ends. Those calls are ordered on the GPU across streams
- * (each waits for the previous one on its device) except under stream
- * capture, where a captured call neither waits nor is waited for: a graph
- * that contains one is ordered only by the stream it is launched on.
+ * until the process ends. Each call takes a part of it. Calls that use the
+ * same part are ordered on the GPU whatever their streams (each waits for the
+ * previous one); different streams get different parts while these last, and
+ * their calls may run side by side. A call under stream capture neither waits
+ * nor is waited for: a graph that contains one is ordered only by the stream
+ * it is launched on, and must not run concurrently with other streams' calls
+ * that use the scratch.
  */
 #ifndef GFX906_AMD_ATTN_H
 #define GFX906_AMD_ATTN_H
@@ -107,7 +110,7 @@ int attn_fwd_split(const void* q, const void* k, const void* v, void* o,
  * the same as attn_fwd_split()'s whenever attn_split_workspace_bytes() <=
  * capacity (then the results are bit-identical), fewer splits or none
  * otherwise. Problems that do not split use no scratch. Calls that use the
- * scratch are ordered across streams on one device (see the top of this
+ * same part of the scratch are ordered across streams (see the top of this
  * file); under stream capture the first such call on a device must have
  * been made outside capture (it sets the scratch up), else status 1; problems
  * that fill the GPU do not use the scratch under capture and run unsplit. Same

@@ -55,8 +55,8 @@ int conv3d_fwd(const void* x, const void* w, const void* bias, const void* res, 
  * more workgroups: each range's fp32 sums go to a workspace and a second
  * kernel adds them up. launch_conv3d() and conv3d_fwd() keep them in the
  * library's static scratch (attn_split_scratch_capacity() bytes; such calls
- * are ordered across streams on one device, see gfx906_amd_attn.h) and do not
- * split under stream capture. conv3d_fwd_split() takes a caller workspace
+ * are ordered where they use the same part of it, see gfx906_amd_attn.h) and
+ * do not split under stream capture. conv3d_fwd_split() takes a caller workspace
  * instead (16-byte aligned, conv3d_workspace_bytes() bytes, with
  * M = nB*Z*P*Q and KG = C*T*R*S; 0: not split) and needs no ordering. Both
  * give the same bits. No counterpart in the reference. */
