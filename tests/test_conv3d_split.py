@@ -89,7 +89,7 @@ def test_forced_split_counts(monkeypatch, cfg, i, nsplit):
 
 
 @pytest.mark.gpu
-def test_small_layer_is_split_and_accurate_in_a_graph():
+def test_small_layer_is_split_and_accurate_in_a_graph(monkeypatch):
     x, w, b, res = oc.make_case((1, 256, 3, 18, 18), (256, 3, 3, 3), (1, 1, 1), True, True, 510)
     print("case conv split: planner's own choice, eager and captured", flush=True)
     assert lib().conv3d_workspace_bytes(256, 256, 256 * 27) > 0
@@ -103,11 +103,17 @@ def test_small_layer_is_split_and_accurate_in_a_graph():
     with torch.cuda.graph(graph):
         call.run(ext)
         unsplit = run_capi(call)  # the C entry takes no scratch under capture
+    with monkeypatch.context() as m:
+        m.setenv("GFX906_AMD_CONV_NSPLIT", "1")
+        plain = run_capi(call)
+    assert not torch.equal(plain, eager)
     for _ in range(3):
         call.out.zero_()
+        unsplit.zero_()
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(call.out, eager)
+        assert torch.equal(unsplit, plain)
         check(unsplit, oc.conv3d_gemm(x, w, b, res, (1, 1, 1)), "captured C entry")
 
 

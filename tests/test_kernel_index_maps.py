@@ -1,7 +1,7 @@
 """CPU checks of two index maps the HIP kernels rely on, restated from the
 kernel source (the GPU parity tests check the kernels themselves):
 
-* the token-contiguous D = 512 attention tiles (attn_fwd_d512<T, true>): the
+* the token-contiguous D = 512 attention tiles (attn_fwd_tok512): the
   direct loads' chunk choice, the transposed K reads (ds_read_b64_tr_b16: in
   each 16-lane group, lane i receives element i%4 of the 8 bytes read by lanes
   4e + i/4, e = 0..3) and the V^T reads deliver exactly the MFMA operands, P's
