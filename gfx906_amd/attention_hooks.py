@@ -127,8 +127,8 @@ class DitRouter:
 def _token_view(x):
     """[b, c, h, w] -> [b, 1, h*w, c] view (sequence stride 1, channel stride
     h*w). The op reads and writes such views in place, or has the library make
-    row copies where it cannot (h*w not a multiple of 8) or that is faster
-    (h*w > 6400)."""
+    row copies where it cannot (h*w not a multiple of 8) or h*w > 6400, where
+    they are faster."""
     b, c, h, w = x.shape
     return x.reshape(b, c, h * w).transpose(1, 2).unsqueeze(1)
 

@@ -589,8 +589,9 @@ __device__ __forceinline__ void block_exp(const f32x4& S0, const f32x4& S1,
 #endif
 
 // grid: ceil(Sq / BM) * B*H workgroups (SPLIT: whole + tail * nsplit), query
-// tiles of one head adjacent, see work_item; block: NW*64 threads. The second launch bound is HIP's minimum waves per SIMD
-// (amdgpu_waves_per_eu): OCC workgroups of NW waves over the CU's four SIMDs.
+// tiles of one head adjacent, see work_item; block: NW*64 threads. The second
+// launch bound is HIP's minimum waves per SIMD (amdgpu_waves_per_eu): OCC
+// workgroups of NW waves over the CU's four SIMDs.
 template <class C, bool PAD, class T, bool SPLIT, bool TILEMAX>
 __global__ void __launch_bounds__(C::NT, C::OCC * C::NW / 4)
 attn_fwd_pipe(const KArgs a) {
@@ -2476,9 +2477,9 @@ long long first_split_row(int whole, int Sq, int D) {
 // as there are key tiles at most, fewer where n does not divide them into
 // non-empty ranges of whole tiles (the same rule as below), and no split
 // when n = 1 or when the partial results would not fit ws_cap.
-// tail: whether the call can run a split tail after whole rounds (the kernels
-// of the token-contiguous layout and of 16 rows per wave cannot, and the
-// K/V-resident kernel balances its items itself).
+// tail: whether the call can run a split tail after whole rounds (the 16-row
+// D = 512 kernel, a test override, cannot; the K/V-resident kernel balances its
+// items itself).
 SplitPlan plan_split(int B, int H, int Sq, int Skv, int D, bool tail,
                      size_t ws_cap = (size_t)-1) {
     const int bm = query_tile(D);

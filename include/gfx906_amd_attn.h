@@ -7,7 +7,8 @@
  * attn_fwd_ex() also takes bf16 and per-tensor strides.
  * D must be <= 64 and a multiple of 8, or 128, or 512. Sq != Skv is allowed.
  * o[b,h,i,:] = sum_j softmax_j(scale * <q[b,h,i,:], k[b,h,j,:]>) v[b,h,j,:],
- * rounded to the element type; rows with Skv == 0 are written as zeros.
+ * rounded to the element type; rows with Skv == 0 are written as zeros. A
+ * score of -inf weighs nothing; a row of nothing else is NaN (0 for D = 128).
  * Calls are asynchronous on `stream`. The only state kept between calls is
  * the static scratch of the calls that split key ranges without a caller
  * workspace (launch(), attn_fwd(), attn_fwd_split_static(), and conv3d_fwd()
@@ -87,8 +88,8 @@ size_t attn_split_workspace_bytes(int B, int H, int Sq, int Skv, int D);
 
 /* attn_fwd_ex() that, when B*H*Sq is too small to fill the GPU (a VAE
  * attention over one head, short problems) or leaves its last round of
- * workgroups nearly empty, splits key ranges over more workgroups: each writes its unnormalised partial output and running
- * max/sum to `workspace` (device memory, 16-byte aligned, at least
+ * workgroups nearly empty, splits key ranges over more workgroups: each
+ * writes its unnormalised partial output and running max/sum to `workspace` (device memory, 16-byte aligned, at least
  * attn_split_workspace_bytes() bytes; may be NULL when that is 0) and a
  * second kernel merges them into o. Same arguments and return codes as
  * attn_fwd_ex(), plus 1 for a missing or short workspace (problems that fill
@@ -126,7 +127,7 @@ int attn_fwd_split_static(const void* q, const void* k, const void* v, void* o,
  * are first transposed into `copies` (16-byte aligned,
  * attn_row_copies_bytes() bytes, one launch) and the row-contiguous kernel
  * runs on those. For layouts that attn_fwd_split() does not read in place,
- * and faster than reading in place from about 7000 tokens. No counterpart in
+ * and faster than reading in place from about 5500 tokens. No counterpart in
  * the reference. */
 size_t attn_row_copies_bytes(int B, int H, int Sq, int Skv, int D);
 int attn_fwd_split_copied(const void* q, const void* k, const void* v, void* o, int B, int H,
