@@ -508,31 +508,32 @@ int fail(const char* msg) {
 bool mult8(long v) { return v >= 0 && v % 8 == 0; }
 
 // The kernel configurations: voxels / 64, KB, channels per workgroup (64*CW),
-// workgroups per CU, the time in us of a 64-voxel x 256-channel piece of a tile
-// (`per_kg` for a reduction of 13824 elements, `fixed` for start-up and
-// epilogue; fitted on MI355X, see plan_conv) and how much longer a workgroup
-// that shares its CU takes than one alone; launcher. The last two have four
-// waves along the voxels: 256 voxels x 128 channels in one workgroup of eight
-// waves load a quarter less per output than two workgroups of 128 x 128 (a
-// strided 128 -> 128 layer of 65,536 voxels 69 -> 64 us, stride 1 66 -> 58),
-// 128 x 64 wastes less on 64 and 192 channels (64 -> 64 of 98,304 voxels 49 ->
-// 35 us) and makes more, shorter workgroups of small problems (512 -> 512 of
-// 256 voxels 22 -> 16 us).
+// workgroups per CU, ring stages; the time in us of a 64-voxel x 256-channel
+// piece of a tile (`per_kg` for a reduction of 13824 elements, `fixed` for
+// start-up and epilogue); how much of it a workgroup that shares its CU takes
+// longer than one alone, and an odd last one; the factor on per_kg where C < 64
+// (taps change within a k-tile); launcher. Fitted on MI355X, see plan_conv. The
+// last two have four waves along the voxels: 256 voxels x 128 channels in one
+// workgroup of eight waves load a quarter less per output than two workgroups of
+// 128 x 128 (a strided 128 -> 128 layer of 65,536 voxels 69 -> 64 us, stride 1
+// 66 -> 58), 128 x 64 wastes less on 64 and 192 channels (64 -> 64 of 98,304
+// voxels 49 -> 35 us) and makes more, shorter workgroups of small problems (512
+// -> 512 of 256 voxels 22 -> 16 us).
 struct ConvKernel {
-    int nb, kb, bch, occ;
-    double per_kg, fixed, shared;
+    int nb, kb, bch, occ, nst;
+    double per_kg, fixed, shared, odd, small_c;
     void (*launch)(const ConvArgs&, hipStream_t);
 };
 const ConvKernel kKernels[] = {
-    {4, 32, 128, 2, 91.2, 3.7, 0.82, launch_cfg<4, 3, 32, 2>},
-    {3, 64, 128, 2, 91.9, 3.4, 0.55, launch_cfg<3, 2, 64, 2>},
-    {2, 64, 128, 2, 103.7, 3.9, 0.55, launch_cfg<2, 2, 64, 2>},
-    {4, 32, 256, 1, 74.7, 3.7, 0.0, launch_cfg<4, 4, 32, 4>},
-    {3, 64, 256, 1, 87.4, 3.0, 0.0, launch_cfg<3, 2, 64, 4>},
-    {2, 64, 256, 1, 77.8, 4.6, 0.0, launch_cfg<2, 3, 64, 4>},
-    {3, 32, 256, 1, 91.0, 3.1, 0.0, launch_cfg<3, 4, 32, 4>},
-    {4, 64, 128, 1, 81.4, 4.7, 0.0, launch_cfg<2, 3, 64, 2, 4>},
-    {2, 64, 64, 2, 116.2, 5.6, 0.77, launch_cfg<1, 3, 64, 1, 4>},
+    {4, 32, 128, 2, 3, 85.0, 3.6, 0.88, 0.15, 0.88, launch_cfg<4, 3, 32, 2>},
+    {3, 64, 128, 2, 2, 88.0, 3.8, 0.40, 0.32, 0.85, launch_cfg<3, 2, 64, 2>},
+    {2, 64, 128, 2, 2, 93.0, 4.7, 0.18, 0.63, 0.85, launch_cfg<2, 2, 64, 2>},
+    {4, 32, 256, 1, 4, 77.0, 3.6, 0.0, 0.0, 0.92, launch_cfg<4, 4, 32, 4>},
+    {3, 64, 256, 1, 2, 86.0, 3.4, 0.0, 0.0, 0.92, launch_cfg<3, 2, 64, 4>},
+    {2, 64, 256, 1, 3, 79.0, 3.8, 0.0, 0.0, 1.22, launch_cfg<2, 3, 64, 4>},
+    {3, 32, 256, 1, 4, 86.0, 3.6, 0.0, 0.0, 0.85, launch_cfg<3, 4, 32, 4>},
+    {4, 64, 128, 1, 3, 79.0, 5.0, 0.0, 0.0, 1.09, launch_cfg<2, 3, 64, 2, 4>},
+    {2, 64, 64, 2, 3, 112.0, 6.7, 0.74, 0.05, 1.24, launch_cfg<1, 3, 64, 1, 4>},
 };
 constexpr int kNumKernels = sizeof(kKernels) / sizeof(kKernels[0]);
 
@@ -552,15 +553,21 @@ int find_kernel(int nb, int kb, int bch) {
 // nsplit ranges of whole 64-element units: without it a 32x32x2-voxel layer of
 // 512 channels (64 tiles of 216 serial k-tiles) left three quarters of the
 // CUs idle and took 183 us; in 8 ranges it takes 42.
-// Estimate: R x tile size x (per_kg x range / 13824 + fixed), R the
-// workgroups on the busiest CU in units of one workgroup's time (for two per
-// CU: halves of a pair's time, one workgroup alone taking 2 - `shared` halves
-// and an odd last one 1.25), plus for a split the reduce kernel: a launch, a
-// little per range (its loads go out four ranges at a time) and the partial
-// sums' traffic. Fitted to 24 layers on MI355X (1 to 3x3x3 windows, 16 to 512
-// channels, 256 to 150,000 voxels) over every configuration and 1 to 24
-// ranges: the chosen pair is within 1 % of the fastest one on average, 6 % at
-// worst.
+// Estimate: tile size x (R x per_kg x range / 13824 + R' x fixed), the range in
+// whole groups of ring stages, R the workgroups on the busiest CU in units of one
+// workgroup's time (for two per CU: halves of a pair's time, one workgroup alone
+// taking 2 - `shared` halves and an odd last one 1 + `odd`; of the fixed part,
+// which is latency, one alone takes 2 - kFixedShared), plus for a split the
+// reduce kernel: a launch, a little per range (its loads go out four ranges at a
+// time) and the partial sums' traffic. Fitted to 900 layers on MI355X (1x1x1 to
+// 3x3x3 windows, 8 to 512 channels, 200 to 200,000 voxels) over every
+// configuration and 1 to 48 ranges. On 360 others the chosen pair is 0.6 % behind
+// the fastest one on average, and 2 of them are more than 3 % (up to 11 %) slower
+// than with the seven 128- and 256-channel configurations and no split, as they
+// were chosen before the last two configurations and the splits came. A fit to 24
+// layers, hardly any with C < 64 or a reduction under 500, was 1.6 % behind and
+// slower there on one layer in 20, up to 22 % (384 -> 512 of 8250 voxels, 1x1x1
+// window: 17.3 us, 14.4 with what is chosen now).
 // For tests, read on every call: GFX906_AMD_CONV_CFG = "<NB>x<KB>" (128
 // channels) or "<NB>x<KB>x<channels>" (a row of kKernels) fixes the
 // configuration, unsplit unless GFX906_AMD_CONV_NSPLIT = n asks for n ranges
@@ -571,9 +578,12 @@ constexpr int kSplitMinUnits = 4;  // shortest range worth a workgroup
 constexpr int kSplitMax = 64;
 // A split has to be this much better than none: CUs left idle let the others
 // hold a higher clock (512 -> 512 of 17,812 voxels, 186 workgroups unsplit: 250
-// us, and 274 in two ranges that the estimate has 1.4 % ahead).
+// us, and 274 in two ranges that the estimate has 7 % ahead).
 constexpr double kSplitMargin = 1.12;
-constexpr double kRedLaunch = 1.2, kRedPerSplit = 0.15, kRedPerByte = 0.14e-6;  // us
+constexpr double kRedLaunch = 1.33, kRedPerSplit = 0.09, kRedPerByte = 0.17e-6;  // us
+constexpr double kFixedShared = 0.57;
+constexpr int kSmallC = 64;
+constexpr double kSmallCFixed = 1.2;  // factor on `fixed` where C < 64
 struct ConvPlan {
     int cfg, nsplit, split_len;
 };
@@ -582,7 +592,7 @@ size_t conv_ws_bytes(const ConvPlan& p, long M, int K) {
     return p.nsplit <= 1 ? 0 : (size_t)p.nsplit * M * K * 4;
 }
 
-ConvPlan plan_conv(long M, int K, long KG, size_t ws_cap) {
+unsigned conv_cus() {
     static const unsigned ncu = [] {
         int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -591,19 +601,46 @@ ConvPlan plan_conv(long M, int K, long KG, size_t ws_cap) {
             n = 256;
         return (unsigned)n;
     }();
-    int only = -1;  // forced configuration
-    if (const char* e = getenv("GFX906_AMD_CONV_CFG")) {
-        int nb = 0, kb = 0, bch = 128;
-        if (sscanf(e, "%dx%dx%d", &nb, &kb, &bch) >= 2) only = find_kernel(nb, kb, bch);
+    return ncu;
+}
+
+// Tiles of a configuration (held to 2^24, an output past the device's memory, so
+// that 32 bits count the ranges too).
+unsigned conv_tiles(const ConvKernel& c, long M, int K) {
+    return (unsigned)std::min((M + 64 * c.nb - 1) / (64 * c.nb) * (((long)K + c.bch - 1) / c.bch),
+                              1L << 24);
+}
+
+// Estimated time of `wgs` workgroups over `range` reduction elements each.
+double conv_cost(const ConvKernel& c, unsigned wgs, unsigned range, unsigned ncu, bool small_c) {
+    const unsigned group = (unsigned)(c.nst * c.kb);
+    const double kgu = (double)((range + group - 1) / group * group) / 13824.0;
+    const unsigned n = (wgs + ncu - 1) / ncu;
+    double r = n, r_fixed = n;  // workgroups on the busiest CU
+    if (c.occ == 2 && n == 1) {
+        r = 2.0 - c.shared;
+        r_fixed = 2.0 - kFixedShared;
+    } else if (c.occ == 2 && (n & 1)) {
+        r += c.odd;
     }
+    return c.nb * c.bch / 256.0 * (r * c.per_kg * (small_c ? c.small_c : 1.0) * kgu +
+                                   r_fixed * c.fixed * (small_c ? kSmallCFixed : 1.0));
+}
+
+// The configuration that GFX906_AMD_CONV_CFG names, or -1.
+int forced_kernel() {
+    const char* e = getenv("GFX906_AMD_CONV_CFG");
+    int nb = 0, kb = 0, bch = 128;
+    return e && sscanf(e, "%dx%dx%d", &nb, &kb, &bch) >= 2 ? find_kernel(nb, kb, bch) : -1;
+}
+
+ConvPlan plan_conv(long M, int K, long KG, size_t ws_cap) {
+    const unsigned ncu = conv_cus();
+    const int only = forced_kernel();
     const long units = (KG + kSplitUnit - 1) / kSplitUnit;
     unsigned tiles1[kNumKernels], fewest = ~0u;  // tiles of each configuration, unsplit
     for (int i = 0; i < kNumKernels; ++i) {
-        const ConvKernel& c = kKernels[i];
-        // (held to 2^24, an output past the device's memory, so that 32 bits count the ranges too)
-        tiles1[i] = (unsigned)std::min((M + 64 * c.nb - 1) / (64 * c.nb) *
-                                           (((long)K + c.bch - 1) / c.bch),
-                                       1L << 24);
+        tiles1[i] = conv_tiles(kKernels[i], M, K);
         fewest = std::min(fewest, tiles1[i]);
     }
     // More than four rounds of workgroups gain nothing (and the search costs
@@ -622,23 +659,38 @@ ConvPlan plan_conv(long M, int K, long KG, size_t ws_cap) {
         const ConvPlan p{0, (int)((units + per - 1) / per), (int)(per * kSplitUnit)};
         if (ns > ns_lo && p.nsplit != ns) continue;  // the same ranges as a smaller count
         if (conv_ws_bytes(p, M, K) > ws_cap) break;
-        const double kgu = (double)std::min<long>(KG, p.split_len) / 13824.0;
+        const unsigned range = (unsigned)std::min<long>(KG, p.split_len);
         const double red = p.nsplit > 1 ? kRedLaunch + kRedPerSplit * p.nsplit +
                                               kRedPerByte * (double)conv_ws_bytes(p, M, K)
                                         : 0.0;
         for (int i = 0; i < kNumKernels; ++i) {
             if (only >= 0 && i != only) continue;
-            const ConvKernel& c = kKernels[i];
-            const unsigned n = (tiles1[i] * (unsigned)p.nsplit + ncu - 1) / ncu;
-            double r = n;  // workgroups on the busiest CU
-            if (c.occ == 2) r += n == 1 ? 1.0 - c.shared : n & 1 ? 0.25 : 0.0;  // (halves)
-            double cost = r * c.nb * c.bch / 256.0 * (c.per_kg * kgu + c.fixed) + red;
+            double cost =
+                conv_cost(kKernels[i], tiles1[i] * (unsigned)p.nsplit, range, ncu, false) + red;
             if (p.nsplit > 1) cost *= kSplitMargin;
             if (cost < best_cost) {
                 best_cost = cost;
                 best = p;
                 best.cfg = i;
             }
+        }
+    }
+    return best;
+}
+
+// The plan's configuration where C < 64, for the same ranges (the workspace, and
+// with it the ranges, is planned without C).
+int small_c_kernel(const ConvPlan& p, long M, int K, long KG) {
+    if (forced_kernel() >= 0) return p.cfg;
+    const unsigned ncu = conv_cus(), range = (unsigned)std::min<long>(KG, p.split_len);
+    int best = p.cfg;
+    double best_cost = 1e300;
+    for (int i = 0; i < kNumKernels; ++i) {
+        const double cost = conv_cost(kKernels[i], conv_tiles(kKernels[i], M, K) * (unsigned)p.nsplit,
+                                      range, ncu, true);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = i;
         }
     }
     return best;
@@ -735,6 +787,7 @@ int conv3d_impl(const void* x, const void* w, const void* bias, const void* res,
     a.nsplit = p.nsplit;
     a.split_len = p.split_len;
     a.ws = (float*)workspace;
+    if (C < kSmallC) p.cfg = small_c_kernel(p, M, K, KG);
     kKernels[p.cfg].launch(a, stream);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && p.nsplit > 1) {

@@ -89,6 +89,22 @@ def test_forced_split_counts(monkeypatch, cfg, i, nsplit):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nsplit", [1, 2, 3])
+@pytest.mark.parametrize("c,k", [(8, 24), (16, 200), (32, 64), (40, 136), (56, 512)])
+def test_small_channel_counts(monkeypatch, c, k, nsplit):
+    """C < 64: the configuration is chosen anew for the planned ranges."""
+    print(f"case conv split: C{c} K{k} n{nsplit}", flush=True)
+    x, w, b, res = oc.make_case((1, c, 4, 12, 21), (k, 3, 3, 3), (1, 1, 1), True, True, seed=600 + c)
+    call = kitchen.plan(to_dev(x), to_dev(w), to_dev(b), to_dev(res), [1, 1, 1])
+    monkeypatch.setenv("GFX906_AMD_CONV_NSPLIT", str(nsplit))
+    got = call.run(gfx906_amd.extension()).clone()
+    capi = run_capi(call)
+    torch.cuda.synchronize()
+    check(got, oc.conv3d_gemm(x, w, b, res, (1, 1, 1)), f"C{c} n{nsplit}")
+    assert torch.equal(got, capi)
+
+
+@pytest.mark.gpu
 def test_small_layer_is_split_and_accurate_in_a_graph(monkeypatch):
     x, w, b, res = oc.make_case((1, 256, 3, 18, 18), (256, 3, 3, 3), (1, 1, 1), True, True, 510)
     print("case conv split: planner's own choice, eager and captured", flush=True)
