@@ -2551,8 +2551,10 @@ size_t split_ws_bytes(const SplitPlan& p, int B, int H, int Sq, int D) {
 //
 // Both kernels' times are estimated in us and the smaller wins (the few-rows
 // kernel has to be kRowsMargin better, kRowsMarginRounds over several rounds,
-// where the estimate is 10-15 % off at times: B2 H4 Sq2439 Skv387 D64, 312
-// workgroups, 15.7 against 14.9). Few-rows: start + rounds of workgroups
+// where the estimate is up to 20 % off: B2 H4 Sq2439 Skv387 D64, 312 workgroups,
+// 15.7 against 14.9; B1 H12 S3400 D64 66.3 against 60.6; B1 H5 S9565 D32 148
+// against 116. With these margins none of 800 drawn shapes is more than 3 %
+// slower than the ring kernel; with 1.13 and no kRingNarrow 10 were, up to 29 %). Few-rows: start + rounds of workgroups
 // (one per CU) x (fixed + step x steps of the busiest wave), combined in
 // quadrature with K and V's way from HBM, plus a split's merge. Ring:
 // start + rounds x (fixed + tile x tiles, in fours) of `ring`'s plan, plus its
@@ -2582,7 +2584,10 @@ constexpr double kRingFixed[2] = {4.7, 2.0}, kRingTile[2] = {1.66, 2.2};  // D =
 constexpr double kRingStart = 1.3, kRingAlone = 0.68;
 constexpr double kRingMergeLaunch = 2.4, kRingMergeSplit = 0.13, kRingMergeByte = 0.27e-6;
 constexpr double kRowsHbm = 6.9e6;  // bytes per us
-constexpr double kRowsMargin = 1.06, kRowsMarginRounds = 1.13;
+constexpr double kRowsMargin = 1.06, kRowsMarginRounds = 1.22;
+// The ring kernel's time per tile for D <= 48 and D <= 32 (32 or 48 dims of PV,
+// one or two Q fragments) against D = 64.
+constexpr double kRingNarrow[2] = {0.9, 0.8};
 RowsPlan rows_plan(int B, int H, int Sq, int Skv, int D, const SplitPlan& ring, size_t ws_cap) {
     if (D > 128 || Skv == 0 || ring.whole > 0) return kNoRows;
     const int bn = D == 128 ? CfgRows<128, 2>::BN : CfgRows<64, 2>::BN;
@@ -2604,8 +2609,10 @@ RowsPlan rows_plan(int B, int H, int Sq, int Skv, int D, const SplitPlan& ring, 
     const long long wgs = bh * ((Sq + query_tile(D) - 1) / query_tile(D)) * ring.nsplit;
     const int per_ring = (tiles + ring.nsplit - 1) / ring.nsplit;
     const double alone = D != 128 && wgs <= cus ? kRingAlone : 1.0;
+    const double narrow = D <= 32 ? kRingNarrow[1] : D <= 48 ? kRingNarrow[0] : 1.0;
+    const double tile = kRingTile[cls] * alone * narrow;
     double best_t = kRingStart + (double)((wgs + slots - 1) / slots) *
-                                     (kRingFixed[cls] + kRingTile[cls] * alone * ((per_ring + 3) / 4 * 4));
+                                     (kRingFixed[cls] + tile * ((per_ring + 3) / 4 * 4));
     if (ring.nsplit > 1)
         best_t += kRingMergeLaunch + kRingMergeSplit * ring.nsplit +
                   kRingMergeByte * rows_bytes * ring.nsplit;
