@@ -126,7 +126,9 @@ struct KArgs {
     // ws_o[s][r][0..D) and its (m, l) to ws_ml[s][r][0..1], r < tail_rows the
     // row's place (head-major) among the tail's, which start at row0;
     // attn_combine merges them.
-    int BH, nsplit, split_len, whole, tail;
+    // Split units are taken `group` at a time (a head's where every unit is
+    // split, else the whole tail), range by range (work_item).
+    int BH, nsplit, split_len, whole, tail, group;
     long long row0, tail_rows;
     float* ws_o;
     float* ws_ml;
@@ -163,25 +165,38 @@ struct WorkItem {
 // to XCD w % 8; where the count divides by 8, consecutive items go to one XCD,
 // and items enumerate the query tiles of one key range consecutively, so that
 // an XCD's L2 streams the K/V of as few heads (or key ranges) as possible
-// (c2 +2 %).
+// (c2 +2 %). Where every unit is split the ranges of one head follow each other,
+// so that an XCD also reads the Q of as few heads as possible (range by range
+// over all heads: 16 heads of 2111, D = 128, 65.3 us, and 63.3 this way; 20 of
+// 3933, D = 64, 126.5 and 124.3); a tail may start inside a head and goes range by
+// range.
 __device__ __forceinline__ int xcd_order(int w, int n) {
     return (n & 7) == 0 ? (w & 7) * (n >> 3) + (w >> 3) : w;
 }
-template <bool SPLIT, bool TAIL>
+// Which units of a SPLIT kernel's grid are split: all, a tail, or either.
+enum SplitUnits { kAllSplit, kTailSplit, kAnySplit };
+template <bool SPLIT, SplitUnits UNITS>
 __device__ __forceinline__ WorkItem work_item(const KArgs& a, int blk, int n, int nqt) {
     WorkItem it;
     it.split = 0;
     it.part = false;
     int unit;
     if constexpr (SPLIT) {
-        const int whole = TAIL ? a.whole : 0;
+        const int whole = UNITS == kAllSplit ? 0 : a.whole;
         if (blk < whole) {
             unit = xcd_order(blk, whole);
         } else {
             const int w = xcd_order(blk - whole, n - whole);
-            it.split = w / a.tail;
-            unit = whole + (w - it.split * a.tail);
+            const int group = UNITS == kAllSplit ? nqt : UNITS == kTailSplit ? a.tail : a.group;
+            const int range = w / group, head = UNITS == kTailSplit ? 0 : range / a.nsplit;
+            it.split = range - head * a.nsplit;
+            unit = whole + head * group + (w - range * group);
             it.part = true;
+            if constexpr (UNITS == kAllSplit) {
+                it.bh = head;
+                it.qt = unit - head * nqt;
+                return it;
+            }
         }
     } else {
         unit = xcd_order(blk, n);
@@ -623,7 +638,8 @@ attn_fwd_pipe(const KArgs a) {
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i = lane & 15, g = lane >> 4;
     const int nqt = (Sq + C::BM - 1) / C::BM;
-    const WorkItem it = work_item<SPLIT, C::TAIL>(a, blockIdx.x, gridDim.x, nqt);
+    constexpr SplitUnits kUnits = C::TAIL ? kTailSplit : kAllSplit;
+    const WorkItem it = work_item<SPLIT, kUnits>(a, blockIdx.x, gridDim.x, nqt);
     const int qt = it.qt, bh = it.bh;
     const int b = bh / a.H, h = bh - b * a.H;
     // This workgroup's keys: [kv0, kv0 + Skv) of the head.
@@ -758,7 +774,7 @@ attn_fwd_pipe(const KArgs a) {
             int bytes = 0, off = 0;
             if (resident > 0 && (resident & 7) == 0 && nb < (long long)gridDim.x &&
                 span < (1LL << 31)) {  // (uniform)
-                const WorkItem next = work_item<SPLIT, C::TAIL>(a, (int)nb, gridDim.x, nqt);
+                const WorkItem next = work_item<SPLIT, kUnits>(a, (int)nb, gridDim.x, nqt);
                 const int qt2 = next.qt, bh2 = next.bh;
                 const int b2 = bh2 / a.H, h2 = bh2 - b2 * a.H;
                 const int rows = min(Sq - qt2 * C::BM, C::BM);
@@ -1095,7 +1111,9 @@ attn_fwd_pipe(const KArgs a) {
     const KArgs& ea = C::TAIL ? args_here() : a;
     const int Sqe = ea.Sq, De = ea.D;
     const WorkItem ite =
-        C::TAIL ? work_item<SPLIT, C::TAIL>(ea, block_here(), gridDim.x, (Sqe + C::BM - 1) / C::BM) : it;
+        C::TAIL ? work_item<SPLIT, kUnits>(ea, block_here(), gridDim.x,
+                                           (Sqe + C::BM - 1) / C::BM)
+                : it;
     const int be = C::TAIL ? ite.bh / ea.H : b, he = C::TAIL ? ite.bh - be * ea.H : h;
     T* const Oe = C::TAIL ? (T*)ea.o + be * ea.so.b + he * ea.so.h : Oh;
     // 1 / l where l is 0: a row whose scores are all -inf (NaN, but 0 for D = 128), or no keys.
@@ -1485,7 +1503,7 @@ __global__ void __launch_bounds__((CfgRows<DP, NBQ>::NT), 2) attn_fwd_rows(const
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i = lane & 15, g = lane >> 4;
     const int nqt = (Sq + C::BM - 1) / C::BM;
-    const WorkItem it = work_item<SPLIT, false>(a, blockIdx.x, gridDim.x, nqt);
+    const WorkItem it = work_item<SPLIT, kAllSplit>(a, blockIdx.x, gridDim.x, nqt);
     const int b = it.bh / a.H, h = it.bh - b * a.H;
     const int kv0 = SPLIT ? it.split * a.split_len : 0;
     const int Skv = SPLIT ? max(0, min(a.Skv - kv0, a.split_len)) : a.Skv;
@@ -2843,6 +2861,7 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
     a.ncu = cu_count();
     a.whole = 0;
     a.tail = 0;
+    a.group = 1;
     a.row0 = 0;
     a.tail_rows = (long long)B * H * Sq;
     const bool tl = token_contiguous(sk, sv, D);
@@ -2893,7 +2912,9 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, int B, i
         a.nsplit = p.nsplit;
         a.split_len = p.split_len;
         a.whole = p.whole;
-        a.tail = B * H * ((Sq + query_tile(D) - 1) / query_tile(D)) - p.whole;
+        const int nqt = (Sq + query_tile(D) - 1) / query_tile(D);
+        a.tail = B * H * nqt - p.whole;
+        a.group = p.whole ? a.tail : nqt;
         a.row0 = first_split_row(p.whole, Sq, D);
         a.tail_rows -= a.row0;
         a.ws_o = (float*)workspace;
